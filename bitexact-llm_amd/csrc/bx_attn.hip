@@ -1580,19 +1580,51 @@ __device__ __forceinline__ int pre_vpos(int key) {   // tile key -> its Vp posit
   return ((key >> 2) & 3) * 16 + ((key >> 4) & 3) * 4 + (key & 3);
 }
 
-__global__ __launch_bounds__(256) void pre_split_kernel(AttnArgs p, int8_t* kp, int8_t* vp, int64_t* tab2, int Z, int Sp,
+// The 2^-f table as the main kernel keeps it in LDS: U[i] = floor((2^60 - lut[i]) / 2^29), 32 bits an entry (64 KiB
+// for the table instead of the 128 KiB of its int64 entries, so it fits beside the ring). pre_table_block (one block per 256 entries) writes it
+// to scratch with one word per block: 1 when its entries can take the short weight rule, i.e. 2^59 <= lut[i] <=
+// 2^60, 0 <= U[i + 1] - U[i] < 2^20 and U[i + 1] > 0 (true of the 2^-f table; any other table takes the general rule).
+constexpr int kTabN = 1 << kExp2Bits;                  // entries [0, kTabN]
+constexpr int kTabBlocks = kTabN / 256;
+constexpr int kTabPad = kTabN + 4;                     // words of U in scratch and LDS (16-byte multiple)
+// Factors of the table in float64: lut[128 h + l] is within 2^10 of F[h] F[129 + l] (F[h] = lut[128 h], F[129 + l] =
+// lut[l] / 2^60; three roundings of 2^-53 and the table's own), checked for every entry by pre_table_block.
+constexpr int kTabF = 129 + 128;
+__device__ __forceinline__ double pre_f(const int64_t* lut, int j) {
+  return j < 129 ? (double)lut[j * 128] : ldexp((double)lut[j - 129], -kExp2One);
+}
+__device__ __forceinline__ uint32_t pre_u(int64_t a) {
+  const bool in = a >= (1LL << 59) && a <= (1LL << 60);
+  return in ? (uint32_t)(((1LL << 60) - a) >> 29) : 0xffffffffu;
+}
+__device__ __forceinline__ void pre_table_block(const int64_t* lut, uint32_t* tab, int b) {
+  const int i = b * 256 + threadIdx.x;
+  const uint32_t u0 = pre_u(lut[i]), u1 = pre_u(lut[i + 1]);
+  tab[i] = u0;
+  if (i == kTabN - 1) {
+#pragma unroll
+    for (int j = 0; j < kTabPad - kTabN; ++j) tab[kTabN + j] = u1;
+  }
+  const double df = pre_f(lut, i >> 7) * pre_f(lut, 129 + (i & 127)) - (double)(lut[i] & ~1023LL);
+  const double de = pre_f(lut, (i + 1) >> 7) * pre_f(lut, 129 + ((i + 1) & 127)) - (double)(lut[i + 1] & ~1023LL);
+  const bool ok = u0 != 0xffffffffu && u1 != 0xffffffffu && u1 - u0 < (1u << 20) && u1 > 0 && df >= -1024.0 &&
+                  df <= 2048.0 && de >= -1024.0 && de <= 2048.0;
+  const bool all = __syncthreads_and(ok);
+  if (threadIdx.x == 0) tab[kTabPad + b] = all ? 1u : 0u;
+}
+
+__global__ __launch_bounds__(256) void pre_split_kernel(AttnArgs p, int8_t* kp, int8_t* vp, uint32_t* tab, int Z, int Sp,
                                                         int HD) {
+  if (blockIdx.x < kTabBlocks) {
+    pre_table_block(p.lut, tab, blockIdx.x);
+    return;
+  }
   const int CR = HD / 16;
   const int64_t nk = (int64_t)Z * Sp * CR;          // K units: (z, key, 16-dim chunk)
   const int64_t nv = (int64_t)Z * (Sp / 4) * (HD / 4);   // V units: (z, 4 keys, 4 dims)
-  const int64_t nt = 1 << kExp2Bits;                 // table pairs: (lut[i], lut[i + 1] - lut[i])
-  for (int64_t u = blockIdx.x * 256LL + threadIdx.x; u < nk + nv + nt; u += (int64_t)gridDim.x * 256) {
-    if (u >= nk + nv) {
-      const int64_t i = u - nk - nv;
-      const int64_t a = p.lut[i];
-      tab2[2 * i] = a;
-      tab2[2 * i + 1] = p.lut[i + 1] - a;
-    } else if (u < nk) {
+  for (int64_t u = (blockIdx.x - kTabBlocks) * 256LL + threadIdx.x; u < nk + nv;
+       u += (int64_t)(gridDim.x - kTabBlocks) * 256) {
+    if (u < nk) {
       const int c = (int)(u % CR), s = (int)((u / CR) % Sp), z = (int)(u / ((int64_t)CR * Sp));
       uint32_t l[3][4];
 #pragma unroll
@@ -1629,58 +1661,94 @@ __global__ __launch_bounds__(256) void pre_split_kernel(AttnArgs p, int8_t* kp, 
   }
 }
 
-// attn_pre2_kernel: a block (8 waves at head_dim 64, 4 at 128) owns 16 rows per wave of consecutive query rows of
-// one group z, wave w rows 16 w .. 16 w + 15.
-// The 64-key tiles of the limb planes stream through an NS-stage LDS ring filled by buffer_load ... lds (1 KiB
-// per wave instruction; 16-byte chunks XOR-swizzled by row so the 16 rows an MFMA operand read touches fall in
-// distinct bank groups). QK is computed transposed: A = K limb plane j (16 keys x 64 dims), B = limb i of the
-// wave's 16 queries (registers), so lane l receives query l & 15's scores for keys 16 kb + 4 (l >> 4) + e; the
-// nine limb products accumulate by weight i + j in five int32 sets, joined in int64. Sweep 1 keeps the per-query
-// maxima. Sweep 2 forms the weights in the same lanes; their three limbs, packed in key order 4 kb + e, are the
-// PV A operand as they stand (16 queries x 64 keys in Vp's order), and B = V limb plane j (64 keys x 16 dims):
-// five int32 sets per 16-dim block (exact while S 3 2^14 < 2^31), joined in int64 at the end. The table loads of
-// a tile's 16 weights go out together, before the tile's next ring stage is requested.
-// Byte k of each of four words, in order, as one word (two v_perm_b32 and an or).
-template <int k>
-__device__ __forceinline__ uint32_t gather_bytes(const uint32_t (&a)[4]) {
-  const uint32_t lo = __builtin_amdgcn_perm(a[1], a[0], 0x0c0c0400u + k * 0x101u);        // a0.k, a1.k, 0, 0
-  const uint32_t hi = __builtin_amdgcn_perm(a[3], a[2], 0x04000c0cu + k * 0x01010000u);    // 0, 0, a2.k, a3.k
-  return lo | hi;
+// The three signed base-256 limbs of four values 0 <= x <= 2^22, each as one word of four bytes: byte i of x + 0x8080
+// is limb i + 128 for i = 0, 1 and limb 2 for i = 2 (the adds' carries are the digits' borrows); the bytes of the
+// four words are transposed with seven v_perm_b32.
+__device__ __forceinline__ void limb_words(const int32_t (&x)[4], uint32_t& l0, uint32_t& l1, uint32_t& l2) {
+  uint32_t y[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = (uint32_t)x[e] + 0x8080u;
+  const uint32_t a = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u);   // y0.0 y1.0 y0.1 y1.1
+  const uint32_t b = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u);
+  const uint32_t c = __builtin_amdgcn_perm(y[1], y[0], 0x0c0c0602u);   // y0.2 y1.2 0 0
+  l0 = __builtin_amdgcn_perm(b, a, 0x05040100u) ^ 0x80808080u;
+  l1 = __builtin_amdgcn_perm(b, a, 0x07060302u) ^ 0x80808080u;
+  l2 = __builtin_amdgcn_perm(y[3], y[2], 0x06020c0cu) | c;             // 0 0 y2.2 y3.2
 }
 
 template <int HD>
 struct Pre2 {
-  static constexpr int KK = HD / 64, CR = HD / 16, DB = HD / 16;
-  static constexpr int NS = HD == 64 ? 3 : 2;        // ring stages
-  static constexpr int PB = 3 * 64 * HD;             // one operand's three planes of a tile (bytes)
-  static constexpr int STAGE = 2 * PB;               // K then V
-  static constexpr int KI = PB / 1024;               // 1 KiB instructions per operand
-  static constexpr int NW = HD == 64 ? 8 : 4;        // waves (16 query rows each): 2 per SIMD at HD 64, 1 at 128
-  static constexpr int LPK = (KI + NW - 1) / NW;     // sweep 1 (K only): instructions per issuing wave
-  static constexpr int LPT = 2 * KI / NW;            // sweep 2: instructions per wave
-  static constexpr size_t LDS = (size_t)NS * STAGE;
+  static constexpr int KK = HD / 64, CR = HD / 16;
+  static constexpr int PB = 3 * 64 * HD;             // one operand's three planes of a tile (bytes): a ring slot
+  static constexpr int SLOTS = 3;                    // ring: K of tile t, V of tile t, K of tile t + 1, V of t + 1, ...
+  static constexpr int KI = PB / 1024;               // 1 KiB instructions per slot
+  // Waves that share 16 query rows, and waves of a block: two waves per SIMD (200 and 219 registers). Measured at
+  // head_dim 64 (4 x 1024 tokens): 8 waves 198 us, 12 waves (168 registers, spills) 305, 12 waves of pairs (156
+  // registers) 221; at head_dim 128 (1337 tokens): 8 waves of pairs 157 us, 4 single waves (one per SIMD) 234.
+  static constexpr int SW = HD == 64 ? 1 : 2;
+  static constexpr int NW = 8;
+  static constexpr int LP = (KI + NW - 1) / NW;      // instructions per issuing wave and slot
+  static constexpr int KB = 4 / SW, DB = HD / 16 / SW;   // 16-key blocks and 16-dim blocks of a wave
+  static constexpr int QR = 16 * NW / SW;            // query rows per block
+  static constexpr int XB = SW == 1 ? 0 : 3 * 16 * QR * 4;   // p exchange between the waves of a pair (bytes)
+  // LDS: the table first (its reads then need no address add), the ring, the exchange, the table's factors
+  static constexpr int RO = 4 * kTabPad, XO = RO + SLOTS * PB, FO = XO + XB;
+  static constexpr size_t LDS = FO + 8 * kTabF;
+  static_assert(RO % 16 == 0 && FO % 8 == 0, "LDS alignment");
+  static_assert(KI % LP == 0, "a wave issues LP instructions or none");
 };
 
 __device__ __forceinline__ int pre_swzk(int k, int HD) { return HD == 64 ? (k >> 2) & 3 : (k >> 1) & 7; }
 __device__ __forceinline__ int pre_swzv(int d) { return (d >> 2) & 3; }
 
+// An empty use: the value is formed where it stands (no branch around its computation).
+__device__ __forceinline__ void pin_v(int32_t& x) { asm("" : "+v"(x)); }
+__device__ __forceinline__ void pin_v(uint32_t& x) { asm("" : "+v"(x)); }
+
+// attn_pre2_kernel: SW waves own 16 consecutive query rows of one group z (SW = 2: each forms the scores and weights
+// of half of a tile's keys and p V of half of the dims, the weights' limbs meet in LDS; accumulators per wave halve).
+// The 64-key tiles of the limb planes stream through a 3-slot LDS ring filled by buffer_load ... lds
+// (1 KiB per wave instruction; 16-byte chunks XOR-swizzled by row so the 16 rows an MFMA operand read touches fall
+// in distinct bank groups). QK is computed transposed: A = K limb plane j (16 keys x 64 dims), B = limb i of the
+// 16 queries (registers), so lane l receives query l & 15's scores for keys 16 kb + 4 (l >> 4) + e; the
+// nine limb products accumulate by weight i + j in five int32 sets, joined in int64. Sweep 1 keeps the per-query
+// maxima. Sweep 2 forms the weights in the same lanes; their three limbs, packed in key order 4 kb + e, are the
+// PV A operand as they stand (16 queries x 64 keys in Vp's order), and B = V limb plane j (64 keys x 16 dims):
+// five int32 sets per 16-dim block (exact while S 3 2^14 < 2^31), joined in int64 at the end. The next key block's
+// MFMAs are issued before a block's weights are formed.
+//
+// The short weight rule (`fast`: no query of the wave has a negative exponent shift, 0 <= l2e < 2^31, and the table
+// passed pre_table_block's check). With U the LDS table, y = (2^60 - v) / 2^29 of the interpolated value v lies in
+// [Uc - 2^-30, Uc + 2) for Uc = U0 + ((U1 - U0) rr >> 12): both entries (fractions at most 1 - 2^-29) and the
+// product are floors, v's own rounding is 2^-30 of the unit. The weight rshc(v, 38 + n) = floor((2^31 + 2^(8+n) - y) / 2^(9+n)) for n <= 22 is
+// then 2^(22-n) + (T >> (9+n)), T = 2^(8+n) - Uc, whatever y is, unless T mod 2^(9+n) <= 1: such a score (2 in
+// 2^(9+n)) takes its value from the table's float64 factors, and from the int64 table where even that is within
+// 2^-25 of a rounding boundary. From n = 23 the weight is 0, v being below 2^60, except at the single position n =
+// 23, f = 0 (Uc = 0: T = 2^31 marks it). Before, every score gathered
+// its 16-byte table pair through L1: with attention scores of unit spread that was 140 of 341 us (4 x 1024 tokens,
+// 32 / 8 heads of 64), the lanes' lines missing the 32 KiB L1. Now 198 us (1337 tokens, heads of 128: 233 -> 157):
+// bound by the integer work per score (about 40 VALU instructions), with sweep 1 about 55 us of it. The second-step
+// values come from LDS too because one wave's memory round trip holds its block at the tile's barrier (238 us).
 template <int HD>
 __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArgs p, const int8_t* planes, int Z,
-                                                                         int Sp, const char* tab2) {
+                                                                         int Sp, const uint32_t* tab) {
   using C = Pre2<HD>;
-  constexpr int QR = 16 * C::NW;                     // query rows per block
-  constexpr int KK = C::KK, DB = C::DB, NS = C::NS;
+  constexpr int QR = C::QR, SW = C::SW;
+  constexpr int KK = C::KK, DB = C::DB, SL = C::SLOTS;
   extern __shared__ __align__(16) char smem[];
+  uint32_t* U = (uint32_t*)smem;
+  char* ring = smem + C::RO;
   __shared__ int s_kend;
   const int tiles = (p.nq + QR - 1) / QR;
   const int z = blockIdx.x % Z, q0 = (tiles - 1 - blockIdx.x / Z) * QR;    // late (long) row tiles first
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kl = lane & 15, c = lane >> 4;
+  const int wr = w / SW, wp = w % SW;                // row group, part of it
   const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(planes), (short)0, kBufRange, 0x00020000);
   const int64_t vbase = (int64_t)Z * 3 * Sp * HD;
 
   // the lane's query (B operand rows) and its position / exponent
-  const int qr = q0 + 16 * w + kl;
+  const int qr = q0 + 16 * wr + kl;
   v4i qb[3][KK];
   {
     const int32_t* qp = p.q + (int64_t)z * p.sq_tile + (int64_t)min(qr, p.nq - 1) * p.sq_row;
@@ -1700,227 +1768,246 @@ __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArg
   const int64_t shift = live ? (int64_t)(kFK + 3 - kFZ) - p.sh[z * p.sh_tile + qr] : 0;
   if (threadIdx.x == 0) s_kend = 0;
   __syncthreads();
-  {
-    int64_t ke = wave_max64(my_qpos + 1);
-    if (lane == 0) atomicMax(&s_kend, (int)ke);
-  }
+  const int wmax_qpos = (int)wave_max64(my_qpos);    // the rows' largest position
+  const int wmin_qpos = (int)-wave_max64(-(int64_t)my_qpos);      // and smallest
+  if (lane == 0) atomicMax(&s_kend, wmax_qpos + 1);
   __syncthreads();
   const int kend = min(s_kend, p.S);                 // keys [0, kend) are visible to some row of the block
   const int ntile = (kend + 63) / 64;
 
-  // DMA offsets of the wave's instructions (tile 0) and their per-tile step
-  auto dma_off = [&](int n, int& off, int& step) {
-    if (n < C::KI) {
-      const int j = n / (C::KI / 3), o = (n % (C::KI / 3)) * 1024 + lane * 16;
-      const int k = o / HD, cc = ((o % HD) / 16) ^ pre_swzk(k, HD);
-      off = (int)((((int64_t)z * 3 + j) * Sp + k) * HD + cc * 16);
-      step = 64 * HD;
-    } else {
-      const int m = n - C::KI;
-      const int j = m / (C::KI / 3), o = (m % (C::KI / 3)) * 1024 + lane * 16;
-      const int d = o / 64, cc = ((o % 64) / 16) ^ pre_swzv(d);
-      off = (int)(vbase + (((int64_t)z * 3 + j) * HD + d) * Sp + cc * 16);
-      step = 64;
-    }
+  // DMA offsets of the wave's instructions of a K and of a V slot at tile 0 (a tile further: 64 HD and 64 bytes)
+  int offk[C::LP], offv[C::LP];
+  const bool issuer = w * C::LP < C::KI;
+#pragma unroll
+  for (int i = 0; i < C::LP; ++i) {
+    const int n = min(w * C::LP + i, C::KI - 1), j = n / (C::KI / 3), o = (n % (C::KI / 3)) * 1024 + lane * 16;
+    const int k = o / HD, kc = ((o % HD) / 16) ^ pre_swzk(k, HD);
+    offk[i] = (int)((((int64_t)z * 3 + j) * Sp + k) * HD + kc * 16);
+    const int d = o / 64, vc = ((o % 64) / 16) ^ pre_swzv(d);
+    offv[i] = (int)(vbase + (((int64_t)z * 3 + j) * HD + d) * Sp + vc * 16);
+  }
+  auto issue = [&](const int (&off)[C::LP], int step, int slot) {
+    if (!issuer) return;
+#pragma unroll
+    for (int i = 0; i < C::LP; ++i) buf_lds16(rs, ring + slot * C::PB + (w * C::LP + i) * 1024, off[i] + step, 0);
   };
-  int off1[C::LPK], stp1[C::LPK], off2[C::LPT], stp2[C::LPT];
-#pragma unroll
-  for (int i = 0; i < C::LPK; ++i) dma_off(min(w * C::LPK + i, C::KI - 1), off1[i], stp1[i]);
-#pragma unroll
-  for (int i = 0; i < C::LPT; ++i) dma_off(w * C::LPT + i, off2[i], stp2[i]);
-  const bool k_issuer = w * C::LPK < C::KI;          // sweep 1: the waves that load K
-  auto issue1 = [&](int t) {
-    char* base = smem + (t % NS) * C::STAGE;
-#pragma unroll
-    for (int i = 0; i < C::LPK; ++i)
-      if (w * C::LPK + i < C::KI) buf_lds16(rs, base + (w * C::LPK + i) * 1024, off1[i] + t * stp1[i], 0);
-  };
-  auto issue2 = [&](int t) {
-    char* base = smem + (t % NS) * C::STAGE;
-#pragma unroll
-    for (int i = 0; i < C::LPT; ++i) buf_lds16(rs, base + (w * C::LPT + i) * 1024, off2[i] + t * stp2[i], 0);
-  };
-  // scores of 16-key block kb of the staged tile for the lane's query: keys 16 kb + 4 c + e
-  auto qk = [&](const int8_t* kbase, int kb, int64_t (&raw)[4]) {
-    v4i acc[5];
+  // the nine limb products of 16-key block kb of the staged tile with the lane's query: keys 16 kb + 4 c + e
+  const int ksw = pre_swzk(kl, HD);                  // (of key 16 kb + kl: the same for every kb)
+  auto qk = [&](const int8_t* kbase, int kb, v4i (&acc)[5]) {
 #pragma unroll
     for (int u = 0; u < 5; ++u) acc[u] = v4i{0, 0, 0, 0};
-    const int k = kb * 16 + kl;
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk)
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const v4i a = *(const v4i*)(kbase + j * 64 * HD + k * HD + (((kk * 4 + c) ^ pre_swzk(k, HD)) * 16));
+        const v4i a = *(const v4i*)(kbase + j * 64 * HD + (kb * 16 + kl) * HD + (((kk * 4 + c) ^ ksw) * 16));
 #pragma unroll
         for (int i = 0; i < 3; ++i) acc[i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, qb[i][kk], acc[i + j], 0, 0, 0);
       }
-    // |acc| <= 64 KK 2^14 = 2^(20 + KK - 1): the pairs acc0 + 2^8 acc1 and acc2 + 2^8 acc3 are exact in int32
+  };
+  // |acc| <= 64 KK 2^14 = 2^(20 + KK - 1): the pairs acc0 + 2^8 acc1 and acc2 + 2^8 acc3 are exact in int32; the
+  // second joins by one 32 x 32 + 64-bit multiply-add (k64k: 2^16 the compiler cannot see)
+  int32_t k64k = 65536;
+  asm("" : "+s"(k64k));
+  auto join = [&](const v4i (&acc)[5], int64_t (&raw)[4]) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int32_t lo = acc[0][e] + (acc[1][e] << 8), mid = acc[2][e] + (acc[3][e] << 8);
-      raw[e] = (int64_t)lo + ((int64_t)mid << 16) + ((int64_t)acc[4][e] << 32);
+      const uint64_t base = ((uint64_t)(uint32_t)(acc[4][e] + (lo >> 31)) << 32) | (uint32_t)lo;
+      raw[e] = (int64_t)mid * k64k + (int64_t)base;
     }
   };
 
   // ---- sweep 1: the lane's query maximum over its keys ----
   int64_t mx = kNeg;
+  if (ntile > 0) issue(offk, 0, 0);
+  if (ntile > 1) issue(offk, 64 * HD, 1);
+  // the weight table into LDS behind the first tiles: sweep 2 reads it
+  {
+    const auto rt = buf_rsrc(tab);
+    constexpr int TI = kTabN * 4 / 1024;             // 64 instructions; the last words follow by plain stores
+    for (int i = w; i < TI; i += C::NW) buf_lds16(rt, (char*)U + i * 1024, i * 1024 + lane * 16, 0);
+    if (threadIdx.x < kTabPad - kTabN) U[kTabN + threadIdx.x] = tab[kTabN + threadIdx.x];
+  }
+  double* F = (double*)(smem + C::FO);
+  for (int i = threadIdx.x; i < kTabF; i += 64 * C::NW) F[i] = pre_f(p.lut, i);
+  const bool tab_ok = __builtin_amdgcn_ballot_w64(tab[kTabPad + lane] == 0) == 0;
+  static_assert(kTabBlocks == 64, "one table check word per lane");
+  for (int t = 0, sl = 0; t < ntile; ++t) {
+    if (t == 0 || t + 1 >= ntile) ring_barrier<0>();
+    else ring_barrier<C::LP>();
+    if (t + 2 < ntile) issue(offk, (t + 2) * 64 * HD, sl == 0 ? 2 : sl - 1);
+    const int8_t* kbase = (const int8_t*)ring + sl * C::PB;
+    sl = sl == 2 ? 0 : sl + 1;
+    auto scan = [&](auto full_t) {
 #pragma unroll
-  for (int t = 0; t < NS - 1; ++t)
-    if (t < ntile) issue1(t);
-  for (int t = 0; t < ntile; ++t) {
-    if (k_issuer && t + NS - 2 < ntile)
-      ring_barrier<C::LPK * (NS - 2)>();
-    else
-      ring_barrier<0>();
-    if (t + NS - 1 < ntile) issue1(t + NS - 1);
-    const int8_t* kbase = (const int8_t*)smem + (t % NS) * C::STAGE;
+      for (int i = 0; i < C::KB; ++i) {
+        const int kb = wp * C::KB + i;
+        v4i acc[5];
+        int64_t raw[4];
+        qk(kbase, kb, acc);
+        join(acc, raw);
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      int64_t raw[4];
-      qk(kbase, kb, raw);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (t * 64 + kb * 16 + 4 * c + e <= my_qpos) mx = imax(mx, raw[e]);
-    }
+        for (int e = 0; e < 4; ++e)
+          if (decltype(full_t)::value || t * 64 + kb * 16 + 4 * c + e <= my_qpos) mx = imax(mx, raw[e]);
+      }
+    };
+    if (t * 64 + 63 <= wmin_qpos) scan(std::true_type{});     // wave-uniform: every key is visible to every row
+    else if (t * 64 <= wmax_qpos) scan(std::false_type{});    // some key is visible to some row
   }
   mx = imax(mx, __shfl_xor(mx, 16, 64));
   mx = imax(mx, __shfl_xor(mx, 32, 64));
   ring_barrier<0>();                                 // every wave is done with the ring
+  if constexpr (SW == 2) {                           // the pair's maxima meet in slot 2 (free until K of tile 1)
+    int64_t* xm = (int64_t*)(ring + 2 * C::PB);
+    if (lane < 16) xm[w * 16 + lane] = mx;
+    ring_barrier<0>();
+    mx = imax(mx, xm[(w ^ 1) * 16 + kl]);
+  }
 
   // ---- sweep 2: weights, den, p V ----
-  // (fast: no query of the wave has a negative exponent shift and l2e < 2^31, so no visible key's zf or zf l2e
-  // can wrap: weight_at_nn)
-  const bool fast = tab2 != nullptr && __builtin_amdgcn_ballot_w64(shift < 0) == 0 && p.l2e >= 0 &&
-                    p.l2e < (1LL << 31);
-  const auto rtab = buf_rsrc(tab2 != nullptr ? (const void*)tab2 : (const void*)p.lut);   // (entry, next - entry)
+  const bool fast = tab_ok && __builtin_amdgcn_ballot_w64(shift < 0) == 0 && p.l2e >= 0 && p.l2e < (1LL << 31);
   int64_t den = 0;
   v4i pacc[DB][5];
 #pragma unroll
   for (int d = 0; d < DB; ++d)
 #pragma unroll
     for (int u = 0; u < 5; ++u) pacc[d][u] = v4i{0, 0, 0, 0};
-#pragma unroll
-  for (int t = 0; t < NS - 1; ++t)
-    if (t < ntile) issue2(t);
+  if (ntile > 0) {
+    issue(offk, 0, 0);
+    issue(offv, 0, 1);
+  }
   // fast: zf = rshc(mx - raw, s) = (cz - raw) >> s with cz = mx + 2^(s - 1) (wrapping, as rshc's add), s clamped
-  // to 62 as rshc clamps it; the weight's interpolation reads the (entry, next - entry) pair table in one load
+  // to 62 as rshc clamps it
   const int s62 = (int)imin(imax(shift, 0), 62);
   const int64_t cz = add_wrap(mx, s62 > 0 ? (1LL << (s62 - 1)) : 0);
-  const int wmin_qpos = (int)-wave_max64(-(int64_t)my_qpos);      // the wave's smallest position
-  auto tile2 = [&](int t, auto fast_t, auto full_t) {
-    constexpr bool kFast = decltype(fast_t)::value, kFull = decltype(full_t)::value;   // kFull: every key visible
-    const int8_t* kbase = (const int8_t*)smem + (t % NS) * C::STAGE;
-    const int8_t* vbs = kbase + C::PB;
-    int64_t raw[4][4];
-    int32_t x[4][4];
-    if constexpr (kFast) {
-      // two halves of the tile: the first half's scores, table positions and table loads, then the second half's,
-      // so the second half's MFMAs and integer work run while the first half's table rows are in flight; then the
-      // next stage's request
-      int idx[4][4], n[4][4], rr[4][4];
-      v4i tv[4][4];
+  // the general rule: four weights, or one
+  auto weights_gen = [&](const int64_t (&raw)[4], int32_t (&x)[4]) {
+    WeightAt wa[4];
+    int64_t ta[4], tb[4];
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-#pragma unroll
-      for (int kb = 2 * hf; kb < 2 * hf + 2; ++kb) qk(kbase, kb, raw[kb]);
-#pragma unroll
-      for (int kb = 2 * hf; kb < 2 * hf + 2; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          uint64_t zf = (uint64_t)((cz - raw[kb][e]) >> s62);
-          zf = zf < (48ULL << kFZ) ? zf : (48ULL << kFZ);     // hidden keys (negative) clamp too: inside the table
-          const uint64_t prod = (uint64_t)(uint32_t)zf * (uint64_t)(uint32_t)p.l2e + (1ULL << 27);
-          // n = prod >> 54 and f = (prod >> 28) mod 2^26 from the product's two words
-          const uint32_t ph = (uint32_t)(prod >> 32), pl = (uint32_t)prod;
-          n[kb][e] = (int)(ph >> (28 + kFT2 - 32));
-          const uint32_t f = __builtin_amdgcn_alignbit(ph, pl, 28) & ((1u << kFT2) - 1);
-          idx[kb][e] = n[kb][e] < kZeroN ? (int)(f >> (kFT2 - kExp2Bits)) : 0;
-          rr[kb][e] = (int)(f & ((1u << (kFT2 - kExp2Bits)) - 1));
-        }
-#pragma unroll
-      for (int kb = 2 * hf; kb < 2 * hf + 2; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) tv[kb][e] = buf_load16(rtab, idx[kb][e] * 16);
-      __builtin_amdgcn_sched_barrier(0);
-      }
-      if (t + NS - 1 < ntile) issue2(t + NS - 1);    // after the table loads: waiting for them leaves it in flight
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t av = (int64_t)(((uint64_t)(uint32_t)tv[kb][e][1] << 32) | (uint32_t)tv[kb][e][0]);
-          const int64_t dv = (int64_t)(((uint64_t)(uint32_t)tv[kb][e][3] << 32) | (uint32_t)tv[kb][e][2]);
-          const int64_t v = av + ((dv * rr[kb][e] + (1LL << (kFT2 - kExp2Bits - 1))) >> (kFT2 - kExp2Bits));
-          // rshc(v, 38 + n) for 0 <= v < 2^61: ((v >> (s - 1)) + 1) >> 1 with s = min(38 + n, 62)
-          const int sh2 = min(kExp2One - kFP + n[kb][e], 62) - 1;
-          int32_t w = ((int32_t)(v >> sh2) + 1) >> 1;
-          if (!kFull && t * 64 + kb * 16 + 4 * c + e > my_qpos) w = 0;
-          x[kb][e] = w;
-        }
-    } else {
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) qk(kbase, kb, raw[kb]);
-      WeightAt wa[4][4];
-      int64_t ta[4][4], tb[4][4];
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) wa[kb][e] = weight_at(mx - raw[kb][e], shift, p.l2e);
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          ta[kb][e] = p.lut[wa[kb][e].idx];
-          tb[kb][e] = p.lut[wa[kb][e].idx + 1];
-        }
-      if (t + NS - 1 < ntile) issue2(t + NS - 1);
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          x[kb][e] = t * 64 + kb * 16 + 4 * c + e <= my_qpos ? (int32_t)weight_of(wa[kb][e], ta[kb][e], tb[kb][e]) : 0;
+    for (int e = 0; e < 4; ++e) {
+      wa[e] = weight_at(mx - raw[e], shift, p.l2e);
+      ta[e] = p.lut[wa[e].idx];
+      tb[e] = p.lut[wa[e].idx + 1];
     }
-    v4i pa[3] = {v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}};
-    int32_t dt = 0;                                   // the tile's weight sum: <= 64 2^22, exact in int32
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      // 0 <= x <= 2^22: signed base-256 limbs; limb_lo(x) as a byte is x & 255, the next digit is
-      // (x + 128) >> 8 and the one after it (x + 128 + 2^15) >> 16 (nested floors), so limb i's byte is byte i of
-      // x, x + 128 and x + 32896; four keys' bytes go into one word with two byte permutes and an or
-      uint32_t v0[4], v1[4], v2[4];
+    for (int e = 0; e < 4; ++e) x[e] = (int32_t)weight_of(wa[e], ta[e], tb[e]);
+  };
+  auto weight_gen = [&](int64_t raw) { return (int32_t)attn_weight(mx - raw, shift, p.lut, p.l2e); };
+  auto weights_fast = [&](const int64_t (&raw)[4], int32_t (&x)[4]) {
+    uint32_t f[4], ph[4], u0[4], u1[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        dt += x[kb][e];
-        v0[e] = (uint32_t)x[kb][e];
-        v1[e] = v0[e] + 128u;
-        v2[e] = v0[e] + 32896u;
-      }
-      pa[0][kb] = (int)gather_bytes<0>(v0);
-      pa[1][kb] = (int)gather_bytes<1>(v1);
-      pa[2][kb] = (int)gather_bytes<2>(v2);
+    for (int e = 0; e < 4; ++e) {
+      uint64_t zf = (uint64_t)((cz - raw[e]) >> s62);
+      zf = zf < (48ULL << kFZ) ? zf : (48ULL << kFZ);      // hidden keys (negative) clamp too: inside the table
+      const uint64_t prod = (uint64_t)(uint32_t)zf * (uint64_t)(uint32_t)p.l2e + (1ULL << 27);
+      // t = prod >> 28: n = t >> 26 = prod >> 54 and f = t mod 2^26 from the product's two words
+      ph[e] = (uint32_t)(prod >> 32);
+      f[e] = __builtin_amdgcn_alignbit(ph[e], (uint32_t)prod, 28);        // t mod 2^32
+      pin_v(ph[e]);
+      const uint32_t* u = (const uint32_t*)((const char*)U + ((ph[e] >> 6) & (4 * kTabN - 4)));
+      u0[e] = u[0];
+      u1[e] = u[1];
     }
-    den += dt;
+    bool amb[4];
 #pragma unroll
-    for (int d = 0; d < DB; ++d) {
-      const int row = d * 16 + kl;
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t n = ph[e] >> 22;
+      const uint32_t uc = u0[e] + __umulhi(u1[e] - u0[e], f[e] << 20);
+      const uint32_t sb = (n < 22u ? n : 22u) + 9;         // n > 22: the weight is 0, T only marks the exception
+      const int32_t T = (int32_t)((256u << (n & 31)) - uc);
+      int32_t wf = (int32_t)(0x400000u >> (n & 31)) + (T >> sb);
+      pin_v(wf);
+      x[e] = n > 22u ? 0 : wf;
+      amb[e] = __builtin_amdgcn_ubfe((uint32_t)T, 0, sb) < 2u;
+    }
+    if (__builtin_amdgcn_ballot_w64(amb[0] | amb[1] | amb[2] | amb[3]) != 0) {
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const v4i b = *(const v4i*)(vbs + j * HD * 64 + row * 64 + ((c ^ pre_swzv(row)) * 16));
-#pragma unroll
-        for (int i = 0; i < 3; ++i) pacc[d][i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(pa[i], b, pacc[d][i + j], 0, 0, 0);
-      }
+      for (int e = 0; e < 4; ++e)
+        if (__builtin_amdgcn_ballot_w64(amb[e]) != 0) {
+          // the value from the table's float64 factors: v within 2^12, so v 2^-(38+n) + 1/2 within 2^-26 decides the
+          // weight unless it lies that close to an integer (then the int64 table itself)
+          const uint32_t i0 = (f[e] >> 12) & (kTabN - 1), i1 = i0 + 1;
+          const double a = F[i0 >> 7] * F[129 + (i0 & 127)], b = F[i1 >> 7] * F[129 + (i1 & 127)];
+          const double v = a + (b - a) * ((double)(int32_t)(f[e] & 4095u) * (1.0 / 4096.0));
+          const double tt = ldexp(v, -(kExp2One - kFP) - (int)(ph[e] >> 22)) + 0.5;
+          const int32_t wi = (int32_t)tt;
+          const double fr = tt - (double)wi;
+          x[e] = amb[e] ? wi : x[e];
+          if (__builtin_amdgcn_ballot_w64(amb[e] && (fr < 0x1p-25 || fr > 1.0 - 0x1p-25)) != 0)
+            x[e] = amb[e] ? weight_gen(raw[e]) : x[e];
+        }
     }
   };
   auto sweep2 = [&](auto fast_t) {
+    constexpr bool kFast = decltype(fast_t)::value;
+    uint32_t* xp = (uint32_t*)(smem + C::XO) + wr * (3 * 16 * 16);   // the pair's p limbs
+    int ks = 0;                                      // slot of K of this tile; V's is the next, K's of t + 1 the third
     for (int t = 0; t < ntile; ++t) {
-      if (t + NS - 2 < ntile)
-        ring_barrier<C::LPT * (NS - 2)>();
-      else
-        ring_barrier<0>();
-      if (t * 64 + 63 <= wmin_qpos)               // wave-uniform: every key of the tile is visible to every query
-        tile2(t, fast_t, std::true_type{});
-      else
-        tile2(t, fast_t, std::false_type{});
+      const int vs = ks == 2 ? 0 : ks + 1, ns = vs == 2 ? 0 : vs + 1;
+      // K of this tile is in and every wave is done with V of the tile before
+      ring_barrier<C::LP>();
+      if (t + 1 < ntile) issue(offk, (t + 1) * 64 * HD, ns);
+      const int8_t* kbase = (const int8_t*)ring + ks * C::PB;
+      const int8_t* vbs = (const int8_t*)ring + vs * C::PB;
+      const bool some = t * 64 <= wmax_qpos;         // wave-uniform
+      const bool full = t * 64 + 63 <= wmin_qpos;    // wave-uniform: every key of the tile is visible to every query
+      v4i pa[3] = {v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}};
+      if (some) {
+        int32_t dt = 0;                              // the tile's weight sum: <= 64 2^22, exact in int32
+        uint32_t pw[3][C::KB];
+        v4i acc[2][5];
+        qk(kbase, wp * C::KB, acc[0]);
+#pragma unroll
+        for (int i = 0; i < C::KB; ++i) {
+          const int kb = wp * C::KB + i;
+          int64_t raw[4];
+          int32_t x[4];
+          if (i + 1 < C::KB) qk(kbase, kb + 1, acc[(i + 1) & 1]);
+          join(acc[i & 1], raw);
+          if constexpr (kFast) weights_fast(raw, x);
+          else weights_gen(raw, x);
+          if (!full) {
+            const int key0 = t * 64 + kb * 16 + 4 * c;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = key0 + e <= my_qpos ? x[e] : 0;
+          }
+          dt += x[0] + x[1];
+          dt += x[2] + x[3];
+          limb_words(x, pw[0][i], pw[1][i], pw[2][i]);
+        }
+        den += dt;
+#pragma unroll
+        for (int l = 0; l < 3; ++l)
+          if constexpr (SW == 1) {
+            pa[l] = v4i{(int)pw[l][0], (int)pw[l][C::KB - 3], (int)pw[l][C::KB - 2], (int)pw[l][C::KB - 1]};
+          } else {
+            // 16 bytes per (limb, query, chunk): word kb of lane (query kl, chunk c)
+            *(uint2*)&xp[((l * 16 + kl) * 4 + (c ^ ((kl >> 2) & 3))) * 4 + wp * 2] = uint2{pw[l][0], pw[l][1]};
+          }
+      }
+      // V of this tile is in and every wave is done with K of this tile
+      if (t + 1 < ntile) ring_barrier<C::LP>();
+      else ring_barrier<0>();
+      if (t + 1 < ntile) issue(offv, (t + 1) * 64, ks);
+      ks = ns;
+      if (some) {
+        if constexpr (SW == 2) {
+#pragma unroll
+          for (int l = 0; l < 3; ++l) pa[l] = *(const v4i*)&xp[((l * 16 + kl) * 4 + (c ^ ((kl >> 2) & 3))) * 4];
+        }
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+          const int row = (wp * DB + d) * 16 + kl;
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            const v4i b = *(const v4i*)(vbs + j * HD * 64 + row * 64 + ((c ^ pre_swzv(row)) * 16));
+#pragma unroll
+            for (int i = 0; i < 3; ++i) pacc[d][i + j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(pa[i], b, pacc[d][i + j], 0, 0, 0);
+          }
+        }
+      }
     }
   };
   if (fast)
@@ -1929,10 +2016,17 @@ __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArg
     sweep2(std::false_type{});
   den += __shfl_xor(den, 16, 64);
   den += __shfl_xor(den, 32, 64);
-  // outputs: lane holds queries 4 c + e of the wave, dims 16 d + kl
+  if constexpr (SW == 2) {                           // the pair's weight sums (the ring is free: after every wave's last read)
+    int64_t* xd = (int64_t*)ring;
+    ring_barrier<0>();
+    if (lane < 16) xd[w * 16 + lane] = den;
+    ring_barrier<0>();
+    den += xd[(w ^ 1) * 16 + kl];
+  }
+  // outputs: lane holds queries 4 c + e of the rows, dims 16 d + kl
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int qw = 4 * c + e, r = q0 + 16 * w + qw;
+    const int qw = 4 * c + e, r = q0 + 16 * wr + qw;
     const int64_t dq = __shfl(den, qw, 64);
     if (r >= p.nq) continue;
 #pragma unroll
@@ -1940,9 +2034,9 @@ __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArg
       int64_t v = 0;
 #pragma unroll
       for (int u = 0; u < 5; ++u) v += (int64_t)pacc[d][u][e] << (8 * u);
-      p.num[z * p.snum_tile + (int64_t)r * p.snum_row + d * 16 + kl] = v;
+      p.num[z * p.snum_tile + (int64_t)r * p.snum_row + (wp * DB + d) * 16 + kl] = v;
     }
-    if (kl == 0) p.den[z * p.sden_tile + r] = dq;
+    if (kl == 0 && wp == 0) p.den[z * p.sden_tile + r] = dq;
   }
 }
 
@@ -2280,17 +2374,19 @@ extern "C" int bx_exact_attn_prefill(const int32_t* qg, int64_t sq_z, int64_t sq
                (long long)tmp_bytes, (long long)need);
     const int Sp = (S + 63) / 64 * 64;
     int8_t* pl = (int8_t*)tmp;
-    const int64_t units = (int64_t)Z * Sp * (HD / 16) + (int64_t)Z * (Sp / 4) * (HD / 4) + (1LL << kExp2Bits);
-    int64_t* tab2 = (int64_t*)(pl + pre2_planes(Z, S, HD));
-    pre_split_kernel<<<(int)std::min<int64_t>((units + 255) / 256, 8192), 256, 0, st>>>(
-        p, pl, pl + (int64_t)Z * 3 * Sp * HD, tab2, Z, Sp, HD);
+    const int64_t units = (int64_t)Z * Sp * (HD / 16) + (int64_t)Z * (Sp / 4) * (HD / 4);
+    uint32_t* tab = (uint32_t*)(pl + pre2_planes(Z, S, HD));
+    pre_split_kernel<<<kTabBlocks + (int)std::min<int64_t>((units + 255) / 256, 8192), 256, 0, st>>>(
+        p, pl, pl + (int64_t)Z * 3 * Sp * HD, tab, Z, Sp, HD);
     if (int rc = check_launch("pre_split_kernel")) return rc;
     if (HD == 64) {
       allow_lds_attn((const void*)attn_pre2_kernel<64>, Pre2<64>::LDS);
-      attn_pre2_kernel<64><<<Z * ((gT + 127) / 128), 512, Pre2<64>::LDS, st>>>(p, pl, Z, Sp, (const char*)tab2);
+      attn_pre2_kernel<64><<<Z * ((gT + Pre2<64>::QR - 1) / Pre2<64>::QR), 64 * Pre2<64>::NW, Pre2<64>::LDS, st>>>(
+          p, pl, Z, Sp, tab);
     } else {
       allow_lds_attn((const void*)attn_pre2_kernel<128>, Pre2<128>::LDS);
-      attn_pre2_kernel<128><<<Z * ((gT + 63) / 64), 256, Pre2<128>::LDS, st>>>(p, pl, Z, Sp, (const char*)tab2);
+      attn_pre2_kernel<128><<<Z * ((gT + Pre2<128>::QR - 1) / Pre2<128>::QR), 64 * Pre2<128>::NW, Pre2<128>::LDS, st>>>(
+          p, pl, Z, Sp, tab);
     }
     return check_launch("attn_pre2_kernel");
   }

@@ -195,6 +195,62 @@ def test_prefill_attention_full_size(dev, HD, T, Z):
                                                                                      ref_den[0])
 
 
+@pytest.mark.parametrize("HD", [64, 128])
+@pytest.mark.parametrize("table", ["exp2", "noisy", "steps"])
+def test_prefill_weight_positions(dev, HD, table):
+    """The limb-plane form's short weight rule at the table positions where it can go wrong, against the oracle:
+    scores placed one by one (z = max - raw exactly, shift 0) on both sides of every integer n (the weight's binade
+    changes, n = 22 / 23 where it becomes 1 and 0), at table entries, and 1400 positions in the first three binades
+    (a few of them within the 32-bit table's uncertainty of a rounding boundary). "noisy": a table whose entries are
+    off by more than its float64 factors allow; "steps": one outside [2^59, 2^60]; both take the general rule."""
+    from bitexact.exact.attention import prefill
+    l2e = R.L2E28_HD[HD]
+    rng = np.random.default_rng(HD)
+    lut = R.exp2_table().copy()
+    if table == "noisy":
+        lut[1:-1] += rng.integers(-(1 << 20), 1 << 20, len(lut) - 2)
+    elif table == "steps":
+        lut = (lut >> 3) << 2
+    zf = [0]
+    for n in range(27):
+        for f in (0, 1, 4095, 4096, 1 << 25):
+            z0 = (((n << 26) + f) << 28) // l2e
+            zf += [z0 - 1, z0, z0 + 1, z0 + 2]
+    zf = np.concatenate([np.clip(np.array(zf, dtype=np.int64), 0, None), rng.integers(0, 3 << 26, 1400)])
+    rng.shuffle(zf)
+    S, T, Z = len(zf), 70, 1
+    K = np.zeros((Z, S, HD), np.int64)
+    K[0, :, 0], K[0, :, 1] = (-zf) >> 20, (-zf) & ((1 << 20) - 1)     # raw = 2^20 K0 + K1 = -zf
+    V = rng.integers(-R.LIM3, R.LIM3 + 1, (Z, S, HD))
+    q = np.zeros((Z, T, HD), np.int64)
+    q[0, :, 0], q[0, :, 1] = 1 << 20, 1
+    sh = np.full((Z, T, 1), -6)                                        # shift FK + 3 - FZ - sh = 0
+    qpos = np.sort(rng.integers(0, S, (Z, T, 1)), axis=1)
+    ref_num, ref_den = R.attention_prefill(q, sh, K, V, qpos, lut, l2e)
+    t32 = lambda x: torch.from_numpy(x).to(torch.int32).to(dev)
+    num, den = prefill(t32(q), torch.from_numpy(sh).to(dev), t32(K), t32(V), torch.from_numpy(qpos).to(dev),
+                       torch.from_numpy(lut).to(dev), l2e)
+    assert np.array_equal(den.cpu().numpy(), ref_den) and np.array_equal(num.cpu().numpy(), ref_num)
+
+
+@pytest.mark.parametrize("HD,T", [(64, 1), (64, 31), (64, 33), (128, 15), (128, 17), (64, 65)])
+def test_prefill_row_tiles(dev, HD, T):
+    """Row tiles at their edges (128 rows at head_dim 64, 64 at 128; 4 T rows) with key tiles whole, one short and
+    one over, rows that see no key (position -1) among them, against the register-staged form."""
+    from bitexact.exact.attention import prefill
+    g = torch.Generator().manual_seed(T)
+    Z, S = 3, T + 63
+    qg = torch.randint(-(1 << 22), (1 << 22) + 1, (Z, 4 * T, HD), generator=g).to(torch.int32).to(dev)
+    shg = torch.randint(-24, -18, (Z, 4 * T, 1), generator=g).to(dev)
+    K = (torch.randn(Z, S, HD, generator=g) * 2 ** 17).to(torch.int32).to(dev)
+    V = torch.randint(-R.LIM3, R.LIM3 + 1, (Z, S, HD), generator=g).to(torch.int32).to(dev)
+    qpos = torch.randint(-1, S, (Z, 4 * T, 1), generator=g).to(dev)
+    args = (qg, shg, K, V, qpos, _lut(dev), R.L2E28_HD[HD])
+    n1, d1 = prefill(*args, planes=True)
+    n2, d2 = prefill(*args, planes=False)
+    assert torch.equal(n1, n2) and torch.equal(d1, d2)
+
+
 def test_bmm_exact(dev):
     from bitexact.bmm import bmm
     g = torch.Generator().manual_seed(0)
