@@ -30,9 +30,26 @@ def _attend_fake(q, sh, qpos, cache, bt, rmap, lut, l2e, nsplit):
     return empty((R, HKV, M, HD), torch.long, q), empty((R, HKV, M, 1), torch.long, q)
 
 
+# The grouped form for at least ROWS_MIN (token, KV head, dim)s and ROWS_PER_SEQ tokens per block-table row. Measured (8
+# KV heads of 64, grouped against per-token, us): 8 sequences of 512 181 / 1116, of 32 27 / 45, of 32 past 1000 keys 119
+# / 178, one of 256 41 / 56; below the line it loses: 8 of 16 26 / 23, one of 64 past 2000 keys 196 / 88 (two tiles per
+# head: 16 blocks). Heads of 128 cross at half the tokens (8 of 16 25 / 30).
+ROWS_PER_SEQ, ROWS_MIN = 8, 96 * 1024
+
+
+def rows_scratch(R, HKV, M, HD, nrow, keys):
+    """Scratch bytes of the grouped form (bx_exact_attn_paged_rows) where attend takes it, else 0: prefill steps (the
+    table's row count bounds the sequences, the tokens' own rows being known on the device only) of enough tokens for
+    its tiles to fill the chip, whose sequences' limb planes fit that form's 1 GiB."""
+    if R * HKV * HD < ROWS_MIN or R < ROWS_PER_SEQ * nrow:
+        return 0
+    return _hip.lib().bx_attn_paged_rows_scratch(R, nrow, HKV, M, HD, keys)
+
+
 @op("attend_exact(Tensor q, Tensor sh, Tensor qpos, Tensor cache, Tensor bt, Tensor rmap, Tensor lut, int l2e, "
     "int nsplit) -> (Tensor, Tensor)", _attend_fake)
 def _attend(q, sh, qpos, cache, bt, rmap, lut, l2e, nsplit):
+    """nsplit 0: chosen here (the grouped form for prefills, else default_nsplit)."""
     _hip.require_cuda(q, sh, qpos, cache, bt, rmap, lut)
     R, HKV, M, HD = q.shape
     assert M <= BQ and cache.shape[1] == HKV and cache.shape[3] >= 6 * HD and cache.stride(3) == 1
@@ -42,6 +59,16 @@ def _attend(q, sh, qpos, cache, bt, rmap, lut, l2e, nsplit):
     rmap, lut = rmap.contiguous().long(), lut.contiguous().long()
     num = torch.empty(R, HKV, M, HD, dtype=torch.long, device=q.device)
     den = torch.empty(R, HKV, M, 1, dtype=torch.long, device=q.device)
+    need = rows_scratch(R, HKV, M, HD, bt.shape[0], bt.shape[1] * cache.shape[2]) if nsplit == 0 else 0
+    if need > 0 and q.data_ptr() % 16 == 0:
+        tmp, tmpb = _hip.scratch(q.device, need)
+        _hip.call("bx_exact_attn_paged_rows", _hip.ptr(q), _hip.ptr(sh), _hip.ptr(qpos), qpos.stride(0), _hip.ptr(cache),
+                  cache.stride(0), cache.stride(1), cache.stride(2), cache.shape[2], _hip.ptr(bt), bt.stride(0),
+                  bt.shape[0], bt.shape[1], _hip.ptr(rmap), _hip.ptr(lut), int(l2e), _hip.ptr(num), _hip.ptr(den), R,
+                  HKV, M, HD, _hip.ptr(tmp), tmpb, _hip.stream_of(q))
+        return num, den
+    if nsplit == 0:
+        nsplit = default_nsplit(R, HKV, bt.shape[1], cache.shape[2])
     ws, wsb = _hip.workspace(q.device, _hip.lib().bx_attn_paged_workspace(R, HKV, M, HD) if nsplit > 1 else 0)
     _hip.call("bx_exact_attn_paged", _hip.ptr(q), _hip.ptr(sh), _hip.ptr(qpos), qpos.stride(0), _hip.ptr(cache),
               cache.stride(0), cache.stride(1), cache.stride(2), cache.shape[2], _hip.ptr(bt), bt.stride(0),
@@ -51,9 +78,8 @@ def _attend(q, sh, qpos, cache, bt, rmap, lut, l2e, nsplit):
 
 
 def attend(q, sh, qpos, cache, bt, rmap, lut, l2e, nsplit=None, bn=64, warps=4):
-    if nsplit is None:
-        nsplit = default_nsplit(q.shape[0], q.shape[1], bt.shape[1], cache.shape[2])
-    return _attend(q, sh, qpos, cache, bt, rmap, lut, int(l2e), int(nsplit))
+    assert nsplit is None or nsplit >= 1, "nsplit in [1, 64]"
+    return _attend(q, sh, qpos, cache, bt, rmap, lut, int(l2e), 0 if nsplit is None else int(nsplit))
 
 
 def rope_fusable(N, HKV, H, nblk, bs):

@@ -1661,6 +1661,104 @@ __global__ __launch_bounds__(256) void pre_split_kernel(AttnArgs p, int8_t* kp, 
   }
 }
 
+// ---- the same attention over the paged cache, for steps of many tokens per sequence ----
+// rows_group_kernel sorts the step's token rows by their block-table row (stable) and cuts each sequence's into
+// tiles of TT tokens; paged_planes_kernel writes the sequences' cached K and V limbs as the planes above;
+// attn_pre2_kernel then runs a (tile, KV head) per block. One wave per table row s counts the tokens of smaller rows
+// (its start in perm) and its own, then writes them in order. Tile slots [start / TT + s, (start + count) / TT + s + 1)
+// belong to sequence s: at least ceil(count / TT) of them, never two sequences' (the spare ones hold 0 tokens).
+struct RowMap {
+  const int32_t* perm;      // [R] token rows, sorted
+  const int4* slots;        // [nslot] (start in perm, tokens, table row, 0)
+  const int32_t* klen;      // [nrow] keys of each sequence visible to some token
+  int64_t sqpos;
+  int nslot, M, hkv;
+};
+
+__global__ __launch_bounds__(256) void rows_group_kernel(const int64_t* rmap, const int64_t* qpos, int64_t sqpos, int R,
+                                                         int M, int nrow, int S, int TT, int nslot, int32_t* perm,
+                                                         int4* slots, int32_t* klen) {
+  const int s = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (s >= nrow) return;
+  constexpr int U = 8;
+  int lt = 0, eq = 0;
+  for (int i0 = 0; i0 < R; i0 += 64 * U) {
+    int64_t r[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) r[u] = i0 + u * 64 + lane < R ? rmap[i0 + u * 64 + lane] : nrow;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      lt += __popcll(__builtin_amdgcn_ballot_w64(r[u] < s));
+      eq += __popcll(__builtin_amdgcn_ballot_w64(r[u] == s));
+    }
+  }
+  int at = lt;
+  int64_t kmax = -1;
+  for (int i0 = 0; eq > 0 && i0 < R; i0 += 64 * U) {
+    int64_t r[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) r[u] = i0 + u * 64 + lane < R ? rmap[i0 + u * 64 + lane] : nrow;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint64_t m = __builtin_amdgcn_ballot_w64(r[u] == s);
+      if (r[u] == s) {
+        const int i = i0 + u * 64 + lane;
+        perm[at + __popcll(m & ((1ULL << lane) - 1))] = i;
+        for (int j = 0; j < M; ++j) kmax = imax(kmax, qpos[i * sqpos + j]);
+      }
+      at += __popcll(m);
+    }
+  }
+  kmax = wave_max64(kmax);
+  const int first = lt / TT + s, next = s + 1 < nrow ? (lt + eq) / TT + s + 1 : nslot;
+  for (int j = first + lane; j < next; j += 64) {
+    const int o = (j - first) * TT;
+    slots[j] = int4{lt + o, min(max(eq - o, 0), TT), s, 0};
+  }
+  if (lane == 0) klen[s] = (int)imin(kmax + 1, S);
+}
+
+// Block kTabBlocks + ((row HKV + h) ntile + tile): 64 keys of one (sequence, KV head). K rows are copied as they
+// stand; V goes 4 keys x 4 dims at a time through a byte transpose. Keys past klen are left as they are: no query
+// sees them, so their weights are 0.
+template <int HD>
+__global__ __launch_bounds__(256) void paged_planes_kernel(AttnArgs p, const int32_t* klen, int8_t* kp, int8_t* vp,
+                                                           uint32_t* tab, int Sp, int ntile) {
+  if (blockIdx.x < kTabBlocks) {
+    pre_table_block(p.lut, tab, blockIdx.x);
+    return;
+  }
+  const int b = blockIdx.x - kTabBlocks, z = b / ntile, k0 = (b - z * ntile) * 64;
+  const int row = z / p.hkv, h = z - row * p.hkv;
+  const int nk = min(klen[row] - k0, 64);
+  if (nk <= 0) return;
+  __shared__ int64_t s_off[64];
+  if (threadIdx.x < 64) {
+    const int s = k0 + min((int)threadIdx.x, nk - 1);
+    s_off[threadIdx.x] = (int64_t)p.bt[row * p.sbt + s / p.bs] * p.sc_nb + (int64_t)h * p.sc_h + (int64_t)(s % p.bs) * p.sc_bs;
+  }
+  __syncthreads();
+  constexpr int CH = 3 * HD / 16;
+  for (int u = threadIdx.x; u < 64 * CH; u += 256) {
+    const int k = u / CH, ch = u - k * CH, j = ch / (HD / 16), cc = ch - j * (HD / 16);
+    if (k < nk)
+      *(v4i*)(kp + (((int64_t)z * 3 + j) * Sp + k0 + k) * HD + cc * 16) = *(const v4i*)(p.cache + s_off[k] + ch * 16);
+  }
+  for (int u = threadIdx.x; u < 16 * 3 * (HD / 4); u += 256) {
+    const int s4 = u & 15, jd = u >> 4, j = jd / (HD / 4), d4 = jd - j * (HD / 4);
+    uint32_t y[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) y[m] = *(const uint32_t*)(p.cache + s_off[s4 * 4 + m] + (3 + j) * HD + d4 * 4);
+    const uint32_t a0 = __builtin_amdgcn_perm(y[1], y[0], 0x05010400u), a1 = __builtin_amdgcn_perm(y[1], y[0], 0x07030602u);
+    const uint32_t b0 = __builtin_amdgcn_perm(y[3], y[2], 0x05010400u), b1 = __builtin_amdgcn_perm(y[3], y[2], 0x07030602u);
+    const uint32_t o[4] = {__builtin_amdgcn_perm(b0, a0, 0x05040100u), __builtin_amdgcn_perm(b0, a0, 0x07060302u),
+                           __builtin_amdgcn_perm(b1, a1, 0x05040100u), __builtin_amdgcn_perm(b1, a1, 0x07060302u)};
+    int8_t* dst = vp + (((int64_t)z * 3 + j) * HD + d4 * 4) * Sp + k0 + pre_vpos(s4 * 4);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) *(uint32_t*)(dst + (int64_t)d * Sp) = o[d];
+  }
+}
+
 // The three signed base-256 limbs of four values 0 <= x <= 2^22, each as one word of four bytes: byte i of x + 0x8080
 // is limb i + 128 for i = 0, 1 and limb 2 for i = 2 (the adds' carries are the digits' borrows); the bytes of the
 // four words are transposed with seven v_perm_b32.
@@ -1729,9 +1827,10 @@ __device__ __forceinline__ void pin_v(uint32_t& x) { asm("" : "+v"(x)); }
 // 32 / 8 heads of 64), the lanes' lines missing the 32 KiB L1. Now 198 us (1337 tokens, heads of 128: 233 -> 157):
 // bound by the integer work per score (about 40 VALU instructions), with sweep 1 about 55 us of it. The second-step
 // values come from LDS too because one wave's memory round trip holds its block at the tile's barrier (238 us).
-template <int HD>
+// ROWS: the paged form. Block (slot, KV head h); the block's query i is query i % M of the slot's token i / M.
+template <int HD, bool ROWS>
 __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArgs p, const int8_t* planes, int Z,
-                                                                         int Sp, const uint32_t* tab) {
+                                                                         int Sp, const uint32_t* tab, RowMap rm) {
   using C = Pre2<HD>;
   constexpr int QR = C::QR, SW = C::SW;
   constexpr int KK = C::KK, DB = C::DB, SL = C::SLOTS;
@@ -1739,19 +1838,44 @@ __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArg
   uint32_t* U = (uint32_t*)smem;
   char* ring = smem + C::RO;
   __shared__ int s_kend;
-  const int tiles = (p.nq + QR - 1) / QR;
-  const int z = blockIdx.x % Z, q0 = (tiles - 1 - blockIdx.x / Z) * QR;    // late (long) row tiles first
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kl = lane & 15, c = lane >> 4;
   const int wr = w / SW, wp = w % SW;                // row group, part of it
+  // the group z of the planes, and where query i of the block lives: (token row, query) group g, row r
+  int z, q0 = 0, h = 0;
+  int4 slot = {};
+  if constexpr (ROWS) {
+    slot = rm.slots[rm.nslot - 1 - (int)(blockIdx.x / rm.hkv)];            // late (long) tiles of a sequence first
+    if (slot.y == 0) return;                         // the whole block: a spare slot
+    h = blockIdx.x % rm.hkv;
+    z = slot.z * rm.hkv + h;
+  } else {
+    const int tiles = (p.nq + QR - 1) / QR;
+    z = blockIdx.x % Z;
+    q0 = (tiles - 1 - blockIdx.x / Z) * QR;          // late (long) row tiles first
+  }
+  auto locate = [&](int i, int64_t& g, int& r) {     // false: no such query (g, r then name a readable one)
+    if constexpr (ROWS) {
+      const int tok = i / rm.M;
+      r = i - tok * rm.M;
+      g = (int64_t)rm.perm[slot.x + min(tok, slot.y - 1)] * rm.hkv + h;
+      return tok < slot.y;
+    } else {
+      r = min(q0 + i, p.nq - 1);
+      g = z;
+      return q0 + i < p.nq;
+    }
+  };
   const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(planes), (short)0, kBufRange, 0x00020000);
   const int64_t vbase = (int64_t)Z * 3 * Sp * HD;
 
   // the lane's query (B operand rows) and its position / exponent
-  const int qr = q0 + 16 * wr + kl;
+  int64_t qg;
+  int qr;
+  const bool live = locate(16 * wr + kl, qg, qr);
   v4i qb[3][KK];
   {
-    const int32_t* qp = p.q + (int64_t)z * p.sq_tile + (int64_t)min(qr, p.nq - 1) * p.sq_row;
+    const int32_t* qp = p.q + qg * p.sq_tile + (int64_t)qr * p.sq_row;
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
       uint32_t l[3][4];
@@ -1761,11 +1885,10 @@ __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArg
       for (int i = 0; i < 3; ++i) qb[i][kk] = v4i{(int)l[i][0], (int)l[i][1], (int)l[i][2], (int)l[i][3]};
     }
   }
-  const bool live = qr < p.nq;
   // (positions past S - 1 see every key: the caller's contract keeps qpos < S, so the clamp changes nothing)
   const int my_qpos =
-      live ? (int)imin(p.qpos[(z / p.qpos_div) * p.qpos_tile + (int64_t)qr * p.qpos_row], (int64_t)p.S) : -1;
-  const int64_t shift = live ? (int64_t)(kFK + 3 - kFZ) - p.sh[z * p.sh_tile + qr] : 0;
+      live ? (int)imin(p.qpos[(qg / p.qpos_div) * p.qpos_tile + (int64_t)qr * p.qpos_row], (int64_t)p.S) : -1;
+  const int64_t shift = live ? (int64_t)(kFK + 3 - kFZ) - p.sh[qg * p.sh_tile + qr] : 0;
   if (threadIdx.x == 0) s_kend = 0;
   __syncthreads();
   const int wmax_qpos = (int)wave_max64(my_qpos);    // the rows' largest position
@@ -2026,17 +2149,19 @@ __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArg
   // outputs: lane holds queries 4 c + e of the rows, dims 16 d + kl
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int qw = 4 * c + e, r = q0 + 16 * wr + qw;
+    const int qw = 4 * c + e;
     const int64_t dq = __shfl(den, qw, 64);
-    if (r >= p.nq) continue;
+    int64_t g;
+    int r;
+    if (!locate(16 * wr + qw, g, r)) continue;
 #pragma unroll
     for (int d = 0; d < DB; ++d) {
       int64_t v = 0;
 #pragma unroll
       for (int u = 0; u < 5; ++u) v += (int64_t)pacc[d][u][e] << (8 * u);
-      p.num[z * p.snum_tile + (int64_t)r * p.snum_row + (wp * DB + d) * 16 + kl] = v;
+      p.num[g * p.snum_tile + (int64_t)r * p.snum_row + (wp * DB + d) * 16 + kl] = v;
     }
-    if (kl == 0 && wp == 0) p.den[z * p.sden_tile + r] = dq;
+    if (kl == 0 && wp == 0) p.den[g * p.sden_tile + r] = dq;
   }
 }
 
@@ -2342,6 +2467,86 @@ extern "C" int64_t bx_attn_prefill_scratch(int32_t Z, int32_t S, int32_t HD) {
   return b < kBufRange - 16 ? b : 0;                 // larger: the register-staged form (no scratch)
 }
 
+// bx_exact_attn_paged_rows's scratch: the token order, the tile slots and key counts, the weight table, the planes
+struct RowsLayout {
+  int TT, nslot, Sp;
+  int64_t slots, klen, tab, planes, total;   // byte offsets (perm at 0)
+};
+static RowsLayout rows_layout(int64_t R, int64_t nrow, int64_t HKV, int64_t M, int64_t HD, int64_t keys) {
+  RowsLayout l;
+  l.TT = (HD == 64 ? Pre2<64>::QR : Pre2<128>::QR) / (int)M;
+  l.nslot = (int)(R / l.TT + nrow);
+  l.Sp = (int)((keys + 63) / 64 * 64);
+  auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
+  l.slots = up(R * 4);
+  l.klen = l.slots + up(l.nslot * 16LL);
+  l.tab = l.klen + up(nrow * 4);
+  l.planes = l.tab + up(4LL * (kTabPad + kTabBlocks));
+  l.total = l.planes + 6 * nrow * HKV * l.Sp * HD;
+  return l;
+}
+constexpr int64_t kRowsScratchMax = 1LL << 30;
+
+extern "C" int64_t bx_attn_paged_rows_scratch(int32_t R, int32_t nrow, int32_t HKV, int32_t M, int32_t HD, int32_t keys) {
+  if (R <= 0 || nrow <= 0 || HKV <= 0 || M < 1 || M > 4 || (HD != 64 && HD != 128) || keys <= 0 || keys >= 43690) return 0;
+  const int64_t b = rows_layout(R, nrow, HKV, M, HD, keys).total;
+  return b <= kRowsScratchMax ? b : 0;
+}
+
+extern "C" int bx_exact_attn_paged_rows(const int32_t* q, const int64_t* sh, const int64_t* qpos, int64_t sqpos_r,
+                                        const int8_t* cache, int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs,
+                                        const int32_t* bt, int64_t sbt, int32_t nrow, int32_t nblk, const int64_t* rmap,
+                                        const int64_t* lut, int64_t l2e, int64_t* num, int64_t* den, int32_t R,
+                                        int32_t HKV, int32_t M, int32_t HD, void* tmp, int64_t tmp_bytes,
+                                        bx_stream_t stream) {
+  BX_REQUIRE(R >= 0 && nrow >= 0 && HKV > 0 && M >= 1 && M <= 4, "need 1 <= M <= 4 queries per (row, KV head)");
+  BX_REQUIRE(HD == 64 || HD == 128, "head_dim must be 64 or 128");
+  BX_REQUIRE(nblk >= 0 && bs > 0 && (int64_t)nblk * bs < 43690, "keys per row must stay below 43690");
+  BX_REQUIRE(sc_bs >= 6 * HD && sc_nb % 16 == 0 && sc_h % 16 == 0 && sc_bs % 16 == 0 && ((uintptr_t)cache & 15) == 0,
+             "cache rows must hold the 6 HD limb bytes, 16-byte aligned");
+  BX_REQUIRE(q && sh && qpos && bt && rmap && lut && num && den, "null pointer");
+  BX_REQUIRE(((uintptr_t)q & 15) == 0, "q must be 16-byte aligned");
+  if (R == 0) return BX_OK;
+  BX_REQUIRE(nrow > 0 && nblk > 0, "empty block table");
+  const RowsLayout l = rows_layout(R, nrow, HKV, M, HD, (int64_t)nblk * bs);
+  BX_REQUIRE(l.total <= kRowsScratchMax, "limb planes above %lld bytes: use bx_exact_attn_paged", (long long)kRowsScratchMax);
+  BX_REQUIRE(tmp && tmp_bytes >= l.total && ((uintptr_t)tmp & 15) == 0, "scratch too small (%lld < %lld) or not 16-byte aligned",
+             (long long)tmp_bytes, (long long)l.total);
+  char* t = (char*)tmp;
+  int32_t* perm = (int32_t*)t;
+  int4* slots = (int4*)(t + l.slots);
+  int32_t* klen = (int32_t*)(t + l.klen);
+  uint32_t* tab = (uint32_t*)(t + l.tab);
+  int8_t* kp = (int8_t*)(t + l.planes);
+  int8_t* vp = kp + 3LL * nrow * HKV * l.Sp * HD;
+  AttnArgs p = {};
+  p.q = q; p.sq_tile = (int64_t)M * HD; p.sq_row = HD;
+  p.sh = sh; p.sh_tile = M;
+  p.qpos = qpos; p.qpos_tile = sqpos_r; p.qpos_row = 1; p.qpos_div = HKV; p.nq = M;
+  p.cache = cache; p.sc_nb = sc_nb; p.sc_h = sc_h; p.sc_bs = sc_bs; p.bt = bt; p.sbt = sbt;
+  p.bs = bs; p.hkv = HKV; p.nblk = nblk; p.S = nblk * bs;
+  p.lut = lut; p.l2e = l2e;
+  p.num = num; p.den = den; p.snum_tile = (int64_t)M * HD; p.snum_row = HD; p.sden_tile = M;
+  p.nsplit = 1;
+  hipStream_t st = (hipStream_t)stream;
+  rows_group_kernel<<<(nrow + 3) / 4, 256, 0, st>>>(rmap, qpos, sqpos_r, R, M, nrow, p.S, l.TT, l.nslot, perm, slots, klen);
+  if (int rc = check_launch("rows_group_kernel")) return rc;
+  const int ntile = l.Sp / 64, Z = nrow * HKV;
+  const RowMap rm = {perm, slots, klen, sqpos_r, l.nslot, M, HKV};
+  if (HD == 64) {
+    paged_planes_kernel<64><<<kTabBlocks + Z * ntile, 256, 0, st>>>(p, klen, kp, vp, tab, l.Sp, ntile);
+    if (int rc = check_launch("paged_planes_kernel")) return rc;
+    allow_lds_attn((const void*)attn_pre2_kernel<64, true>, Pre2<64>::LDS);
+    attn_pre2_kernel<64, true><<<l.nslot * HKV, 64 * Pre2<64>::NW, Pre2<64>::LDS, st>>>(p, kp, Z, l.Sp, tab, rm);
+  } else {
+    paged_planes_kernel<128><<<kTabBlocks + Z * ntile, 256, 0, st>>>(p, klen, kp, vp, tab, l.Sp, ntile);
+    if (int rc = check_launch("paged_planes_kernel")) return rc;
+    allow_lds_attn((const void*)attn_pre2_kernel<128, true>, Pre2<128>::LDS);
+    attn_pre2_kernel<128, true><<<l.nslot * HKV, 64 * Pre2<128>::NW, Pre2<128>::LDS, st>>>(p, kp, Z, l.Sp, tab, rm);
+  }
+  return check_launch("attn_pre2_kernel(rows)");
+}
+
 extern "C" int bx_exact_attn_prefill(const int32_t* qg, int64_t sq_z, int64_t sq_row, const int64_t* shg,
                                      int64_t ssh_z, const int64_t* qpos, int64_t sqpos_z, int64_t sqpos_row,
                                      const int32_t* K, int64_t sk_z, int64_t sk_s, const int32_t* V, int64_t sv_z,
@@ -2380,13 +2585,13 @@ extern "C" int bx_exact_attn_prefill(const int32_t* qg, int64_t sq_z, int64_t sq
         p, pl, pl + (int64_t)Z * 3 * Sp * HD, tab, Z, Sp, HD);
     if (int rc = check_launch("pre_split_kernel")) return rc;
     if (HD == 64) {
-      allow_lds_attn((const void*)attn_pre2_kernel<64>, Pre2<64>::LDS);
-      attn_pre2_kernel<64><<<Z * ((gT + Pre2<64>::QR - 1) / Pre2<64>::QR), 64 * Pre2<64>::NW, Pre2<64>::LDS, st>>>(
-          p, pl, Z, Sp, tab);
+      allow_lds_attn((const void*)attn_pre2_kernel<64, false>, Pre2<64>::LDS);
+      attn_pre2_kernel<64, false><<<Z * ((gT + Pre2<64>::QR - 1) / Pre2<64>::QR), 64 * Pre2<64>::NW, Pre2<64>::LDS, st>>>(
+          p, pl, Z, Sp, tab, RowMap{});
     } else {
-      allow_lds_attn((const void*)attn_pre2_kernel<128>, Pre2<128>::LDS);
-      attn_pre2_kernel<128><<<Z * ((gT + Pre2<128>::QR - 1) / Pre2<128>::QR), 64 * Pre2<128>::NW, Pre2<128>::LDS, st>>>(
-          p, pl, Z, Sp, tab);
+      allow_lds_attn((const void*)attn_pre2_kernel<128, false>, Pre2<128>::LDS);
+      attn_pre2_kernel<128, false><<<Z * ((gT + Pre2<128>::QR - 1) / Pre2<128>::QR), 64 * Pre2<128>::NW, Pre2<128>::LDS, st>>>(
+          p, pl, Z, Sp, tab, RowMap{});
     }
     return check_launch("attn_pre2_kernel");
   }

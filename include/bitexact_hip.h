@@ -136,6 +136,19 @@ int bx_exact_attn_paged(const int32_t* q, const int64_t* sh, const int64_t* qpos
                         int32_t R, int32_t HKV, int32_t M, int32_t HD, int32_t nsplit, void* ws, int64_t ws_bytes,
                         bx_stream_t stream);
 
+/* The same attention for steps of many tokens per sequence (prefill chunks; the same reference call): the token rows
+ * are grouped by block-table row on the device, each sequence's cached K / V limbs are laid out once per call as
+ * planes in tmp, and a block runs many tokens of one sequence against each key tile (bx_exact_attn_prefill's main
+ * kernel). bt has nrow rows; every rmap value lies in [0, nrow) (the output rows of others are not written). q
+ * 16-byte aligned. tmp: 16-byte aligned, bx_attn_paged_rows_scratch bytes, no contents kept; the query returns 0 where
+ * that form is not available (planes of all nrow sequences above 1 GiB, or sizes bx_exact_attn_paged rejects). */
+int64_t bx_attn_paged_rows_scratch(int32_t R, int32_t nrow, int32_t HKV, int32_t M, int32_t HD, int32_t keys);
+int bx_exact_attn_paged_rows(const int32_t* q, const int64_t* sh, const int64_t* qpos, int64_t sqpos_r,
+                             const int8_t* cache, int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs, const int32_t* bt,
+                             int64_t sbt, int32_t nrow, int32_t nblk, const int64_t* rmap, const int64_t* lut, int64_t l2e,
+                             int64_t* num, int64_t* den, int32_t R, int32_t HKV, int32_t M, int32_t HD, void* tmp,
+                             int64_t tmp_bytes, bx_stream_t stream);
+
 /* Replaces the decode step's exact_fuse.qkv + tri_exact_attn.attend pair (src/bitexact/vllm_plugin/exact_fuse.py:
  * 372-386, tri_exact_attn.py:138-165) when every token of the step belongs to its own sequence (decode): one launch
  * does the rope kernel's work (bx_rope_qgroup_store: RoPE of the q and k heads of y int64 [R, >= (H + 2 HKV) HD]

@@ -195,6 +195,38 @@ def test_prefill_attention_full_size(dev, HD, T, Z):
                                                                                      ref_den[0])
 
 
+@pytest.mark.parametrize("HD,M,bs", [(64, 4, 16), (64, 3, 16), (64, 1, 32), (128, 4, 16), (128, 2, 16)])
+@pytest.mark.parametrize("order", ["runs", "mixed"])
+def test_paged_rows_equal_decode_form(dev, HD, M, bs, order):
+    """attend's grouped form (prefill steps) against the per-token form, bit for bit: sequences whose token counts are
+    at a tile's edges (0, 1, one short of a tile, a tile, one over, several), chunks that start past other keys,
+    padding tokens (position -1), the tokens of a sequence in a row or all mixed, strided cache heads."""
+    from bitexact.vllm_plugin import tri_exact_attn, tri_paged
+    g = torch.Generator().manual_seed(HD + M)
+    HKV, TT = 2, (128 if HD == 64 else 64) // M
+    counts, start = [0, 1, TT - 1, TT, TT + 1, 1200, 70], [0, 300, 5, 64, 63, 0, 129]
+    nrow, nblk = len(counts), -(-(max(s + n for s, n in zip(start, counts))) // bs)
+    c = torch.randint(-R.LIM3, R.LIM3 + 1, (nrow * nblk, HKV, bs, 2 * HD), generator=g).to(torch.int32)
+    cl = tri_paged.to_limbs(c.to(dev))
+    bt = torch.randperm(nrow * nblk, generator=g).to(torch.int32).view(nrow, nblk).to(dev)
+    rmap = torch.cat([torch.full((n,), i) for i, n in enumerate(counts)])
+    pos = torch.cat([torch.arange(n) + s for s, n in zip(start, counts)])
+    if order == "mixed":
+        p = torch.randperm(len(pos), generator=g)
+        rmap, pos = rmap[p], pos[p]
+    pos[::17] = -1
+    Rr = len(pos)
+    qpos = pos[:, None].expand(Rr, M).contiguous()
+    q = torch.randint(-(1 << 22), (1 << 22) + 1, (Rr, HKV, M, HD), generator=g).to(torch.int32)
+    sh = torch.randint(-46, -36, (Rr, HKV, M), generator=g)
+    args = (q.to(dev), sh.to(dev), qpos.to(dev), cl, bt, rmap.to(dev), _lut(dev), R.L2E28_HD[HD])
+    assert tri_exact_attn.rows_scratch(Rr, HKV, M, HD, nrow, nblk * bs) > 0
+    n1, d1 = tri_exact_attn.attend(*args, nsplit=1)
+    for _ in range(2):
+        n2, d2 = tri_exact_attn.attend(*args)
+        assert torch.equal(n1, n2) and torch.equal(d1, d2)
+
+
 @pytest.mark.parametrize("HD", [64, 128])
 @pytest.mark.parametrize("table", ["exp2", "noisy", "steps"])
 def test_prefill_weight_positions(dev, HD, table):
