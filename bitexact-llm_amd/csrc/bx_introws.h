@@ -115,6 +115,51 @@ __device__ __forceinline__ int64_t silu_elem(int64_t g, int64_t u, int64_t la, i
   return mul_wrap(sv, u);
 }
 
+// silu_index and silu_elem at FR = 24 in a short form: table position idx, the remainder rr and ph (n = ph >> 22) from
+// one 32 x 32-bit product (t = prod >> 28 as silu_index's t; n = t >> 26, f = t mod 2^26 its entry and remainder).
+struct SiluAt {
+  uint32_t ph, rr;
+  int idx;
+};
+__device__ __forceinline__ SiluAt silu_at24(int64_t g) {
+  const uint64_t ga = g < 0 ? 0 - (uint64_t)g : (uint64_t)g;
+  const uint32_t gm = ga < (1ULL << 30) ? (uint32_t)ga : 1u << 30;
+  const uint64_t prod = (uint64_t)gm * (uint32_t)kL2E30 + (1u << 27);
+  SiluAt a;
+  a.ph = (uint32_t)(prod >> 32);
+  a.rr = (uint32_t)(prod >> 28) & 4095u;
+  a.idx = (int)((a.ph >> 8) & 16383u);
+  return a;
+}
+
+// silu(g) u of one element; false where the short form does not hold (P is then undefined and the caller takes
+// silu_elem): |g|, |u| < 2^30 and a table value v in [0, 2^60]. sig = floor(N / den + 1/2) comes from a float64
+// quotient: 1 / den after two Newton steps is within a few 2^-52, N / den <= 2^30, so the floor stands unless the
+// quotient plus 1/2 lies within 2^-16 of an integer. In this range silu_mul's bounds hold (ok).
+__device__ __forceinline__ bool silu_short24(int64_t g, int64_t u, const SiluAt& a, int64_t la, int64_t lb, int64_t& P) {
+  const int64_t v = la + (int64_t)(((lb - la) * (int64_t)a.rr + 2048) >> 12);
+  const uint32_t n = a.ph >> 22;
+  // rshc(v, min(30 + n, 62)) for 0 <= v <= 2^60, as a nested floor
+  const uint32_t E = ((uint32_t)(v >> (n < 32u ? 29 + n : 61u)) + 1u) >> 1;
+  const double den = (double)((1u << 30) + E), N = g >= 0 ? 0x1p60 : (double)E * 0x1p30;
+  double x = __builtin_amdgcn_rcp(den);
+  x = __builtin_fma(x, __builtin_fma(-den, x, 1.0), x);
+  x = __builtin_fma(x, __builtin_fma(-den, x, 1.0), x);
+  const double t = __builtin_fma(N, x, 0.5), fr = t - __builtin_floor(t);
+  const int32_t sig = (int32_t)(uint32_t)t;
+  const int32_t sv = (int32_t)(((int64_t)(int32_t)g * sig + (1 << 29)) >> 30);
+  P = (int64_t)sv * (int32_t)u;
+  const uint64_t rg = (uint64_t)(g + (1 << 30)) | (uint64_t)(u + (1 << 30));
+  return (rg >> 31) == 0 && (uint64_t)v <= (1ULL << 60) && fr > 0x1p-16 && fr < 1.0 - 0x1p-16;
+}
+
+// silu_elem by the short form where it holds
+__device__ __forceinline__ int64_t silu_any(int64_t g, int64_t u, int64_t la, int64_t lb, int FR, int& bad) {
+  int64_t P;
+  if (FR == 24 && silu_short24(g, u, silu_at24(g), la, lb, P)) return P;
+  return silu_elem(g, u, la, lb, FR, bad);
+}
+
 // ops.softmax_w's weight of one visible key (src/bitexact/exact/ops.py:133-143 over exp2neg_lut, 108-116): z =
 // max - raw >= 0, zshift = kbits + 3 - sh - FZ, weight at fp bits.
 __device__ __forceinline__ int64_t weight64(int64_t z, int64_t zshift, const int64_t* lut, int64_t l2e, int fp) {

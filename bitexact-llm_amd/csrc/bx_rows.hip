@@ -185,7 +185,7 @@ __global__ __launch_bounds__(kRowThreads) void silu_quant_kernel(const int64_t* 
   for (int k = 0; k < kSiluU; ++k) {
     const int i = i0 + k * kRowThreads;
     if (i >= ff) continue;
-    const int64_t P = silu_elem(gv[k], uv[k], la[k], lb[k], FR, bad);
+    const int64_t P = silu_any(gv[k], uv[k], la[k], lb[k], FR, bad);
     Ps[i] = P;
     if (P != 0) emax = imax(emax, bitlen(P < 0 ? (int64_t)(0 - (uint64_t)P) : P) + eps);
   }
@@ -195,6 +195,100 @@ __global__ __launch_bounds__(kRowThreads) void silu_quant_kernel(const int64_t* 
   const int64_t shr = imax(emax - kQB, kNegBig);
   for (int i = threadIdx.x; i < ff; i += kRowThreads) q[(int64_t)blockIdx.x * ldq + i] = (int32_t)rshc(Ps[i], shr - eps);
   if (threadIdx.x == 0) sh[blockIdx.x] = shr;
+}
+
+// ---- the same stage for many rows (FR = 24): one 1024-thread block per CU walks rows with the 2^-f table in LDS ----
+// A row-per-block launch gathered two 8-byte table entries an element through L1 (the 128 KiB table misses its 32
+// KiB) and divided twice per element, once for each sign of g: 4096 rows of 2 x 8192 took 337 us against 134 us
+// for their bytes at 5 TB/s. Here the gathers are LDS reads, the quotient is one float64 estimate, a thread keeps its
+// products in registers (8 columns a chunk of 8192) and the next chunk's 16-byte loads are in flight while this one
+// is worked: 121 us (5.5 TB/s of the bytes it must move), bound by HBM.
+constexpr int kSiluTab = 16385;
+typedef int64_t v2l __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint64_t wave_or64(uint64_t v) {
+  v |= (uint64_t)dpp64<0x121>((int64_t)v);
+  v |= (uint64_t)dpp64<0x122>((int64_t)v);
+  v |= (uint64_t)dpp64<0x124>((int64_t)v);
+  v |= (uint64_t)dpp64<0x128>((int64_t)v);
+  return (uint64_t)(readlane64((int64_t)v, 0) | readlane64((int64_t)v, 16) | readlane64((int64_t)v, 32) |
+                    readlane64((int64_t)v, 48));
+}
+template <int NCH>
+__global__ __launch_bounds__(1024) void silu_rows_kernel(const int64_t* gu, int64_t ldgu, int ff, const int64_t* lut,
+                                                         int32_t* q, int64_t ldq, int64_t* sh, int M, int32_t* err) {
+  extern __shared__ __align__(16) int64_t T[];       // the table
+  __shared__ uint64_t sor[2][16];
+  constexpr int FR = 24, eps = -2 * FR;
+  const int tid = threadIdx.x;
+  v2l G[4], V[4];
+  auto load = [&](int r, int ch) {                   // columns past the row: its last pair (their products are not used)
+    const int64_t* row = gu + (int64_t)r * ldgu;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int c = min(ch * 8192 + (k * 1024 + tid) * 2, ff - 2);
+      G[k] = __builtin_nontemporal_load((const v2l*)(row + c));
+      V[k] = __builtin_nontemporal_load((const v2l*)(row + ff + c));
+    }
+  };
+  load(blockIdx.x, 0);
+  for (int i = tid; i < kSiluTab; i += 1024) T[i] = lut[i];
+  __syncthreads();
+  int par = 0;
+  for (int r = blockIdx.x; r < M; r += gridDim.x, par ^= 1) {
+    int64_t P[NCH * 8];
+    uint64_t any = 0;                                // the products' magnitudes ored: the row's bit length
+    int bad = 0;
+    bool least = false;                              // a product of -2^63, whose magnitude wraps (bitlen 0)
+#pragma unroll
+    for (int ch = 0; ch < NCH; ++ch) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        SiluAt a[2];
+        int64_t la[2], lb[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          a[e] = silu_at24(G[k][e]);
+          la[e] = T[a[e].idx];
+          lb[e] = T[a[e].idx + 1];
+        }
+        const bool in = ch * 8192 + (k * 1024 + tid) * 2 < ff;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          int64_t v;
+          const bool ok = silu_short24(G[k][e], V[k][e], a[e], la[e], lb[e], v);
+          if (!ok) {
+            int b = 0;
+            v = silu_elem(G[k][e], V[k][e], la[e], lb[e], FR, b);
+            if (in) bad |= b;
+            if (in && v == INT64_MIN) least = true;
+          }
+          P[ch * 8 + k * 2 + e] = v;
+          const uint64_t m = v < 0 ? 0 - (uint64_t)v : (uint64_t)v;
+          if (in) any |= m & (uint64_t)INT64_MAX;
+        }
+      }
+      if (ch + 1 < NCH) load(r, ch + 1);
+      else if (r + (int)gridDim.x < M) load(r + gridDim.x, 0);
+    }
+    if (bad) err[0] = 1;
+    any = wave_or64(any) | (wave_or(least ? 1 : 0) ? 1ULL << 63 : 0);
+    if ((tid & 63) == 0) sor[par][tid >> 6] = any;
+    lds_sync();                                      // the other buffer serves the next row, so one barrier a row
+    any = wave_or64(sor[par][tid & 15]);
+    const int64_t len = 64 - __clzll((long long)(any & (uint64_t)INT64_MAX));
+    const int64_t emax = (any & (uint64_t)INT64_MAX) != 0 ? len + eps : any != 0 ? eps : kNegBig;
+    const int64_t shr = imax(emax - kQB, kNegBig);
+    const int64_t s = imin(imax(shr - eps, -62), 62);
+    int32_t* qr = q + (int64_t)r * ldq;
+#pragma unroll
+    for (int ch = 0; ch < NCH; ++ch)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int c = ch * 8192 + (k * 1024 + tid) * 2;
+        if (c < ff) *(int2*)(qr + c) = int2{(int)rshc(P[ch * 8 + k * 2], s), (int)rshc(P[ch * 8 + k * 2 + 1], s)};
+      }
+    if (tid == 0) sh[r] = shr;
+  }
 }
 
 // ---- intops.first_argmax (src/bitexact/intops.py:55-59): index of the first maximum of each int64 row. A lane
@@ -329,7 +423,7 @@ __global__ __launch_bounds__(kSiluPartThreads) void silu_fused_kernel(const int6
     for (int k = 0; k < U; ++k) {
       const int i = i0 + k * kSiluPartThreads;
       if (i >= i_hi) continue;
-      const int64_t v = silu_elem(gv[k], uv[k], la[k], lb[k], FR, bad);
+      const int64_t v = silu_any(gv[k], uv[k], la[k], lb[k], FR, bad);
       Ps[i - i_lo] = v;
       if (v != 0) emax = imax(emax, bitlen(v < 0 ? (int64_t)(0 - (uint64_t)v) : v) + eps);
     }
@@ -542,6 +636,22 @@ extern "C" int bx_silu_quant(const int64_t* gu, int64_t ldgu, int32_t ff, const 
   BX_REQUIRE(FR >= 0 && FR <= 24, "FR outside [0, 24]");
   BX_REQUIRE(gu && lut && q && sh && err, "null pointer");
   if (M == 0) return BX_OK;
+  // many rows, whole pairs of columns, 16-byte rows: the table-in-LDS kernel (one block per CU; below 2 rows a block the
+  // table's 128 KiB copy costs what it saves)
+  const int cus = device_cus();
+  if (FR == 24 && M >= 2 * cus && ff >= 2048 && ff % 2 == 0 && ldgu % 2 == 0 && ldq % 2 == 0 &&
+      ((uintptr_t)gu & 15) == 0 && ((uintptr_t)q & 7) == 0) {
+    constexpr size_t tl = kSiluTab * 8 + 8;
+    const dim3 grid(std::min(M, cus));
+    if (ff <= 8192) {
+      allow_lds_rows((const void*)silu_rows_kernel<1>, tl);
+      silu_rows_kernel<1><<<grid, 1024, tl, (hipStream_t)stream>>>(gu, ldgu, ff, lut, q, ldq, sh, M, err);
+    } else {
+      allow_lds_rows((const void*)silu_rows_kernel<2>, tl);
+      silu_rows_kernel<2><<<grid, 1024, tl, (hipStream_t)stream>>>(gu, ldgu, ff, lut, q, ldq, sh, M, err);
+    }
+    return check_launch("silu_rows_kernel");
+  }
   const size_t lds = (size_t)ff * 8;
   allow_lds_rows((const void*)silu_quant_kernel, lds);
   silu_quant_kernel<<<M, kRowThreads, lds, (hipStream_t)stream>>>(gu, ldgu, ff, lut, FR, q, ldq, sh, err);

@@ -142,6 +142,42 @@ def test_gu_silu_split(dev, M, ff):
     assert bool(ops.gu_silu_y(bad.to(dev), L, split=True)[2]) and R.gu_silu_y(bad.numpy(), lut)[2]
 
 
+@pytest.mark.parametrize("ff", [2048, 2050, 8192, 8194, 14336])
+def test_gu_silu_many_rows(dev, ff):
+    """The many-row SiLU kernel (table in LDS, one block per CU walking rows) at its chunk edges, against the oracle on
+    a row sample and against the row-per-block kernel (taken for rows of odd stride) on every row: N(0, 1) rows, rows
+    around the short form's bounds (|g|, |u| near 2^30 and 2^32), zero rows, a product of -2^63, both flags."""
+    from bitexact.exact import ops
+    M = 2 * torch.cuda.get_device_properties(dev).multi_processor_count + 3
+    g = torch.Generator().manual_seed(ff)
+    gu = (torch.randn(M, 2 * ff, generator=g) * 2.0 ** 24).long()
+    edge = torch.tensor([0, 1, -1, (1 << 30) - 1, 1 << 30, -(1 << 30), -(1 << 30) - 1, (1 << 31), -(1 << 31), 1 << 28, -(1 << 28)])
+    gu[1] = edge[torch.randint(0, len(edge), (2 * ff,), generator=g)]
+    gu[2], gu[3, :ff], gu[M - 1, ff:] = 0, 0, 0
+    gu[4] = torch.randint(-(1 << 31), 1 << 31, (2 * ff,), generator=g)
+    gu[5] >>= 14
+    lut = R.exp2_table()
+    L = torch.from_numpy(lut).to(dev)
+
+    def both(x):
+        a = ops.gu_silu_y(x.to(dev), L, split=False)
+        odd = torch.zeros(M, 2 * ff + 1, dtype=torch.long, device=dev)
+        odd[:, :2 * ff] = x.to(dev)
+        b = ops.gu_silu_y(odd[:, :2 * ff], L, split=False)
+        assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1]) and bool(a[2]) == bool(b[2])
+        return a
+    q, sh, err = both(gu)
+    rows = [0, 1, 2, 3, 4, 5, M // 2, M - 1]
+    rq, rsh, rf = R.gu_silu_y(gu[rows].numpy(), lut)
+    assert np.array_equal(q[rows].cpu().numpy(), rq) and np.array_equal(sh[rows].cpu().numpy(), rsh) and bool(err) == rf
+    gu[M - 2, 0], gu[M - 2, ff] = 1 << 32, -(1 << 62)              # overflows; silu(2^8) = 2^32: a product of 2^94 wraps
+    gu[7], gu[7, 0], gu[7, ff] = 0, 1 << 30, -(1 << 33)             # the row's one product is -2^63
+    q, sh, err = both(gu)
+    rq, rsh, rf = R.gu_silu_y(gu[[7, M - 2]].numpy(), lut)
+    assert rf and bool(err)
+    assert np.array_equal(q[[7, M - 2]].cpu().numpy(), rq) and np.array_equal(sh[[7, M - 2]].cpu().numpy(), rsh)
+
+
 @pytest.mark.parametrize("ticks", ["0", "1"])
 def test_gu_silu_split_exchange_fallback(dev, monkeypatch, ticks):
     """The column chunks of a row exchange their maxima with a bounded wait; with the wait cut to 0 / 1 tick
