@@ -84,6 +84,18 @@ __device__ __forceinline__ int64_t div_round64(int64_t a, int64_t p, int64_t r, 
   return p >= 0 ? up : down;
 }
 
+// div_round64 in float64 for p >= 0: round-half-up(A / r) for an integer A = a 2^p held exactly (|a| < 2^53), 0 < r <
+// 2^34 and a quotient below 2^50 (the caller checks): the estimate A / r + 1/2 (two roundings of 2^-53) is then
+// within 1/2, its floor within 1 of the result, the remainder A - q r an integer below 2^36 in magnitude that one
+// fused multiply-add gives exactly, and one step either way finishes.
+__device__ __forceinline__ double div_round_f64(double A, double r, double rinv) {
+  const double q = __builtin_floor(__builtin_fma(A, rinv, 0.5));
+  const double rem2 = 2.0 * __builtin_fma(-q, r, A);
+  return q + (rem2 >= r ? 1.0 : 0.0) - (rem2 < -r ? 1.0 : 0.0);
+}
+// floor(log2) + 1 of a positive integer held in a float64: its bit length
+__device__ __forceinline__ int64_t bitlen_f64(double v) { return (__builtin_bit_cast(int64_t, v) >> 52) - 1022; }
+
 constexpr int64_t kL2E30 = 1549082005LL;   // round(log2(e) 2^30) (ops.L2E30)
 
 // ops.exp2neg_lut(t, lut, 30) given the two table entries a = lut[idx], b = lut[idx + 1] at idx = (t mod 2^26) >> 12

@@ -1,6 +1,6 @@
-// Row-wise integer stages around the GEMMs and the attention, one block per row (1024 threads, 512 for the norm:
-// a decode step has few rows, so each row spreads over a whole CU; softmax rows use 256; the SiLU stage of few rows
-// goes over column chunks) with DPP wavefront int64 reductions: RMSNorm + per-row quantization (segs.norm_quant,
+// Row-wise integer stages around the GEMMs and the attention, one block per row (1024 threads for few rows, as in a
+// decode step, so each row spreads over a whole CU; smaller blocks for many; softmax rows use 256; the SiLU stage of
+// few rows goes over column chunks, that of many walks rows with its table in LDS) with DPP wavefront int64 reductions: RMSNorm + per-row quantization (segs.norm_quant,
 // optionally after the residual add or the
 // embedding gather), SiLU gating + quantization (segs.silu_y + quant_silu), the masked softmax weights
 // (segs.softmax), and the attention output rule (segs.attn_out = div_round + regroup + quant).
@@ -15,7 +15,6 @@ BX_PHASE_TABLE
 
 
 constexpr int kRowThreads = 1024;
-constexpr int kRowU = 4;   // elements per thread whose loads are issued together
 
 // ---- segs.norm_quant (src/bitexact/exact/segs.py:59-63) over ops.rms (src/bitexact/exact/ops.py:92-105) and
 // ops.quant (src/bitexact/exact/ops.py:82-89), on the residual row the block first forms:
@@ -42,108 +41,215 @@ struct NormArgs {
   int32_t* err;
   int8_t* planes;   // optional: q's signed int8 limb planes [3][M][D] (limb i of q[m][k] at i M D + m D + k)
   int64_t plane;    // M D
+  bool vec;         // pairs of columns by 16-byte accesses (set by launch_norm)
 };
 
-// One block of kNormThreads per row (a decode row of 2048 is 2 elements a thread, all loads in flight at once):
-// the block reductions stay cheap (wave reductions in DPP, one LDS-only barrier each), and the gamma loads go out
-// with the row's loads rather than after the reductions. 1024 threads measured +0.4 % on the engine step over 512
-// (256: 17.2 vs 12.5 us per launch in an earlier form).
-constexpr int kNormThreads = 1024, kNormU = 2;
-template <int SRC>
-__global__ __launch_bounds__(kNormThreads) void norm_quant_kernel(NormArgs p) {
-  BX_PHASE(0, 0);
-  constexpr int NT = kNormThreads, U = kNormU, NW = NT / 64;
-  extern __shared__ __align__(16) char smem[];
-  int64_t* Xs = (int64_t*)smem;
-  int64_t* Ps = Xs + p.D;
-  __shared__ int64_t sbuf[3][NW];
-  const int D = p.D;
-  int64_t* xr = p.x + (int64_t)blockIdx.x * p.ldx;
-  const int32_t* er_row = nullptr;
-  if (SRC == SRC_EMB) er_row = p.emb + p.ids[blockIdx.x] * (int64_t)D;
-  const int64_t* yr = SRC == SRC_ADD ? p.y + (int64_t)blockIdx.x * p.ldy : nullptr;
-  int64_t amax = 0;
-  int64_t gmv0[U], gev0[U];   // the first group's gamma pairs, requested with the row
-  // U elements per thread at a time, every load issued before the first store (the write-back to x could
-  // alias later loads, which would otherwise wait for it one element at a time)
-  for (int i0 = threadIdx.x; i0 < D; i0 += U * NT) {
-    int64_t v[U];
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const int i = min(i0 + k * NT, D - 1);
-      if (SRC == SRC_EMB) v[k] = er_row[i];
-      else if (SRC == SRC_ADD) v[k] = add_wrap(xr[i], yr[i]);
-      else v[k] = xr[i];
-    }
-    if (i0 == (int)threadIdx.x && p.gm != nullptr) {
-#pragma unroll
-      for (int k = 0; k < U; ++k) {
-        const int i = min(i0 + k * NT, D - 1);
-        gmv0[k] = p.gm[i];
-        gev0[k] = p.ge[i];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const int i = i0 + k * NT;
-      if (i < D) {
-        if (SRC != SRC_X) xr[i] = v[k];
-        Xs[i] = v[k];
-        amax = imax(amax, v[k] < 0 ? -v[k] : v[k]);
-      }
-    }
+// Pairs of columns i, i + 1: 16-byte loads where `vec` (host: aligned bases, even strides), else one by one; columns
+// past D read as 0.
+typedef int64_t v2l __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ v2l ld_pair(const int64_t* a, int i, int D, bool vec) {
+  if (vec) return i < D ? *(const v2l*)(a + i) : v2l{0, 0};
+  return v2l{i < D ? a[i] : 0, i + 1 < D ? a[i + 1] : 0};
+}
+__device__ __forceinline__ void st_q_pair(int32_t* q, int i, int D, bool vec, int32_t a, int32_t b) {
+  if (vec) {
+    if (i < D) *(int2*)(q + i) = int2{a, b};
+  } else {
+    if (i < D) q[i] = a;
+    if (i + 1 < D) q[i + 1] = b;
   }
-  BX_PHASE(0, 1);
-  amax = block_reduce64_dpp<true, NW>(amax, sbuf[0], 0);
+}
+__device__ __forceinline__ void st_limbs(int8_t* dst, int64_t plane, int32_t r) {   // split_q_kernel's limbs
+#pragma unroll
+  for (int l = 0; l < 3; ++l) {
+    const int32_t lo = limb_lo(r);
+    dst[l * plane] = (int8_t)lo;
+    r = (r - lo) >> 8;
+  }
+}
+// max over the block of non-negative float64 values (their bit patterns order as integers)
+template <int NW>
+__device__ __forceinline__ double block_fmax(double v, int64_t* slot) {
+  return __builtin_bit_cast(double, block_reduce64_dpp<true, NW>(__builtin_bit_cast(int64_t, v), slot, 0));
+}
+
+// The row's rule in int64 as the reference states it, on x as it stands in memory: taken by rows the float64 form
+// cannot hold (a value of 2^52 or more, a quotient of 2^50 or more). The quotients are formed twice.
+template <int NT>
+__device__ void norm_row_general(const NormArgs& p, const int64_t* xr) {
+  constexpr int NW = NT / 64;
+  __shared__ int64_t gbuf[3][NW];
+  const int D = p.D;
+  int64_t amax = 0;
+  for (int i = threadIdx.x; i < D; i += NT) amax = imax(amax, xr[i] < 0 ? -xr[i] : xr[i]);
+  amax = block_reduce64_dpp<true, NW>(amax, gbuf[0], 0);
   if (threadIdx.x == 0 && amax >= (1LL << 40)) p.err[0] = 1;
   if (p.gm == nullptr) return;
   const int64_t shx = imax(bitlen(imax(amax, 1)) - 25, -6);
   int64_t S = 0;
   for (int i = threadIdx.x; i < D; i += NT) {
-    const int64_t xs = rshc(Xs[i], shx);
+    const int64_t xs = rshc(xr[i], shx);
     S = add_wrap(S, mul_wrap(xs, xs));
   }
-  S = block_reduce64_dpp<false, NW>(S, sbuf[1], 0);
+  S = block_reduce64_dpp<false, NW>(S, gbuf[1], 0);
   const int64_t T = add_wrap(S, rshc(kEps60 * (int64_t)D, 60 - 2 * (p.FR - shx)));
   const int64_t m = fdiv(62 + p.lg - bitlen(T), 2);
   const int64_t s = 2 * m - p.lg;
   const int64_t V = s >= 0 ? shl(T, s) : sar(T, -s);
   const int64_t r = isqrt64(V), er = shx - p.FR - m;
   const double rinv = 1.0 / (double)r;
-  BX_PHASE(0, 2);
   int64_t emax = kNegBig;
-  for (int i0 = threadIdx.x; i0 < D; i0 += U * NT) {
-    int64_t gmv[U], gev[U];
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const int i = min(i0 + k * NT, D - 1);
-      gmv[k] = i0 == (int)threadIdx.x ? gmv0[k] : p.gm[i];
-      gev[k] = i0 == (int)threadIdx.x ? gev0[k] : p.ge[i];
-    }
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const int i = i0 + k * NT;
-      if (i < D) {
-        const int64_t P = div_round64(mul_wrap(Xs[i], gmv[k]), gev[k] - p.FR - er + p.FN, r, rinv);
-        Ps[i] = P;
-        if (P != 0) emax = imax(emax, bitlen(P < 0 ? -P : P) - p.FN);
-      }
-    }
+  for (int i = threadIdx.x; i < D; i += NT) {
+    const int64_t P = div_round64(mul_wrap(xr[i], p.gm[i]), p.ge[i] - p.FR - er + p.FN, r, rinv);
+    if (P != 0) emax = imax(emax, bitlen(P < 0 ? -P : P) - p.FN);
   }
-  BX_PHASE(0, 3);
-  emax = block_reduce64_dpp<true, NW>(emax, sbuf[2], kNegBig);
+  emax = block_reduce64_dpp<true, NW>(emax, gbuf[2], kNegBig);
   const int64_t shr = imax(emax - kQB, kNegBig);
   for (int i = threadIdx.x; i < D; i += NT) {
-    const int32_t qv = (int32_t)rshc(Ps[i], shr + p.FN);
+    const int64_t P = div_round64(mul_wrap(xr[i], p.gm[i]), p.ge[i] - p.FR - er + p.FN, r, rinv);
+    const int32_t qv = (int32_t)rshc(P, shr + p.FN);
     p.q[(int64_t)blockIdx.x * p.ldq + i] = qv;
-    if (p.planes != nullptr) {   // the limb split of the exact GEMM's activation planes (split_q_kernel's)
-      int8_t* dst = p.planes + (int64_t)blockIdx.x * D + i;
-      int32_t r = qv;
+    if (p.planes != nullptr) st_limbs(p.planes + (int64_t)blockIdx.x * D + i, p.plane, qv);
+  }
+  if (threadIdx.x == 0) p.sh[blockIdx.x] = shr;
+}
+
+// One block of NT threads per row, EPT elements of it in a thread's registers. The arithmetic runs in float64, which
+// holds every integer of the rule exactly in the rows' ordinary range (|x| < 2^52, quotients below 2^50; other rows
+// take norm_row_general): the division by the rms is one estimate, a fused remainder and a correction, the
+// quantization a scale, half and floor. NT = 1024 (2 elements a thread) for few rows, where one row's latency
+// counts; NT = 256 (8 a thread, 8 blocks a CU) from two rows per CU: 4096 rows of 2048 measured 74 us with one
+// 1024-thread block of integer arithmetic a row, 57 us (add, 235 MB) and 40 us (embedding, 134 MB) so, near HBM's
+// rate for reads and writes mixed; a decode step's 32 launches together 39 us less.
+template <int SRC, int NT, int EPT>
+__global__ __launch_bounds__(NT) void norm_quant_kernel(NormArgs p) {
+  BX_PHASE(0, 0);
+  constexpr int NW = NT / 64, H = EPT / 2;
+  __shared__ int64_t sbuf[3][NW];
+  const int D = p.D;
+  const bool vec = p.vec;
+  int64_t* xr = p.x + (int64_t)blockIdx.x * p.ldx;
+  const int32_t* er_row = nullptr;
+  if (SRC == SRC_EMB) er_row = p.emb + p.ids[blockIdx.x] * (int64_t)D;
+  const int64_t* yr = SRC == SRC_ADD ? p.y + (int64_t)blockIdx.x * p.ldy : nullptr;
+  double X[EPT];
+  v2l gm2[H], ge2[H];
+  {
+    v2l v[H], y[H];
 #pragma unroll
-      for (int l = 0; l < 3; ++l) {
-        const int32_t lo = limb_lo(r);
-        dst[l * p.plane] = (int8_t)lo;
-        r = (r - lo) >> 8;
+    for (int h = 0; h < H; ++h) {
+      const int i = 2 * (h * NT + threadIdx.x);
+      if (SRC == SRC_EMB) {
+        if (vec) {
+          const int2 e = i < D ? *(const int2*)(er_row + i) : int2{0, 0};
+          v[h] = v2l{e.x, e.y};
+        } else {
+          v[h] = v2l{i < D ? er_row[i] : 0, i + 1 < D ? er_row[i + 1] : 0};
+        }
+      } else {
+        v[h] = ld_pair(xr, i, D, vec);
+        if (SRC == SRC_ADD) y[h] = ld_pair(yr, i, D, vec);
+      }
+    }
+    if (EPT <= 4 && p.gm != nullptr) {   // the gamma pairs, requested with the row (wide rows: after its sum)
+#pragma unroll
+      for (int h = 0; h < H; ++h) {
+        const int i = 2 * (h * NT + threadIdx.x);
+        gm2[h] = ld_pair(p.gm, i, D, vec);
+        ge2[h] = ld_pair(p.ge, i, D, vec);
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int i = 2 * (h * NT + threadIdx.x);
+      if (SRC == SRC_ADD) v[h] = v2l{add_wrap(v[h][0], y[h][0]), add_wrap(v[h][1], y[h][1])};
+      if (SRC != SRC_X) {
+        if (vec) {
+          if (i < D) *(v2l*)(xr + i) = v[h];
+        } else {
+          if (i < D) xr[i] = v[h][0];
+          if (i + 1 < D) xr[i + 1] = v[h][1];
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) X[2 * h + e] = (double)v[h][e];
+    }
+  }
+  double am = 0;
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) am = __builtin_fmax(am, __builtin_fabs(X[k]));
+  BX_PHASE(0, 1);
+  am = block_fmax<NW>(am, sbuf[0]);
+  if (am >= 0x1p52) {                                // block-uniform: the int64 rule (the row is written: see it whole)
+    __syncthreads();
+    norm_row_general<NT>(p, xr);
+    return;
+  }
+  if (threadIdx.x == 0 && am >= 0x1p40) p.err[0] = 1;
+  if (p.gm == nullptr) return;
+  const int shx = am > 0 ? (int)imax(bitlen_f64(am) - 25, -6) : -6;
+  const double xsc = ldexp(1.0, -shx);
+  int64_t S = 0;
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) {                    // rshc(x, shx): |.| <= 2^25, exact in float64
+    const int32_t xs = (int32_t)__builtin_floor(__builtin_fma(X[k], xsc, 0.5));
+    S += (int64_t)xs * xs;
+  }
+  S = block_reduce64_dpp<false, NW>(S, sbuf[1], 0);
+  if (EPT > 4) {
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int i = 2 * (h * NT + threadIdx.x);
+      gm2[h] = ld_pair(p.gm, i, D, vec);
+      ge2[h] = ld_pair(p.ge, i, D, vec);
+    }
+  }
+  const int64_t T = add_wrap(S, rshc(kEps60 * (int64_t)D, 60 - 2 * (p.FR - shx)));
+  const int64_t m = (62 + p.lg - bitlen(T)) >> 1;
+  const int64_t s = 2 * m - p.lg;
+  const int64_t V = s >= 0 ? shl(T, s) : sar(T, -s);
+  const int64_t r = isqrt64(V), er = shx - p.FR - m;
+  const double rf = (double)r, rinv = 1.0 / rf;
+  BX_PHASE(0, 2);
+  double pm = 0;
+#pragma unroll
+  for (int k = 0; k < EPT; ++k) {
+    const int64_t gm = gm2[k >> 1][k & 1], pe = ge2[k >> 1][k & 1] - p.FR - er + p.FN;
+    const double A0 = X[k] * (double)gm;
+    const bool ok = (__builtin_fabs(A0) < 0x1p52 && pe >= 0 && pe <= 62) || 2 * ((k >> 1) * NT + (int)threadIdx.x) + (k & 1) >= D;
+    X[k] = div_round_f64(ldexp(A0, (int)pe), rf, rinv);   // (a column past D: 0)
+    const double mag = __builtin_fabs(X[k]);
+    pm = __builtin_fmax(pm, ok && mag < 0x1p50 ? mag : __builtin_inf());
+  }
+  BX_PHASE(0, 3);
+  if (r <= 0 || r >= (1LL << 34)) pm = __builtin_inf();
+  pm = block_fmax<NW>(pm, sbuf[2]);
+  if (pm == __builtin_inf()) {
+    __syncthreads();
+    norm_row_general<NT>(p, xr);
+    return;
+  }
+  const int64_t shr = pm > 0 ? imax(bitlen_f64(pm) - p.FN - kQB, kNegBig) : kNegBig;
+  const double qsc = ldexp(1.0, (int)-imin(imax(shr + p.FN, -62), 62));
+  int32_t* qr = p.q + (int64_t)blockIdx.x * p.ldq;
+#pragma unroll
+  for (int h = 0; h < H; ++h) {                      // rshc(P, shr + FN)
+    const int i = 2 * (h * NT + threadIdx.x);
+    int32_t qv[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) qv[e] = (int32_t)__builtin_floor(__builtin_fma(X[2 * h + e], qsc, 0.5));
+    st_q_pair(qr, i, D, vec, qv[0], qv[1]);
+    if (p.planes != nullptr && i < D) {              // (planes: D % 16 == 0)
+      int8_t* dst = p.planes + (int64_t)blockIdx.x * D + i;
+      if (vec) {
+        // byte i of q + 0x808080 is limb i + 128 (the adds' carries are the digits' borrows)
+        const uint32_t y0 = ((uint32_t)qv[0] + 0x808080u) ^ 0x808080u, y1 = ((uint32_t)qv[1] + 0x808080u) ^ 0x808080u;
+#pragma unroll
+        for (int l = 0; l < 3; ++l)
+          *(uint16_t*)(dst + l * p.plane) = (uint16_t)(((y0 >> (8 * l)) & 255u) | (((y1 >> (8 * l)) & 255u) << 8));
+      } else {
+        st_limbs(dst, p.plane, qv[0]);
+        st_limbs(dst + 1, p.plane, qv[1]);
       }
     }
   }
@@ -204,7 +310,6 @@ __global__ __launch_bounds__(kRowThreads) void silu_quant_kernel(const int64_t* 
 // products in registers (8 columns a chunk of 8192) and the next chunk's 16-byte loads are in flight while this one
 // is worked: 121 us (5.5 TB/s of the bytes it must move), bound by HBM.
 constexpr int kSiluTab = 16385;
-typedef int64_t v2l __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint64_t wave_or64(uint64_t v) {
   v |= (uint64_t)dpp64<0x121>((int64_t)v);
   v |= (uint64_t)dpp64<0x122>((int64_t)v);
@@ -378,6 +483,83 @@ __global__ __launch_bounds__(kRowThreads) void attn_out_kernel(const int64_t* nu
   emax = block_max64(emax, sbuf);
   const int64_t shr = imax(emax - kQB, kNegBig);
   for (int c = threadIdx.x; c < W; c += kRowThreads) q[(int64_t)o * ldq + c] = (int32_t)rshc(Os[c], shr + FR);
+  if (threadIdx.x == 0) sh[o] = shr;
+}
+
+// The same stage with the row in registers (EPT elements a thread, pairs of columns of one head) and the quotients in
+// float64 (div_round_f64): rows of at most NT EPT columns, even head_dim, 16-byte aligned. A row that float64 does
+// not hold (|num| 2^(FR - FV) of 2^52 or more, den of 2^34 or more, a quotient of 2^50 or more) forms its quotients
+// in int64, twice. NT = 256 from two rows per CU on: 4096 rows of 2048 took 59 us with one 1024-thread block a row
+// (a float64 division and an int64 one per element), 27 us so (101 MB of HBM traffic).
+template <int NT, int EPT>
+__global__ __launch_bounds__(NT) void attn_out_regs_kernel(const int64_t* num, int64_t sn_group, int64_t sn_query,
+                                                           const int64_t* den, int64_t sd_group, int T, int HKV, int g,
+                                                           int HD, int FR, int FV, int32_t* q, int64_t ldq, int64_t* sh) {
+  constexpr int NW = NT / 64, H = EPT / 2;
+  __shared__ int64_t sbuf[2][NW];
+  const int o = blockIdx.x, b = o / T, t = o - b * T;
+  const int W = HKV * g * HD;
+  auto where = [&](int c, int64_t& nm, int64_t& dn) {   // element offsets of column c's num and its head's den
+    const int hh = c / HD, d = c - hh * HD, kv = hh / g;
+    const int64_t group = (int64_t)b * HKV + kv, query = (int64_t)(hh - kv * g) * T + t;
+    nm = group * sn_group + query * sn_query + d;
+    dn = group * sd_group + query;
+  };
+  v2l n2[H];
+  int64_t d1[H];
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    int64_t nm, dn;
+    where(min(2 * (h * NT + (int)threadIdx.x), W - 2), nm, dn);
+    n2[h] = *(const v2l*)(num + nm);
+    d1[h] = den[dn];
+  }
+  const double up = ldexp(1.0, FR - FV);
+  double P[EPT], pm = 0;
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const bool in = 2 * (h * NT + (int)threadIdx.x) < W;
+    const double r = (double)d1[h];
+    double x = __builtin_amdgcn_rcp(r);               // 1 / r: two Newton steps
+    x = __builtin_fma(x, __builtin_fma(-r, x, 1.0), x);
+    x = __builtin_fma(x, __builtin_fma(-r, x, 1.0), x);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const double A = (double)n2[h][e];
+      const double v = d1[h] > 0 ? div_round_f64(A * up, r, x) : 0.0;   // den = 0: no visible key
+      const double mag = __builtin_fabs(v);
+      P[2 * h + e] = v;
+      if (in) pm = __builtin_fmax(pm, __builtin_fabs(A) < 0x1p52 && d1[h] < (1LL << 34) && mag < 0x1p48 ? mag : __builtin_inf());
+    }
+  }
+  pm = block_fmax<NW>(pm, sbuf[0]);
+  int32_t* qr = q + (int64_t)o * ldq;
+  if (pm == __builtin_inf()) {                       // block-uniform
+    auto quot = [&](int c) {
+      int64_t nm, dn;
+      where(c, nm, dn);
+      return den[dn] > 0 ? div_round64(num[nm], FR - FV, den[dn], 1.0 / (double)den[dn]) : 0;
+    };
+    int64_t emax = kNegBig;
+    for (int c = threadIdx.x; c < W; c += NT) {
+      const int64_t v = quot(c);
+      if (v != 0) emax = imax(emax, bitlen(v < 0 ? -v : v) - FR);
+    }
+    emax = block_reduce64_dpp<true, NW>(emax, sbuf[1], kNegBig);
+    const int64_t shr = imax(emax - kQB, kNegBig);
+    for (int c = threadIdx.x; c < W; c += NT) qr[c] = (int32_t)rshc(quot(c), shr + FR);
+    if (threadIdx.x == 0) sh[o] = shr;
+    return;
+  }
+  const int64_t shr = pm > 0 ? imax(bitlen_f64(pm) - FR - kQB, kNegBig) : kNegBig;
+  const double qsc = ldexp(1.0, (int)-imin(imax(shr + FR, -62), 62));
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const int c = 2 * (h * NT + (int)threadIdx.x);
+    if (c < W)
+      *(int2*)(qr + c) = int2{(int)__builtin_floor(__builtin_fma(P[2 * h], qsc, 0.5)),
+                              (int)__builtin_floor(__builtin_fma(P[2 * h + 1], qsc, 0.5))};
+  }
   if (threadIdx.x == 0) sh[o] = shr;
 }
 
@@ -573,14 +755,23 @@ static int launch_norm(NormArgs& p, int src, int32_t M, bx_stream_t stream) {
   BX_REQUIRE(!p.gm || (p.ge && p.q && p.sh && p.ldq >= p.D), "gamma given without the quantized outputs");
   if (M == 0) return BX_OK;
   p.lg = lg;
-  const size_t lds = (size_t)p.D * 16;
-  const void* k = src == SRC_ADD ? (const void*)norm_quant_kernel<SRC_ADD>
-                  : src == SRC_EMB ? (const void*)norm_quant_kernel<SRC_EMB> : (const void*)norm_quant_kernel<SRC_X>;
-  allow_lds_rows(k, lds);
   hipStream_t st = (hipStream_t)stream;
-  if (src == SRC_ADD) norm_quant_kernel<SRC_ADD><<<M, kNormThreads, lds, st>>>(p);
-  else if (src == SRC_EMB) norm_quant_kernel<SRC_EMB><<<M, kNormThreads, lds, st>>>(p);
-  else norm_quant_kernel<SRC_X><<<M, kNormThreads, lds, st>>>(p);
+  auto al = [](const void* a, unsigned m) { return ((uintptr_t)a & m) == 0; };
+  p.vec = p.D >= 2 && al(p.x, 15) && p.ldx % 2 == 0 && al(p.y, 15) && p.ldy % 2 == 0 && al(p.emb, 7) && al(p.gm, 15) &&
+          al(p.ge, 15) && al(p.q, 7) && p.ldq % 2 == 0 && al(p.planes, 1);
+  const bool many = M >= 2 * device_cus();
+#define BX_NORM(SRCV)                                                                        \
+  do {                                                                                       \
+    if (!many && p.D <= 2048) norm_quant_kernel<SRCV, 1024, 2><<<M, 1024, 0, st>>>(p);       \
+    else if (!many) norm_quant_kernel<SRCV, 1024, 4><<<M, 1024, 0, st>>>(p);                 \
+    else if (p.D <= 1024) norm_quant_kernel<SRCV, 256, 4><<<M, 256, 0, st>>>(p);             \
+    else if (p.D <= 2048) norm_quant_kernel<SRCV, 256, 8><<<M, 256, 0, st>>>(p);             \
+    else norm_quant_kernel<SRCV, 512, 8><<<M, 512, 0, st>>>(p);                              \
+  } while (0)
+  if (src == SRC_ADD) BX_NORM(SRC_ADD);
+  else if (src == SRC_EMB) BX_NORM(SRC_EMB);
+  else BX_NORM(SRC_X);
+#undef BX_NORM
   return check_launch("norm_quant_kernel");
 }
 
@@ -588,7 +779,7 @@ extern "C" int bx_rmsnorm_quant(const int64_t* x, int64_t ldx, const int64_t* gm
                                 int64_t ldq, int64_t* sh, int32_t M, int32_t D, int32_t FR, int32_t FN, int32_t* err,
                                 bx_stream_t stream) {
   BX_REQUIRE(gm && ge && q && sh, "null pointer");
-  NormArgs p = {const_cast<int64_t*>(x), ldx, nullptr, 0, nullptr, nullptr, gm, ge, q, ldq, sh, D, 0, FR, FN, err, nullptr, 0};
+  NormArgs p = {const_cast<int64_t*>(x), ldx, nullptr, 0, nullptr, nullptr, gm, ge, q, ldq, sh, D, 0, FR, FN, err, nullptr, 0, false};
   return launch_norm(p, SRC_X, M, stream);
 }
 
@@ -596,7 +787,7 @@ extern "C" int bx_add_rmsnorm_quant(int64_t* x, int64_t ldx, const int64_t* y, i
                                     const int64_t* ge, int32_t* q, int64_t ldq, int64_t* sh, int32_t M, int32_t D,
                                     int32_t FR, int32_t FN, int32_t* err, bx_stream_t stream) {
   BX_REQUIRE(y && ldy >= D, "y: null or ldy too small");
-  NormArgs p = {x, ldx, y, ldy, nullptr, nullptr, gm, ge, q, ldq, sh, D, 0, FR, FN, err, nullptr, 0};
+  NormArgs p = {x, ldx, y, ldy, nullptr, nullptr, gm, ge, q, ldq, sh, D, 0, FR, FN, err, nullptr, 0, false};
   return launch_norm(p, SRC_ADD, M, stream);
 }
 
@@ -607,7 +798,7 @@ extern "C" int bx_add_rmsnorm_quant_planes(int64_t* x, int64_t ldx, const int64_
   BX_REQUIRE(!y || ldy >= D, "ldy too small");
   BX_REQUIRE(gm && ge && q && sh && planes, "null pointer");
   BX_REQUIRE(D % 16 == 0, "D %% 16 != 0 (the limb planes are the exact GEMM's K-major operand)");
-  NormArgs p = {x, ldx, y, ldy, nullptr, nullptr, gm, ge, q, ldq, sh, D, 0, FR, FN, err, planes, (int64_t)M * D};
+  NormArgs p = {x, ldx, y, ldy, nullptr, nullptr, gm, ge, q, ldq, sh, D, 0, FR, FN, err, planes, (int64_t)M * D, false};
   return launch_norm(p, y ? SRC_ADD : SRC_X, M, stream);   // y null: the norm of x as it is (x not written)
 }
 
@@ -615,7 +806,7 @@ extern "C" int bx_embed_rmsnorm_quant(const int32_t* emb, const int64_t* ids, in
                                       const int64_t* gm, const int64_t* ge, int32_t* q, int64_t ldq, int64_t* sh,
                                       int32_t M, int32_t D, int32_t FR, int32_t FN, int32_t* err, bx_stream_t stream) {
   BX_REQUIRE(emb && ids, "null pointer");
-  NormArgs p = {x, ldx, nullptr, 0, emb, ids, gm, ge, q, ldq, sh, D, 0, FR, FN, err, nullptr, 0};
+  NormArgs p = {x, ldx, nullptr, 0, emb, ids, gm, ge, q, ldq, sh, D, 0, FR, FN, err, nullptr, 0, false};
   return launch_norm(p, SRC_EMB, M, stream);
 }
 
@@ -625,7 +816,7 @@ extern "C" int bx_embed_rmsnorm_quant_planes(const int32_t* emb, const int64_t* 
                                              int32_t FN, int32_t* err, bx_stream_t stream) {
   BX_REQUIRE(emb && ids && gm && ge && q && sh && planes, "null pointer");
   BX_REQUIRE(D % 16 == 0, "D %% 16 != 0 (the limb planes are the exact GEMM's K-major operand)");
-  NormArgs p = {x, ldx, nullptr, 0, emb, ids, gm, ge, q, ldq, sh, D, 0, FR, FN, err, planes, (int64_t)M * D};
+  NormArgs p = {x, ldx, nullptr, 0, emb, ids, gm, ge, q, ldq, sh, D, 0, FR, FN, err, planes, (int64_t)M * D, false};
   return launch_norm(p, SRC_EMB, M, stream);
 }
 
@@ -736,7 +927,21 @@ extern "C" int bx_attn_out(const int64_t* num, int64_t sn_group, int64_t sn_quer
   BX_REQUIRE(ldq >= (int64_t)HKV * g * HD, "ldq too small");
   BX_REQUIRE(num && den && q && sh, "null pointer");
   if (rows == 0) return BX_OK;
-  const size_t lds = (size_t)HKV * g * HD * 8;
+  const int64_t W = (int64_t)HKV * g * HD;
+  if (W <= 4096 && HD % 2 == 0 && FR >= FV && FR - FV <= 62 && ((uintptr_t)num & 15) == 0 && sn_group % 2 == 0 &&
+      sn_query % 2 == 0 && ((uintptr_t)q & 7) == 0 && ldq % 2 == 0) {
+    hipStream_t st = (hipStream_t)stream;
+    const bool many = rows >= 2 * device_cus();
+#define BX_AOUT(NT, EPT) \
+  attn_out_regs_kernel<NT, EPT><<<rows, NT, 0, st>>>(num, sn_group, sn_query, den, sd_group, T, HKV, g, HD, FR, FV, q, ldq, sh)
+    if (!many && W <= 2048) BX_AOUT(1024, 2);
+    else if (!many) BX_AOUT(1024, 4);
+    else if (W <= 2048) BX_AOUT(256, 8);
+    else BX_AOUT(512, 8);
+#undef BX_AOUT
+    return check_launch("attn_out_regs_kernel");
+  }
+  const size_t lds = (size_t)W * 8;
   allow_lds_rows((const void*)attn_out_kernel, lds);
   attn_out_kernel<<<rows, kRowThreads, lds, (hipStream_t)stream>>>(num, sn_group, sn_query, den, sd_group, T, HKV, g, HD, FR,
                                                           FV, q, ldq, sh);
