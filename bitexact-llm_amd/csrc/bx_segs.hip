@@ -25,31 +25,83 @@ __device__ __forceinline__ int64_t seg_block_max(int64_t v, int64_t* sbuf) {
   return r;
 }
 
-// Grid (token, head-row group of 4): wave w of block (token, j) takes head row 4 j + w (one row per wave, so the
-// rows' loads are in flight together instead of one row after another); lane l holds dims l + 64 e.
-template <int HD>
+// Grid (token, group of head rows): HD / 2 lanes take a head row, lane l its dims l and l + HD / 2 (a RoPE pair), so a
+// wave works 64 / (HD / 2) rows at a time with one cos / sin pair per lane and token, and RU of them with all their
+// loads in flight. Before, one lane per dim read every pair twice and every row its own cos / sin: 4096 tokens of 32
+// + 8 + 8 heads of 64 took 104 us, so 44 us (168 MB). Products are 32 x 32 bits: rows with a value of 2^31 or more
+// (flagged) or tables past 32 bits take the wrapping 64-bit products.
+template <int HD, int RU>
 __global__ __launch_bounds__(256) void rope_qgroup_kernel(RopeArgs p) {
-  constexpr int E = HD / 64;
+  constexpr int HALF = HD / 2, RW = 64 / HALF;
   const int token = blockIdx.x, b = token / p.T, t = token - b * p.T;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, d = lane % HALF, sub = lane / HALF;
   const int64_t pos_raw = p.pos[(int64_t)b * p.spb + (int64_t)t * p.spt];
   bool bad = pos_raw < 0 || pos_raw >= p.npos;          // the reference's table index would fail: flagged
   const int64_t pos = imin(imax(pos_raw, 0), p.npos - 1);
+  const int64_t c = p.cos[pos * HALF + d], sn = p.sin[pos * HALF + d];
+  const bool fit = c == (int32_t)c && sn == (int32_t)sn && (int32_t)sn != INT32_MIN;
   const int g = p.H / p.HKV, rows = p.H + 2 * p.HKV;
   const int64_t eps = -(int64_t)(p.FR + p.FT);
-  for (int hr = blockIdx.y * 4 + wave; hr < rows && hr < (int)blockIdx.y * 4 + 4; hr += 4) {
-    int64_t out[E];
-    rope_row<HD>(p, token, hr, pos, lane, out, bad);
+  const int64_t* y = p.y + (int64_t)token * p.ldy;
+  const int r0 = (blockIdx.y * RU * 4 + wave) * RW + sub;
+  int64_t x1[RU], x2[RU];
+#pragma unroll
+  for (int u = 0; u < RU; ++u) {
+    const int64_t* x = y + (int64_t)min(r0 + u * 4 * RW, rows - 1) * HD;
+    x1[u] = x[d];
+    x2[u] = x[d + HALF];
+  }
+#pragma unroll
+  for (int u = 0; u < RU; ++u) {
+    const int hr = r0 + u * 4 * RW;
+    const bool live = hr < rows;
+    const bool in = x1[u] < (1LL << 31) && x1[u] > -(1LL << 31) && x2[u] < (1LL << 31) && x2[u] > -(1LL << 31);
+    bad |= live && !in;
+    int64_t o1 = x1[u], o2 = x2[u];
+    if (hr < p.H + p.HKV) {
+      // _rope_full (src/bitexact/exact/segs.py:66-69): (x1 c - x2 s, x2 c + x1 s)
+      if (in && fit) {
+        const int32_t a = (int32_t)x1[u], e = (int32_t)x2[u], ci = (int32_t)c, si = (int32_t)sn;
+        o1 = (int64_t)a * ci + (int64_t)e * -si;
+        o2 = (int64_t)e * ci + (int64_t)a * si;
+      } else {
+        o1 = add_wrap(mul_wrap(x1[u], c), -mul_wrap(x2[u], sn));
+        o2 = add_wrap(mul_wrap(x2[u], c), mul_wrap(x1[u], sn));
+      }
+    }
+    // the magnitudes ored over the row's lanes: the row's bit length (-2^63 sets bit 63 alone: a bit length of 0)
+    uint64_t any = (o1 < 0 ? 0 - (uint64_t)o1 : (uint64_t)o1) | (o2 < 0 ? 0 - (uint64_t)o2 : (uint64_t)o2);
+    any |= (uint64_t)dpp64<0x121>((int64_t)any);
+    any |= (uint64_t)dpp64<0x122>((int64_t)any);
+    any |= (uint64_t)dpp64<0x124>((int64_t)any);
+    any |= (uint64_t)dpp64<0x128>((int64_t)any);
+    any |= (uint64_t)__shfl_xor((long long)any, 16, 64);
+    if (HD == 128) any |= (uint64_t)__shfl_xor((long long)any, 32, 64);
+    if (!live) continue;
     if (hr < p.H) {
-      // q head: quantized, stored at its grouped row
-      const int64_t shq = rope_q_shift<HD>(p, out, bad);
+      // q head: ops.quant(Pq, -(FR + FT)) over its HD values, stored at its grouped row
+      const uint64_t low = any & (uint64_t)INT64_MAX;
+      const int64_t emax = low != 0 ? bitlen((int64_t)low) + eps : any != 0 ? eps : kSegNegBig;
+      const int64_t shq = imax(emax - kSegQB, kSegNegBig);
+      bad |= shq > p.FK + 3 - p.FZ;
       const int kvh = hr / g, gi = hr - kvh * g;
       const int64_t row = ((int64_t)b * p.HKV + kvh) * ((int64_t)g * p.T) + (int64_t)gi * p.T + t;
-#pragma unroll
-      for (int e = 0; e < E; ++e) p.qg[row * HD + lane + 64 * e] = (int32_t)rshc(out[e], shq - eps);
-      if (lane == 0) p.shg[row] = shq;
+      p.qg[row * HD + d] = (int32_t)rshc(o1, shq - eps);
+      p.qg[row * HD + d + HALF] = (int32_t)rshc(o2, shq - eps);
+      if (d == 0) p.shg[row] = shq;
     } else {
-      rope_kv_store<HD>(p, token, hr, lane, out, bad);
+      const bool isk = hr < p.H + p.HKV;
+      const int h = isk ? hr - p.H : hr - p.H - p.HKV, down = isk ? p.FR + p.FT - p.FK : p.FR - p.FV;
+      const int64_t v1 = rshc(o1, down), v2 = rshc(o2, down);
+      bad |= v1 > kLim3 || v1 < -kLim3 || v2 > kLim3 || v2 < -kLim3;
+      int64_t* dst = isk ? p.k : p.v;
+      if (dst) {
+        dst += ((int64_t)token * p.HKV + h) * HD;
+        dst[d] = v1;
+        dst[d + HALF] = v2;
+      }
+      store_limbs(p, token, h, isk ? 0 : 3, d, v1);
+      store_limbs(p, token, h, isk ? 0 : 3, d + HALF, v2);
     }
   }
   if (wave_or(bad ? 1 : 0) && lane == 0) p.err[0] = 1;
@@ -188,11 +240,18 @@ static int rope_common(const int64_t* y, int64_t ldy, const int64_t* pos, int64_
   BX_REQUIRE(y && pos && cos && sin && qg && shg && err, "null pointer");
   RopeArgs p = {y, ldy, pos, spb, spt, cos, sin, npos, B, T, H, HKV, HD, FR, FT, FK, FV, FZ, qg, shg, k, v, err,
                 cache, sc_nb, sc_h, sc_bs, slot, bs};
-  const dim3 blocks(B * T, (H + 2 * HKV + 3) / 4);
-  if (HD == 64)
-    rope_qgroup_kernel<64><<<blocks, 256, 0, (hipStream_t)stream>>>(p);
-  else
-    rope_qgroup_kernel<128><<<blocks, 256, 0, (hipStream_t)stream>>>(p);
+  // many tokens: a block takes a whole token's rows, 3 a wave in flight; few: a block per 4 waves' rows
+  const int rows = H + 2 * HKV, per = 4 * (128 / HD);
+  hipStream_t st = (hipStream_t)stream;
+  if ((int64_t)B * T >= 2 * device_cus()) {
+    const dim3 blocks(B * T, (rows + 3 * per - 1) / (3 * per));
+    if (HD == 64) rope_qgroup_kernel<64, 3><<<blocks, 256, 0, st>>>(p);
+    else rope_qgroup_kernel<128, 3><<<blocks, 256, 0, st>>>(p);
+  } else {
+    const dim3 blocks(B * T, (rows + per - 1) / per);
+    if (HD == 64) rope_qgroup_kernel<64, 1><<<blocks, 256, 0, st>>>(p);
+    else rope_qgroup_kernel<128, 1><<<blocks, 256, 0, st>>>(p);
+  }
   return check_launch("rope_qgroup_kernel");
 }
 

@@ -34,6 +34,42 @@ def test_rope_qgroup(dev, HD, H, HKV, B, T):
     assert bool(out[4]) == err
 
 
+@pytest.mark.parametrize("HD,H,HKV", [(64, 6, 2), (64, 32, 8), (128, 4, 1), (128, 32, 8)])
+@pytest.mark.parametrize("wide", [False, True])
+def test_rope_qgroup_many_tokens(dev, HD, H, HKV, wide):
+    """The many-token launch (a block takes several rows a wave, rows past the heads masked) against the oracle, with the
+    store into the cache; `wide`: values past 2^31 (flagged) and a table value past 32 bits, whose products wrap."""
+    from bitexact.exact import ops
+    B, T = 1, 2 * torch.cuda.get_device_properties(dev).multi_processor_count + 5
+    g = torch.Generator().manual_seed(HD + H)
+    cos, sin = _tables(300, HD)
+    W = (H + 2 * HKV) * HD
+    y = (torch.randn(T, W, generator=g) * 2.0 ** 24).long()
+    y[3, :HD] = 0
+    if wide:
+        y[5, 1], y[6, W - HD - 1], y[7, 2] = 1 << 31, -(1 << 45), -(1 << 62)
+        cos = cos.copy()
+        cos[299, 0] = 1 << 40
+    pos = torch.randint(0, 300, (B, T), generator=g)
+    pos[0, 9] = 299
+    Pq, k, v = R.rope_y(y.numpy(), pos.numpy(), cos, sin, B, T, (H, HKV, HD))
+    qg, shg, err = R.q_group(Pq, k, v, y.numpy())
+    args = (y.to(dev), pos.to(dev), torch.from_numpy(cos).to(dev), torch.from_numpy(sin).to(dev), B, T, (H, HKV, HD))
+    out = ops.qkv_y(*args)
+    assert np.array_equal(out[0].cpu().numpy(), qg) and np.array_equal(out[1].cpu().numpy(), shg)
+    assert np.array_equal(out[2].cpu().numpy(), k) and np.array_equal(out[3].cpu().numpy(), v)
+    assert bool(out[4]) == err
+    if not wide:
+        from bitexact.vllm_plugin import tri_paged
+        cache = [torch.zeros(T // 16 + 2, HKV, 16, 8 * HD, dtype=torch.int8, device=dev) for _ in range(2)]
+        slot = torch.randperm(16 * (T // 16 + 2), generator=g)[:T]
+        slot[::11] = -1
+        qs, shs, _, _, _ = ops.qkv_y(*args, store=(cache[0], slot.to(dev)))
+        assert torch.equal(qs, out[0]) and torch.equal(shs, out[1])
+        tri_paged.store(cache[1], slot.to(dev), out[2][0], out[3][0])
+        assert torch.equal(cache[0], cache[1])
+
+
 def test_rope_qgroup_flags(dev):
     from bitexact.exact import ops
     HD, H, HKV, B, T = 64, 4, 2, 1, 3
