@@ -45,6 +45,11 @@ SIGNATURES = {
     "bx_int8_gemm_workspace": (I64, [I32, I32, I32, I32]),
     "bx_exact_attn_paged": (ctypes.c_int, [P, P, P, I64, P, I64, I64, I64, I32, P, I64, I32, P, P, I64, P, P, I32, I32,
                                            I32, I32, I32, P, I64, P]),
+    "bx_attn_paged_scores_scratch": (I64, [I32, I32, I32, I32]),
+    "bx_exact_attn_paged_scores": (ctypes.c_int, [P, P, P, I64, P, I64, I64, I64, I32, P, I64, I32, P, P, I64, P, P, I32,
+                                                  I32, I32, I32, I32, P, I64, P, I64, P]),
+    "bx_int8_attn_paged_scores": (ctypes.c_int, [P, P, I64, P, I64, I64, I64, I32, P, I64, I32, P, I32, P, P, I32, I32,
+                                                 I32, I32, I32, P, I64, P, I64, P]),
     "bx_attn_paged_rows_scratch": (I64, [I32, I32, I32, I32, I32, I32]),
     "bx_exact_attn_paged_rows": (ctypes.c_int, [P, P, P, I64, P, I64, I64, I64, I32, P, I64, I32, I32, P, P, I64, P, P,
                                                 I32, I32, I32, I32, P, I64, P]),

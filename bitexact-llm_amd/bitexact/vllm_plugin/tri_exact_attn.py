@@ -6,6 +6,8 @@ with the reference's argument meaning; bn / warps are accepted for signature par
 integers).
 """
 
+import functools
+
 import torch
 
 from bitexact import _hip
@@ -18,8 +20,11 @@ BLOCK_TARGET = 256          # blocks (of 8 waves) to aim for: 1 per MI355X compu
 def default_nsplit(R, HKV, nblk, bs):
     """Key splits: none once the (row, KV head) tiles alone cover half the device (one launch, K read once);
     otherwise enough blocks to fill it, at least 128 keys per split."""
-    tiles = max(1, R * HKV)
-    keys = max(1, nblk * bs)
+    return tile_nsplit(R * HKV, nblk * bs)
+
+
+def tile_nsplit(tiles, keys):
+    tiles, keys = max(1, tiles), max(1, keys)
     if tiles >= 128:
         return 1
     return max(1, min(64, BLOCK_TARGET // tiles, keys // 128))
@@ -28,6 +33,26 @@ def default_nsplit(R, HKV, nblk, bs):
 def _attend_fake(q, sh, qpos, cache, bt, rmap, lut, l2e, nsplit):
     R, HKV, M, HD = q.shape
     return empty((R, HKV, M, HD), torch.long, q), empty((R, HKV, M, 1), torch.long, q)
+
+
+SCORES_MAX = 1 << 28        # bytes of kept scores at most
+
+
+@functools.lru_cache(4096)
+def auto_nsplit(T, keys, HD):
+    """(nsplit, kept-scores scratch bytes or 0) of T query tiles over `keys` keys. The exchange and one-block forms
+    read K once while a split has at most 512 keys or a tile at most 2048; past that they would read it twice, and two
+    launches that keep the scores in between (two blocks per CU) are faster: 16 x 8 tiles of 4096 keys 74 against 134
+    us (heads of 128: 113 / 203), 8 x 8 of 4096 45 / 52 (67 / 73). Of the one-block range only half a chip of tiles
+    over wide rows gains (16 x 8 tiles, 2048 keys, heads of 128: 66 / 75; of 64: 45 / 47)."""
+    ns = tile_nsplit(T, keys)
+    twice = -(-(-(-keys // ns)) // 64) * 64 > 512 if ns > 1 else keys > 2048
+    if (twice and T >= 64) or (128 <= T < 192 and 2048 * 128 <= keys * HD and keys <= 2048):
+        need = _hip.lib().bx_attn_paged_scores_scratch(T, 1, 4, keys)
+        split = min(max(2, 512 // T), max(1, min(64, 4096 // T)))
+        if need <= SCORES_MAX and split > 1:
+            return split, need
+    return ns, 0
 
 
 # The grouped form for at least ROWS_MIN (token, KV head, dim)s and ROWS_PER_SEQ tokens per block-table row. Measured (8
@@ -46,10 +71,16 @@ def rows_scratch(R, HKV, M, HD, nrow, keys):
     return _hip.lib().bx_attn_paged_rows_scratch(R, nrow, HKV, M, HD, keys)
 
 
+@functools.lru_cache(4096)
+def _plan(R, HKV, M, HD, nrow, keys):
+    """attend's form for a step of these sizes: (grouped form's scratch or 0, nsplit, kept scores or 0)."""
+    return rows_scratch(R, HKV, M, HD, nrow, keys), *auto_nsplit(R * HKV, keys, HD)
+
+
 @op("attend_exact(Tensor q, Tensor sh, Tensor qpos, Tensor cache, Tensor bt, Tensor rmap, Tensor lut, int l2e, "
     "int nsplit) -> (Tensor, Tensor)", _attend_fake)
 def _attend(q, sh, qpos, cache, bt, rmap, lut, l2e, nsplit):
-    """nsplit 0: chosen here (the grouped form for prefills, else default_nsplit)."""
+    """nsplit 0: chosen here (the grouped form for prefills, else auto_nsplit)."""
     _hip.require_cuda(q, sh, qpos, cache, bt, rmap, lut)
     R, HKV, M, HD = q.shape
     assert M <= BQ and cache.shape[1] == HKV and cache.shape[3] >= 6 * HD and cache.stride(3) == 1
@@ -59,17 +90,24 @@ def _attend(q, sh, qpos, cache, bt, rmap, lut, l2e, nsplit):
     rmap, lut = rmap.contiguous().long(), lut.contiguous().long()
     num = torch.empty(R, HKV, M, HD, dtype=torch.long, device=q.device)
     den = torch.empty(R, HKV, M, 1, dtype=torch.long, device=q.device)
-    need = rows_scratch(R, HKV, M, HD, bt.shape[0], bt.shape[1] * cache.shape[2]) if nsplit == 0 else 0
-    if need > 0 and q.data_ptr() % 16 == 0:
-        tmp, tmpb = _hip.scratch(q.device, need)
-        _hip.call("bx_exact_attn_paged_rows", _hip.ptr(q), _hip.ptr(sh), _hip.ptr(qpos), qpos.stride(0), _hip.ptr(cache),
-                  cache.stride(0), cache.stride(1), cache.stride(2), cache.shape[2], _hip.ptr(bt), bt.stride(0),
-                  bt.shape[0], bt.shape[1], _hip.ptr(rmap), _hip.ptr(lut), int(l2e), _hip.ptr(num), _hip.ptr(den), R,
-                  HKV, M, HD, _hip.ptr(tmp), tmpb, _hip.stream_of(q))
-        return num, den
+    keep = 0
     if nsplit == 0:
-        nsplit = default_nsplit(R, HKV, bt.shape[1], cache.shape[2])
+        need, nsplit, keep = _plan(R, HKV, M, HD, bt.shape[0], bt.shape[1] * cache.shape[2])
+        if need > 0 and q.data_ptr() % 16 == 0:
+            tmp, tmpb = _hip.scratch(q.device, need)
+            _hip.call("bx_exact_attn_paged_rows", _hip.ptr(q), _hip.ptr(sh), _hip.ptr(qpos), qpos.stride(0),
+                      _hip.ptr(cache), cache.stride(0), cache.stride(1), cache.stride(2), cache.shape[2], _hip.ptr(bt),
+                      bt.stride(0), bt.shape[0], bt.shape[1], _hip.ptr(rmap), _hip.ptr(lut), int(l2e), _hip.ptr(num),
+                      _hip.ptr(den), R, HKV, M, HD, _hip.ptr(tmp), tmpb, _hip.stream_of(q))
+            return num, den
     ws, wsb = _hip.workspace(q.device, _hip.lib().bx_attn_paged_workspace(R, HKV, M, HD) if nsplit > 1 else 0)
+    if keep:
+        tmp, tmpb = _hip.scratch(q.device, keep)
+        _hip.call("bx_exact_attn_paged_scores", _hip.ptr(q), _hip.ptr(sh), _hip.ptr(qpos), qpos.stride(0), _hip.ptr(cache),
+                  cache.stride(0), cache.stride(1), cache.stride(2), cache.shape[2], _hip.ptr(bt), bt.stride(0),
+                  bt.shape[1], _hip.ptr(rmap), _hip.ptr(lut), int(l2e), _hip.ptr(num), _hip.ptr(den), R, HKV, M, HD,
+                  int(nsplit), _hip.ptr(ws), wsb, _hip.ptr(tmp), tmpb, _hip.stream_of(q))
+        return num, den
     _hip.call("bx_exact_attn_paged", _hip.ptr(q), _hip.ptr(sh), _hip.ptr(qpos), qpos.stride(0), _hip.ptr(cache),
               cache.stride(0), cache.stride(1), cache.stride(2), cache.shape[2], _hip.ptr(bt), bt.stride(0),
               bt.shape[1], _hip.ptr(rmap), _hip.ptr(lut), int(l2e), _hip.ptr(num), _hip.ptr(den), R, HKV, M, HD,

@@ -10,6 +10,7 @@ import torch
 
 from bitexact import _hip
 from bitexact._ops import empty, op
+from bitexact.vllm_plugin.tri_exact_attn import auto_nsplit
 
 
 @op("kv_store(Tensor(a!) c, Tensor slot, Tensor k, Tensor v) -> ()", lambda c, slot, k, v: None)
@@ -40,7 +41,6 @@ def to_limbs(c):
 
 
 FE, FP = 30, 20                 # exp table values, int8 attention weights (src/bitexact/int8/segs.py:22)
-SM_TARGET = 256                 # blocks (of 8 waves) to aim for: 1 per MI355X compute unit
 
 
 def weight_table(lut):
@@ -53,12 +53,8 @@ def attend(q, qpos, cache, bt, ptab, nsplit=None, bm=None, bn=None, warps=4):
     """int8-mode paged attention (src/bitexact/vllm_plugin/tri_paged.py:363-401): q int64 [R, HKV, M, HD], qpos int64
     [R, M], cache int8 [nb, HKV, bs, 8 HD], bt int32 [R, *], ptab = weight_table(exp table) -> (num int64
     [R, HKV, M, HD], den int64 [R, HKV, M, 1]). bm / bn / warps are accepted for signature parity."""
-    if nsplit is None:
-        R, HKV, M, _ = q.shape
-        tiles = max(1, R * HKV * ((M + 3) // 4))
-        keys = max(1, bt.shape[1] * cache.shape[2])
-        nsplit = 1 if tiles >= 128 else max(1, min(64, SM_TARGET // tiles, keys // 128))
-    return _attend_int8(q, qpos, cache, bt, ptab, int(nsplit))
+    assert nsplit is None or nsplit >= 1, "nsplit in [1, 64]"
+    return _attend_int8(q, qpos, cache, bt, ptab, 0 if nsplit is None else int(nsplit))
 
 
 def _attend_int8_fake(q, qpos, cache, bt, ptab, nsplit):
@@ -69,6 +65,7 @@ def _attend_int8_fake(q, qpos, cache, bt, ptab, nsplit):
 @op("attend_int8(Tensor q, Tensor qpos, Tensor cache, Tensor bt, Tensor ptab, int nsplit) -> (Tensor, Tensor)",
     _attend_int8_fake)
 def _attend_int8(q, qpos, cache, bt, ptab, nsplit):
+    """nsplit 0: chosen here, as the exact attention's (tri_exact_attn.auto_nsplit)."""
     _hip.require_cuda(q, qpos, cache, bt, ptab)
     R, HKV, M, HD = q.shape
     assert cache.shape[1] == HKV and cache.shape[3] >= 6 * HD and cache.stride(3) == 1
@@ -77,7 +74,17 @@ def _attend_int8(q, qpos, cache, bt, ptab, nsplit):
     q, qpos, ptab = q.contiguous().long(), qpos.contiguous().long(), ptab.contiguous()
     num = torch.empty(R, HKV, M, HD, dtype=torch.long, device=q.device)
     den = torch.empty(R, HKV, M, 1, dtype=torch.long, device=q.device)
+    keep = 0
+    if nsplit == 0:
+        nsplit, keep = auto_nsplit(R * HKV * ((M + 3) // 4), bt.shape[1] * cache.shape[2], HD)
     ws, wsb = _hip.workspace(q.device, _hip.lib().bx_attn_paged_workspace(R, HKV, M, HD) if nsplit > 1 else 0)
+    if keep:
+        tmp, tmpb = _hip.scratch(q.device, keep)
+        _hip.call("bx_int8_attn_paged_scores", _hip.ptr(q), _hip.ptr(qpos), qpos.stride(0), _hip.ptr(cache),
+                  cache.stride(0), cache.stride(1), cache.stride(2), cache.shape[2], _hip.ptr(bt), bt.stride(0),
+                  bt.shape[1], _hip.ptr(ptab), ptab.numel(), _hip.ptr(num), _hip.ptr(den), R, HKV, M, HD, int(nsplit),
+                  _hip.ptr(ws), wsb, _hip.ptr(tmp), tmpb, _hip.stream_of(q))
+        return num, den
     _hip.call("bx_int8_attn_paged", _hip.ptr(q), _hip.ptr(qpos), qpos.stride(0), _hip.ptr(cache), cache.stride(0),
               cache.stride(1), cache.stride(2), cache.shape[2], _hip.ptr(bt), bt.stride(0), bt.shape[1],
               _hip.ptr(ptab), ptab.numel(), _hip.ptr(num), _hip.ptr(den), R, HKV, M, HD, int(nsplit), _hip.ptr(ws),

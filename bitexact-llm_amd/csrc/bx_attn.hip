@@ -159,6 +159,7 @@ struct AttnArgs {
   int64_t* num_ws;                // [groups, nq, HD]
   int64_t* den_ws;                // [groups, nq]
   int32_t* sem;                   // [groups]
+  int64_t* raw;                   // split launches that keep the scores (null: K read in both)
   uint64_t exch_ticks;            // attn_dec_exch_kernel: longest wait for the other splits' maxima (100 MHz ticks)
 };
 
@@ -740,15 +741,16 @@ __device__ __forceinline__ void dec_finish_ao(const AttnArgs& p, const AoArgs& a
   }
 }
 
-// RAW (single launch only): sweep 1 keeps every score of the block's key range (p.S >= hi - lo of them per
-// query) in dynamic LDS and sweep 2 reads them back, so K is read once.
+// RAW (split launches): phase 0 writes every score to p.raw ([tile][key][query] int64, p.S keys a tile) and phase 1
+// reads them back, 32 bytes a key instead of K's 192 again. With enough splits for four blocks a CU in both launches
+// this is the form of long contexts and of grids that neither fill the chip unsplit nor fit the exchange kernel.
 template <int HD, int PHASE, bool RAW>
 __global__ __launch_bounds__(kDecWaves * 64) void attn_dec_kernel(AttnArgs p) {
   __shared__ DecSmem<HD> sm;
-  extern __shared__ __align__(16) int64_t raw_cache[];
   constexpr int KK = HD / 64;
   const int tiles = (p.nq + 3) / 4;
   const int tile = blockIdx.x, T = gridDim.x, sp = blockIdx.y, NS = gridDim.y;
+  int64_t* raws = RAW ? p.raw + (int64_t)tile * p.S * 4 : nullptr;
   const int group = tile / tiles, q0 = (tile % tiles) * 4;
   const int nvalid = min(4, p.nq - q0);
   const int h = group % p.hkv;
@@ -769,6 +771,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void attn_dec_kernel(AttnArgs p) {
   __syncthreads();
   int64_t kend = 0;
   for (int i = 0; i < 4; ++i) kend = imax(kend, sm.qpos[i] + 1);
+  if (RAW) kend = imin(kend, p.S);                 // (qpos < the block table's keys: the scores' bound in any case)
   int64_t lo64, hi64;
   split_range(kend, NS, sp, lo64, hi64);
   const int lo = (int)lo64, hi = (int)hi64;
@@ -789,7 +792,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void attn_dec_kernel(AttnArgs p) {
       if (b + kDecWaves < nb16) dec_rows<HD, true, false>(p, pg, h, min(s + 16 * kDecWaves, hi - 1), nxt);
       if (b + 2 * kDecWaves < nb16) pg = dec_page(p, brow, min(s + 32 * kDecWaves, hi - 1));
       const int64_t raw = dec_score<HD>(qa, cur);
-      if (RAW && s < hi && s - lo < p.S) raw_cache[qo * p.S + (s - lo)] = raw;
+      if (RAW && s < hi) raws[(int64_t)s * 4 + qo] = raw;
       if (s < hi && s <= my_qpos) best = imax(best, raw);
       cur = nxt;
     }
@@ -819,12 +822,16 @@ __global__ __launch_bounds__(kDecWaves * 64) void attn_dec_kernel(AttnArgs p) {
     for (int kk = 0; kk < KK; ++kk) num[i][kk] = 0;
   KvRegs<HD> cur, nxt;
   int pg = 0;
-  if (w < nb16) dec_rows<HD, !RAW, true>(p, dec_page(p, brow, min(lo + w * 16 + kl, hi - 1)), h,
-                                        min(lo + w * 16 + kl, hi - 1), cur);
+  int64_t rcur = 0, rnxt = 0;
+  if (w < nb16) {
+    const int s = min(lo + w * 16 + kl, hi - 1);
+    if (RAW) rcur = raws[(int64_t)s * 4 + qo];
+    dec_rows<HD, !RAW, true>(p, dec_page(p, brow, s), h, s, cur);
+  }
   if (w + kDecWaves < nb16) pg = dec_page(p, brow, min(lo + (w + kDecWaves) * 16 + kl, hi - 1));
   for (int b = w; b < nb16; b += kDecWaves) {
     const int s = lo + b * 16 + kl;
-    const int64_t raw = RAW ? (s < hi && s - lo < p.S ? raw_cache[qo * p.S + (s - lo)] : 0) : dec_score<HD>(qa, cur);
+    const int64_t raw = RAW ? rcur : dec_score<HD>(qa, cur);
     // the weight's table loads go out before the next block's requests (loads complete in order: waiting for
     // them then does not wait for the prefetch) and unconditionally (a hidden key's weight is discarded)
     WeightAt wat;
@@ -837,7 +844,10 @@ __global__ __launch_bounds__(kDecWaves * 64) void attn_dec_kernel(AttnArgs p) {
       i8 = int8_index(raw - mx, p.zsh, p.zmul);
       ta = p.ptab[imin(imax(i8, 0), -kI8ZLo)];   // a visible key has d <= 0, so idx <= -kI8ZLo (z = 0)
     }
-    if (b + kDecWaves < nb16) dec_rows<HD, !RAW, true>(p, pg, h, min(s + 16 * kDecWaves, hi - 1), nxt);
+    if (b + kDecWaves < nb16) {
+      dec_rows<HD, !RAW, true>(p, pg, h, min(s + 16 * kDecWaves, hi - 1), nxt);
+      if (RAW) rnxt = raws[(int64_t)min(s + 16 * kDecWaves, hi - 1) * 4 + qo];
+    }
     if (b + 2 * kDecWaves < nb16) pg = dec_page(p, brow, min(s + 32 * kDecWaves, hi - 1));
     int64_t pw = p.wrule == 0 ? weight_of(wat, ta, tb) : (i8 >= 0 ? ta : 0);
     if (!(qo < nvalid && s < hi && s <= my_qpos)) pw = 0;
@@ -874,6 +884,7 @@ __global__ __launch_bounds__(kDecWaves * 64) void attn_dec_kernel(AttnArgs p) {
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_wave_barrier();
     cur = nxt;
+    rcur = rnxt;
   }
   dec_finish<HD>(p, sm, ws, den, num, tile, sp, NS, group, q0, nvalid);
 }
@@ -2221,13 +2232,20 @@ static int launch_dec(AttnArgs& p, int groups, int64_t max_keys, hipStream_t st)
   const int tiles = (p.nq + 3) / 4;
   dim3 grid(groups * tiles, p.nsplit);
   const int64_t chunk = ((max_keys + p.nsplit - 1) / p.nsplit + 63) / 64 * 64;   // keys per split, at most
-  if (p.nsplit > 1 && chunk <= 64 * kDecWaves && (int64_t)grid.x * grid.y <= kDecExchBlocks) {
+  if (p.raw == nullptr && p.nsplit > 1 && chunk <= 64 * kDecWaves && (int64_t)grid.x * grid.y <= kDecExchBlocks) {
     // BX_ATTN_EXCH_TICKS (tests): a shorter wait, down to 0, where blocks compute the maxima they have not seen
     const char* et = getenv("BX_ATTN_EXCH_TICKS");
     p.exch_ticks = et ? (uint64_t)strtoull(et, nullptr, 10) : kDecExchTicks;
     if (chunk <= 32 * kDecWaves) attn_dec_exch_kernel<HD, 2><<<grid, kDecWaves * 64, 0, st>>>(p);
     else attn_dec_exch_kernel<HD, 4><<<grid, kDecWaves * 64, 0, st>>>(p);
     return check_launch("attn_dec_exch_kernel");
+  }
+  if (p.raw != nullptr) {
+    p.S = (int)max_keys;
+    attn_dec_kernel<HD, 0, true><<<grid, kDecWaves * 64, 0, st>>>(p);
+    if (int rc = check_launch("attn_dec_kernel(scores)")) return rc;
+    attn_dec_kernel<HD, 1, true><<<grid, kDecWaves * 64, 0, st>>>(p);
+    return check_launch("attn_dec_kernel");
   }
   if (p.nsplit > 1) {
     attn_dec_kernel<HD, 0, false><<<grid, kDecWaves * 64, 0, st>>>(p);
@@ -2265,11 +2283,26 @@ extern "C" int64_t bx_attn_paged_workspace(int32_t R, int32_t HKV, int32_t M, in
   return dec_ws_bytes(T, dec_split_cap(T), HD);
 }
 
-extern "C" int bx_exact_attn_paged(const int32_t* q, const int64_t* sh, const int64_t* qpos, int64_t sqpos_r,
-                                   const int8_t* cache, int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs,
-                                   const int32_t* bt, int64_t sbt, int32_t nblk, const int64_t* rmap, const int64_t* lut,
-                                   int64_t l2e, int64_t* num, int64_t* den, int32_t R, int32_t HKV, int32_t M,
-                                   int32_t HD, int32_t nsplit, void* ws, int64_t ws_bytes, bx_stream_t stream) {
+// The kept-scores form's scratch (`tmp` of the *_scores entries): every (tile, key, query) score
+extern "C" int64_t bx_attn_paged_scores_scratch(int32_t R, int32_t HKV, int32_t M, int32_t keys) {
+  if (R <= 0 || HKV <= 0 || M <= 0 || keys <= 0) return 0;
+  return (int64_t)R * HKV * ((M + 3) / 4) * keys * 32;
+}
+
+static int bind_scores(AttnArgs& p, int64_t T, int64_t keys, void* tmp, int64_t tmp_bytes) {
+  BX_REQUIRE(p.nsplit > 1, "the kept-scores form needs nsplit > 1");
+  BX_REQUIRE(tmp_bytes >= T * keys * 32 && ((uintptr_t)tmp & 7) == 0, "scratch too small (%lld < %lld)",
+             (long long)tmp_bytes, (long long)(T * keys * 32));
+  p.raw = (int64_t*)tmp;
+  return BX_OK;
+}
+
+static int exact_paged(const int32_t* q, const int64_t* sh, const int64_t* qpos, int64_t sqpos_r,
+                       const int8_t* cache, int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs,
+                       const int32_t* bt, int64_t sbt, int32_t nblk, const int64_t* rmap, const int64_t* lut,
+                       int64_t l2e, int64_t* num, int64_t* den, int32_t R, int32_t HKV, int32_t M,
+                       int32_t HD, int32_t nsplit, void* ws, int64_t ws_bytes, void* tmp, int64_t tmp_bytes,
+                       bx_stream_t stream) {
   BX_REQUIRE(R >= 0 && HKV > 0 && M >= 1 && M <= 4, "need 1 <= M <= 4 queries per (row, KV head)");
   BX_REQUIRE(HD == 64 || HD == 128, "head_dim must be 64 or 128");
   BX_REQUIRE((int64_t)nblk * bs < 43690, "keys per row must stay below 43690");
@@ -2296,8 +2329,30 @@ extern "C" int bx_exact_attn_paged(const int32_t* q, const int64_t* sh, const in
     p.mx_ws = (int64_t*)ws;
   }
   const int64_t max_keys = (int64_t)nblk * bs;     // qpos < nblk bs: the block table's reach
+  if (tmp != nullptr)
+    if (int rc = bind_scores(p, (int64_t)R * HKV * ((M + 3) / 4), max_keys, tmp, tmp_bytes)) return rc;
   return HD == 64 ? launch_dec<64>(p, R * HKV, max_keys, (hipStream_t)stream)
                   : launch_dec<128>(p, R * HKV, max_keys, (hipStream_t)stream);
+}
+
+extern "C" int bx_exact_attn_paged(const int32_t* q, const int64_t* sh, const int64_t* qpos, int64_t sqpos_r,
+                                   const int8_t* cache, int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs,
+                                   const int32_t* bt, int64_t sbt, int32_t nblk, const int64_t* rmap, const int64_t* lut,
+                                   int64_t l2e, int64_t* num, int64_t* den, int32_t R, int32_t HKV, int32_t M,
+                                   int32_t HD, int32_t nsplit, void* ws, int64_t ws_bytes, bx_stream_t stream) {
+  return exact_paged(q, sh, qpos, sqpos_r, cache, sc_nb, sc_h, sc_bs, bs, bt, sbt, nblk, rmap, lut, l2e, num, den, R, HKV,
+                     M, HD, nsplit, ws, ws_bytes, nullptr, 0, stream);
+}
+
+extern "C" int bx_exact_attn_paged_scores(const int32_t* q, const int64_t* sh, const int64_t* qpos, int64_t sqpos_r,
+                                          const int8_t* cache, int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs,
+                                          const int32_t* bt, int64_t sbt, int32_t nblk, const int64_t* rmap,
+                                          const int64_t* lut, int64_t l2e, int64_t* num, int64_t* den, int32_t R,
+                                          int32_t HKV, int32_t M, int32_t HD, int32_t nsplit, void* ws,
+                                          int64_t ws_bytes, void* tmp, int64_t tmp_bytes, bx_stream_t stream) {
+  BX_REQUIRE(tmp != nullptr || R == 0, "null scratch");
+  return exact_paged(q, sh, qpos, sqpos_r, cache, sc_nb, sc_h, sc_bs, bs, bt, sbt, nblk, rmap, lut, l2e, num, den, R, HKV,
+                     M, HD, nsplit, ws, ws_bytes, tmp, tmp_bytes, stream);
 }
 
 static int attn_rope_common(const int64_t* y, int64_t ldy, const int64_t* pos, int64_t spos, const int64_t* cos,
@@ -2419,11 +2474,12 @@ extern "C" int bx_exact_attn_paged_rope_out_planes(const int64_t* y, int64_t ldy
                        (hipStream_t)stream);
 }
 
-extern "C" int bx_int8_attn_paged(const int64_t* q, const int64_t* qpos, int64_t sqpos_r, const int8_t* cache,
+static int int8_paged(const int64_t* q, const int64_t* qpos, int64_t sqpos_r, const int8_t* cache,
                                   int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs, const int32_t* bt, int64_t sbt,
                                   int32_t nblk, const int32_t* ptab, int32_t ptab_len, int64_t* num, int64_t* den,
                                   int32_t R, int32_t HKV, int32_t M, int32_t HD, int32_t nsplit, void* ws,
-                                  int64_t ws_bytes, bx_stream_t stream) {
+                                  int64_t ws_bytes, void* tmp, int64_t tmp_bytes,
+                      bx_stream_t stream) {
   BX_REQUIRE(R >= 0 && HKV > 0 && M >= 1, "need M >= 1 queries per (row, KV head)");
   BX_REQUIRE(HD == 64 || HD == 128, "head_dim must be 64 or 128");
   BX_REQUIRE((int64_t)nblk * bs < 43690, "keys per row must stay below 43690");
@@ -2453,8 +2509,30 @@ extern "C" int bx_int8_attn_paged(const int64_t* q, const int64_t* qpos, int64_t
     p.mx_ws = (int64_t*)ws;
   }
   const int64_t max_keys = (int64_t)nblk * bs;     // qpos < nblk bs: the block table's reach
+  if (tmp != nullptr)
+    if (int rc = bind_scores(p, (int64_t)R * HKV * ((M + 3) / 4), max_keys, tmp, tmp_bytes)) return rc;
   return HD == 64 ? launch_dec<64>(p, R * HKV, max_keys, (hipStream_t)stream)
                   : launch_dec<128>(p, R * HKV, max_keys, (hipStream_t)stream);
+}
+
+extern "C" int bx_int8_attn_paged(const int64_t* q, const int64_t* qpos, int64_t sqpos_r, const int8_t* cache,
+                                  int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs, const int32_t* bt, int64_t sbt,
+                                  int32_t nblk, const int32_t* ptab, int32_t ptab_len, int64_t* num, int64_t* den,
+                                  int32_t R, int32_t HKV, int32_t M, int32_t HD, int32_t nsplit, void* ws,
+                                  int64_t ws_bytes, bx_stream_t stream) {
+  return int8_paged(q, qpos, sqpos_r, cache, sc_nb, sc_h, sc_bs, bs, bt, sbt, nblk, ptab, ptab_len, num, den,
+                    R, HKV, M, HD, nsplit, ws, ws_bytes, nullptr, 0, stream);
+}
+
+extern "C" int bx_int8_attn_paged_scores(const int64_t* q, const int64_t* qpos, int64_t sqpos_r, const int8_t* cache,
+                                  int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs, const int32_t* bt, int64_t sbt,
+                                  int32_t nblk, const int32_t* ptab, int32_t ptab_len, int64_t* num, int64_t* den,
+                                  int32_t R, int32_t HKV, int32_t M, int32_t HD, int32_t nsplit, void* ws,
+                                  int64_t ws_bytes, void* tmp, int64_t tmp_bytes,
+                                  bx_stream_t stream) {
+  BX_REQUIRE(tmp != nullptr || R == 0, "null scratch");
+  return int8_paged(q, qpos, sqpos_r, cache, sc_nb, sc_h, sc_bs, bs, bt, sbt, nblk, ptab, ptab_len, num, den,
+                    R, HKV, M, HD, nsplit, ws, ws_bytes, tmp, tmp_bytes, stream);
 }
 
 // the limb-plane form's scratch: K and V planes, 3 Z Sp HD bytes each (Sp = S rounded up to 64 keys)

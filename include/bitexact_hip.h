@@ -136,6 +136,17 @@ int bx_exact_attn_paged(const int32_t* q, const int64_t* sh, const int64_t* qpos
                         int32_t R, int32_t HKV, int32_t M, int32_t HD, int32_t nsplit, void* ws, int64_t ws_bytes,
                         bx_stream_t stream);
 
+/* bx_exact_attn_paged with the scores of every (query, key) kept in scratch between its two launches (nsplit > 1), so
+ * K is read once: the same call of the reference. tmp: 8-byte aligned, bx_attn_paged_scores_scratch(R, HKV, M, nblk
+ * bs) bytes, no contents kept. */
+int64_t bx_attn_paged_scores_scratch(int32_t R, int32_t HKV, int32_t M, int32_t keys);
+int bx_exact_attn_paged_scores(const int32_t* q, const int64_t* sh, const int64_t* qpos, int64_t sqpos_r,
+                               const int8_t* cache, int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs,
+                               const int32_t* bt, int64_t sbt, int32_t nblk, const int64_t* rmap, const int64_t* lut,
+                               int64_t l2e, int64_t* num, int64_t* den, int32_t R, int32_t HKV, int32_t M, int32_t HD,
+                               int32_t nsplit, void* ws, int64_t ws_bytes, void* tmp, int64_t tmp_bytes,
+                               bx_stream_t stream);
+
 /* The same attention for steps of many tokens per sequence (prefill chunks; the same reference call): the token rows
  * are grouped by block-table row on the device, each sequence's cached K / V limbs are laid out once per call as
  * planes in tmp, and a block runs many tokens of one sequence against each key tile (bx_exact_attn_prefill's main
@@ -203,6 +214,14 @@ int bx_int8_attn_paged(const int64_t* q, const int64_t* qpos, int64_t sqpos_r, c
                        int64_t sc_h, int64_t sc_bs, int32_t bs, const int32_t* bt, int64_t sbt, int32_t nblk,
                        const int32_t* ptab, int32_t ptab_len, int64_t* num, int64_t* den, int32_t R, int32_t HKV,
                        int32_t M, int32_t HD, int32_t nsplit, void* ws, int64_t ws_bytes, bx_stream_t stream);
+
+/* bx_int8_attn_paged with the scores kept in scratch, as bx_exact_attn_paged_scores (the same call of the reference,
+ * tri_paged.attend, src/bitexact/vllm_plugin/tri_paged.py:363-430). */
+int bx_int8_attn_paged_scores(const int64_t* q, const int64_t* qpos, int64_t sqpos_r, const int8_t* cache, int64_t sc_nb,
+                              int64_t sc_h, int64_t sc_bs, int32_t bs, const int32_t* bt, int64_t sbt, int32_t nblk,
+                              const int32_t* ptab, int32_t ptab_len, int64_t* num, int64_t* den, int32_t R, int32_t HKV,
+                              int32_t M, int32_t HD, int32_t nsplit, void* ws, int64_t ws_bytes, void* tmp,
+                              int64_t tmp_bytes, bx_stream_t stream);
 
 /* Fused form of exact/model.py's attention (src/bitexact/exact/model.py:113-119: bmm(qg, K^T), segs.softmax,
  * bmm(p, V)): qg int32 [Z, gT, HD] (strides sq_z, sq_row), shg int64 [Z, gT] (ssh_z = gT), qpos int64 [Z, gT]

@@ -195,6 +195,44 @@ def test_prefill_attention_full_size(dev, HD, T, Z):
                                                                                      ref_den[0])
 
 
+@pytest.mark.parametrize("mode", ["exact", "int8"])
+@pytest.mark.parametrize("HD,Rr,M,keys", [(64, 16, 4, 2064), (64, 8, 3, 4096), (128, 16, 1, 2048), (128, 9, 4, 4112)])
+def test_paged_kept_scores(dev, mode, HD, Rr, M, keys):
+    """Long contexts keep the scores between their two launches (attend chooses that by size): equal to the one-launch
+    or K-twice forms on every row, with contexts that end anywhere in the table (one key, a split's first and last
+    key, none), and repeated (the workspace is left zero)."""
+    from bitexact.int8.consts import exp_table
+    from bitexact.vllm_plugin import tri_exact_attn, tri_paged
+    g = torch.Generator().manual_seed(keys)
+    HKV, bs = 8, 16
+    nblk = keys // bs
+    tiles = Rr * HKV
+    split, need = tri_exact_attn.auto_nsplit(tiles, keys, HD)
+    assert need > 0 and split > 1
+    lim = R.LIM3 if mode == "exact" else 1 << 14
+    cl = tri_paged.to_limbs(torch.randint(-lim, lim + 1, (Rr * nblk, HKV, bs, 2 * HD), generator=g).to(torch.int32).to(dev))
+    bt = torch.randperm(Rr * nblk, generator=g).to(torch.int32).view(Rr, nblk).to(dev)
+    qpos = torch.full((Rr, M), keys - 1)
+    ends = [0, 1, 63, 64, keys // split - 1, keys // split, keys - 2, -1]
+    for i, e in enumerate(ends):
+        qpos[i] = e
+    qpos[3, 0] = 700
+    qpos = qpos.to(dev)
+    if mode == "exact":
+        q = torch.randint(-(1 << 22), (1 << 22) + 1, (Rr, HKV, M, HD), generator=g).to(torch.int32).to(dev)
+        sh = torch.randint(-44, -36, (Rr, HKV, M), generator=g).to(dev)
+        run = lambda **k: tri_exact_attn.attend(q, sh, qpos, cl, bt, torch.arange(Rr, device=dev), _lut(dev),
+                                                R.L2E28_HD[HD], **k)
+    else:
+        q = torch.randint(-(1 << 15), (1 << 15) + 1, (Rr, HKV, M, HD), generator=g).to(dev)
+        ptab = tri_paged.weight_table(exp_table(dev))
+        run = lambda **k: tri_paged.attend(q, qpos, cl, bt, ptab, **k)
+    n1, d1 = run(nsplit=1)
+    for _ in range(3):
+        n2, d2 = run()
+        assert torch.equal(n1, n2) and torch.equal(d1, d2)
+
+
 @pytest.mark.parametrize("HD,M,bs", [(64, 4, 16), (64, 3, 16), (64, 1, 32), (128, 4, 16), (128, 2, 16)])
 @pytest.mark.parametrize("order", ["runs", "mixed"])
 def test_paged_rows_equal_decode_form(dev, HD, M, bs, order):
