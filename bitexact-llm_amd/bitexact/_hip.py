@@ -6,6 +6,7 @@ RuntimeError. There is no fallback: without the built library or a GPU the impor
 """
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -121,22 +122,43 @@ def lib():
     return _lib
 
 
+# The launch path's own cost bounds the smallest calls (a one-token linear: 15 us of host time around 7 us on the
+# device), so it avoids torch.cuda.Stream and ctypes objects: addresses and stream handles pass as plain integers
+# (the c_void_p argument types convert them) and the library's functions are looked up once.
 def ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # absent from builds without a GPU backend
 
 
 def stream_of(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    """The current stream of t's device, as an integer handle."""
+    i = t.get_device()
+    return torch.cuda.current_stream(i).cuda_stream if _raw_stream is None else _raw_stream(i)
+
+
+_fn = {}
 
 
 def call(name, *args):
-    rc = getattr(lib(), name)(*args)
+    f = _fn.get(name)
+    if f is None:
+        f = _fn[name] = getattr(lib(), name)
+    rc = f(*args)
     if rc == 0:
         return
     msg = lib().bx_last_error().decode(errors="replace")
     if rc == -1:
         raise AssertionError(f"{name}: {msg}")
     raise RuntimeError(f"{name} failed ({rc}): {msg}")
+
+
+@functools.lru_cache(8192)
+def size_query(name, dev, *sizes):
+    """One of the library's size queries (workspace, scratch bytes: functions of the sizes and of device `dev`'s
+    compute units, asked while it is the current device as the launch itself requires)."""
+    return getattr(lib(), name)(*sizes)
 
 
 def require_cuda(*ts):
@@ -153,7 +175,8 @@ _ws = {}
 def _buffer(kind, dev, nbytes):
     if nbytes <= 0:
         return None, 0
-    key = (kind, dev.index, torch.cuda.current_stream(dev).cuda_stream)
+    i = dev.index
+    key = (kind, i, torch.cuda.current_stream(dev).cuda_stream if _raw_stream is None or i is None else _raw_stream(i))
     buf = _ws.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = (torch.zeros if kind == "ws" else torch.empty)(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)

@@ -22,8 +22,8 @@ def int_mm(a, w):
     _check(a, w)
     R, K = a.shape
     N = w.shape[0]
-    c = torch.empty(R, N, dtype=torch.int32, device=a.device)
-    ws, wsb = _hip.workspace(a.device, _hip.lib().bx_int8_gemm_workspace(R, N, K, 1))
+    c = a.new_empty((R, N), dtype=torch.int32)
+    ws, wsb = _hip.workspace(a.device, _hip.size_query("bx_int8_gemm_workspace", a.device.index, R, N, K, 1))
     _hip.call("bx_int8_gemm", _hip.ptr(a), _hip.ptr(w), _hip.ptr(c), R, N, K, _hip.ptr(ws), wsb, _hip.stream_of(a))
     return c
 
@@ -36,8 +36,8 @@ def int_mm_join(a, w, M, nl):
     K = a.shape[1]
     N = w.shape[0]
     assert a.shape[0] >= nl * M
-    y = torch.empty(M, N, dtype=torch.long, device=a.device)
-    ws, wsb = _hip.workspace(a.device, _hip.lib().bx_int8_gemm_workspace(M, N, K, nl))
+    y = a.new_empty((M, N), dtype=torch.long)
+    ws, wsb = _hip.workspace(a.device, _hip.size_query("bx_int8_gemm_workspace", a.device.index, M, N, K, nl))
     _hip.call("bx_int8_gemm_join", _hip.ptr(a), _hip.ptr(w), _hip.ptr(y), M, N, K, nl, _hip.ptr(ws), wsb,
               _hip.stream_of(a))
     return y

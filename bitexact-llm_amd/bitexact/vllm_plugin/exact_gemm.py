@@ -46,10 +46,11 @@ def _exact_linear(q, sh, limbs, d, g, cnt, ec, ev, R, flag, checked, fr, q_plane
     assert limbs.shape[2] == K and sh.shape[0] == M
     if checked:
         assert flag is not None and flag.dtype == torch.int32
-    y = torch.empty(M, N, dtype=torch.long, device=q.device)
+    y = q.new_empty((M, N), dtype=torch.long)
     sh = sh.contiguous()
+    dev = q.device
     if q_planes is not None:
-        ws, wsb = _hip.workspace(q.device, _hip.lib().bx_exact_linear_planes_workspace(M, N, K))
+        ws, wsb = _hip.workspace(dev, _hip.size_query("bx_exact_linear_planes_workspace", dev.index, M, N, K))
         _hip.require_cuda(q_planes)
         assert q_planes.dtype == torch.int8 and q_planes.shape == (3, M, K) and q_planes.is_contiguous()
         _hip.call("bx_exact_linear_planes", _hip.ptr(q), q.stride(0), _hip.ptr(sh), _hip.ptr(limbs), limbs.stride(0),
@@ -57,8 +58,8 @@ def _exact_linear(q, sh, limbs, d, g, cnt, ec, ev, R, flag, checked, fr, q_plane
                   _hip.ptr(ec) if R else None, _hip.ptr(ev) if R else None, R, _hip.ptr(y), M, N, K, fr,
                   int(checked), _hip.ptr(flag), _hip.ptr(ws), wsb, _hip.ptr(q_planes), _hip.stream_of(q))
         return y
-    ws, wsb = _hip.workspace(q.device, _hip.lib().bx_exact_linear_workspace(M, N, K))
-    tmp, tmpb = _hip.scratch(q.device, _hip.lib().bx_exact_linear_scratch(M, N, K))
+    ws, wsb = _hip.workspace(dev, _hip.size_query("bx_exact_linear_workspace", dev.index, M, N, K))
+    tmp, tmpb = _hip.scratch(dev, _hip.size_query("bx_exact_linear_scratch", dev.index, M, N, K))
     _hip.call("bx_exact_linear", _hip.ptr(q), q.stride(0), _hip.ptr(sh), _hip.ptr(limbs), limbs.stride(0),
               limbs.stride(1), _hip.ptr(d), _hip.ptr(g), _hip.ptr(cnt) if R else None,
               _hip.ptr(ec) if R else None, _hip.ptr(ev) if R else None, R, _hip.ptr(y), M, N, K, fr, int(checked),

@@ -88,8 +88,8 @@ def _attend(q, sh, qpos, cache, bt, rmap, lut, l2e, nsplit):
     assert q.dtype == torch.int32 and cache.dtype == torch.int8 and bt.dtype == torch.int32
     q, sh, qpos = q.contiguous(), sh.contiguous().long(), qpos.contiguous().long()
     rmap, lut = rmap.contiguous().long(), lut.contiguous().long()
-    num = torch.empty(R, HKV, M, HD, dtype=torch.long, device=q.device)
-    den = torch.empty(R, HKV, M, 1, dtype=torch.long, device=q.device)
+    num = q.new_empty((R, HKV, M, HD), dtype=torch.long)
+    den = q.new_empty((R, HKV, M, 1), dtype=torch.long)
     keep = 0
     if nsplit == 0:
         need, nsplit, keep = _plan(R, HKV, M, HD, bt.shape[0], bt.shape[1] * cache.shape[2])
@@ -100,7 +100,8 @@ def _attend(q, sh, qpos, cache, bt, rmap, lut, l2e, nsplit):
                       bt.stride(0), bt.shape[0], bt.shape[1], _hip.ptr(rmap), _hip.ptr(lut), int(l2e), _hip.ptr(num),
                       _hip.ptr(den), R, HKV, M, HD, _hip.ptr(tmp), tmpb, _hip.stream_of(q))
             return num, den
-    ws, wsb = _hip.workspace(q.device, _hip.lib().bx_attn_paged_workspace(R, HKV, M, HD) if nsplit > 1 else 0)
+    ws, wsb = _hip.workspace(q.device, _hip.size_query("bx_attn_paged_workspace", q.device.index, R, HKV, M, HD)
+                              if nsplit > 1 else 0)
     if keep:
         tmp, tmpb = _hip.scratch(q.device, keep)
         _hip.call("bx_exact_attn_paged_scores", _hip.ptr(q), _hip.ptr(sh), _hip.ptr(qpos), qpos.stride(0), _hip.ptr(cache),

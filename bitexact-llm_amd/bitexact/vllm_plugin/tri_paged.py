@@ -72,12 +72,13 @@ def _attend_int8(q, qpos, cache, bt, ptab, nsplit):
     assert bt.shape[1] * cache.shape[2] < 43690
     assert cache.dtype == torch.int8 and bt.dtype == torch.int32 and ptab.dtype == torch.int32
     q, qpos, ptab = q.contiguous().long(), qpos.contiguous().long(), ptab.contiguous()
-    num = torch.empty(R, HKV, M, HD, dtype=torch.long, device=q.device)
-    den = torch.empty(R, HKV, M, 1, dtype=torch.long, device=q.device)
+    num = q.new_empty((R, HKV, M, HD), dtype=torch.long)
+    den = q.new_empty((R, HKV, M, 1), dtype=torch.long)
     keep = 0
     if nsplit == 0:
         nsplit, keep = auto_nsplit(R * HKV * ((M + 3) // 4), bt.shape[1] * cache.shape[2], HD)
-    ws, wsb = _hip.workspace(q.device, _hip.lib().bx_attn_paged_workspace(R, HKV, M, HD) if nsplit > 1 else 0)
+    ws, wsb = _hip.workspace(q.device, _hip.size_query("bx_attn_paged_workspace", q.device.index, R, HKV, M, HD)
+                              if nsplit > 1 else 0)
     if keep:
         tmp, tmpb = _hip.scratch(q.device, keep)
         _hip.call("bx_int8_attn_paged_scores", _hip.ptr(q), _hip.ptr(qpos), qpos.stride(0), _hip.ptr(cache),
