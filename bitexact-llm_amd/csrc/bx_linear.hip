@@ -1223,6 +1223,172 @@ __global__ __launch_bounds__(WM * WN * 64) void xtile_kernel(LinArgs p) {
 }
 
 // =====================================================================================================
+// itile kernel: int8-mode prefill GEMMs (NA activation limb planes, one weight plane, K % 64 == 0), pipelined as the
+// xtile kernel: WM x WN waves of 32 TM x 32 TN outputs over NA accumulator sets, an S-stage LDS ring of 64-deep k tiles
+// filled by buffer_load ... lds, the next half-step's operands read while this one's MFMAs run. Bound by the MFMA issue
+// with one LDS read among every one or two of them, and at short K by the 64-bit result stores (one limb: all of it).
+// A CU holds 256 x 128 x NA 32-bit accumulators, 96 to 192 registers a lane (three limbs on eight waves: one spilled
+// register read back per k tile): one block of eight waves, or two of four, whose prologues and stores then overlap the
+// other's MFMAs. M = 2048, N = 16384, K = 2048: one limb 118 -> 110 us, two 231 -> 154, three 309 -> 217, against
+// tile_kernel's 128 x 128 tile, which waits for its operands; M = 256, N = 4096, K = 4096: 28 -> 27, 35 -> 26, 40 -> 26.
+// =====================================================================================================
+template <int NA, int MODE, int WM, int WN, int TM, int TN, int S>
+__global__ __launch_bounds__(64 * WM * WN, 2) void itile_kernel(LinArgs p) {
+  constexpr int NW = WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN, BK = 64;
+  constexpr int SA = NA * BM * BK, STAGE = SA + BN * BK;
+  constexpr int LI = STAGE / 1024, LPW = LI / NW;           // 1 KiB load instructions per stage, per wave
+  static_assert(LI % NW == 0 && SA % 1024 == 0, "every wave issues the same number of loads");
+  extern __shared__ __align__(16) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, wn = wave / WM;
+  // XCD-aware tile order, as the xtile kernel's
+  int tx = blockIdx.x, ty = blockIdx.y;
+  if (p.xcd_remap) {
+    const int T = gridDim.x * gridDim.y, b = blockIdx.y * gridDim.x + blockIdx.x;
+    const int v = (b & 7) * (T >> 3) + (b >> 3), R = p.xcd_remap;
+    const int grp = v / (R * gridDim.x), in = v - grp * R * gridDim.x;
+    ty = grp * R + in % R;
+    tx = in / R;
+  }
+  const int m0 = ty * BM, n0 = tx * BN, nk = p.K / BK;
+
+  // ring loads: instruction n covers 16 rows x 64 bytes of A (planes in order) or B; lane: row lane / 4, 16-byte chunk
+  // lane % 4 swizzled. A wave's instructions may lie on both sides, so it keeps an offset and a base for each.
+  const int lrow = lane >> 2, lch = ((lane & 3) ^ swz<BK>(lrow)) << 4;
+  const __amdgpu_buffer_rsrc_t ra = buf_rsrc(p.a), rb = buf_rsrc(p.w);
+  int voff[LPW];
+#pragma unroll
+  for (int i = 0; i < LPW; ++i) {
+    const int inst = wave * LPW + i;
+    if (inst < SA / 1024) {
+      const int pl = inst / (BM / 16), row = (inst % (BM / 16)) * 16 + lrow;
+      voff[i] = (pl * p.M + min(m0 + row, p.M - 1)) * p.K + lch;
+    } else {
+      const int row = (inst - SA / 1024) * 16 + lrow;
+      voff[i] = min(n0 + row, p.N - 1) * (int)p.ld_row + lch;
+    }
+  }
+  auto issue = [&](int kt, int stage) {
+    char* sbase = smem + stage * STAGE + wave * LPW * 1024;
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) {
+      if (wave * LPW + i < SA / 1024) buf_lds16(ra, sbase + i * 1024, voff[i], kt * BK);   // wave-uniform
+      else buf_lds16(rb, sbase + i * 1024, voff[i], kt * BK);
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < S; ++t)
+    if (t < nk) issue(t, t);
+
+  struct Ops {
+    v4i a[NA][TM], b[TN];
+  };
+  auto load_ops = [&](Ops& o, int stage, int h) {
+    const char* base = smem + stage * STAGE;
+    const int c = 2 * h + (lane >> 5);
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int a2 = 0; a2 < TM; ++a2) {
+        const int arow = (wm * TM + a2) * 32 + (lane & 31);
+        o.a[i][a2] = *(const v4i*)(base + i * BM * BK + arow * BK + ((c ^ swz<BK>(arow)) << 4));
+      }
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+      const int brow = (wn * TN + t) * 32 + (lane & 31);
+      o.b[t] = *(const v4i*)(base + SA + brow * BK + ((c ^ swz<BK>(brow)) << 4));
+    }
+  };
+  v16i acc[NA][TM][TN];
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int a2 = 0; a2 < TM; ++a2)
+#pragma unroll
+      for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][a2][t][e] = 0;
+  auto mfmas = [&](const Ops& o) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int a2 = 0; a2 < TM; ++a2)
+#pragma unroll
+        for (int t = 0; t < TN; ++t)
+          acc[i][a2][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a[i][a2], o.b[t], acc[i][a2][t], 0, 0, 0);
+  };
+  if (S - 1 < nk) ring_barrier<LPW * (S - 1)>();
+  else ring_barrier<0>();
+  Ops cur, nxt;
+  if (nk > 0) load_ops(cur, 0, 0);
+  constexpr int NR = NA * TM + TN, NM = NA * TM * TN;       // LDS reads and MFMAs of a half-step
+  static_assert(NM >= NR && LPW <= NR, "interleave");
+  int st = 0;
+  auto step = [&](int it, auto refill) {
+    constexpr bool REFILL = decltype(refill)::value;
+    const int s1 = st + 1 == S ? 0 : st + 1;
+    load_ops(nxt, st, 1);
+    mfmas(cur);
+#pragma unroll
+    for (int g = 0; g < NR; ++g) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, NM - NR, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    // k tile it + 1 landed (the tiles after it may be in flight), and no wave reads stage st any more
+    if (REFILL) ring_barrier<LPW * (S - 2)>();
+    else ring_barrier<0>();
+    __builtin_amdgcn_sched_barrier(0);
+    if (REFILL) issue(it + S, st);
+    load_ops(cur, s1, 0);
+    mfmas(nxt);
+#pragma unroll
+    for (int g = 0; g < NR; ++g) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if (REFILL && g < LPW) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, NM - NR, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    st = s1;
+  };
+  int it = 0;
+  for (; it + S < nk; ++it) step(it, std::true_type{});
+  for (; it + 1 < nk; ++it) step(it, std::false_type{});
+  if (nk > 0) {
+    load_ops(nxt, st, 1);
+    mfmas(cur);
+    mfmas(nxt);
+  }
+
+  // epilogue: lane (l % 32) owns column (wn TN + t) 32 + l % 32 of each 32-column block and rows (wm TM + a2) 32 +
+  // (e / 4) 8 + (l / 32) 4 + e % 4; 32 lanes store 256 contiguous bytes (64-bit) of a row, streaming
+  const bool full = m0 + BM <= p.M && n0 + BN <= p.N;       // block-uniform
+#pragma unroll
+  for (int a2 = 0; a2 < TM; ++a2)
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+      const int n = n0 + (wn * TN + t) * 32 + (lane & 31);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int m = m0 + (wm * TM + a2) * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+        if (!full && !(m < p.M && n < p.N)) continue;
+        const int64_t o = (int64_t)m * p.N + n;
+        if constexpr (MODE == RAW32) {
+          __builtin_nontemporal_store(acc[0][a2][t][e], (int32_t*)p.out + o);
+        } else {
+          int64_t v = acc[0][a2][t][e];
+          if constexpr (NA > 1) v += (int64_t)acc[1][a2][t][e] << 8;
+          if constexpr (NA > 2) v += (int64_t)acc[2][a2][t][e] << 16;
+          __builtin_nontemporal_store(v, (int64_t*)p.out + o);
+        }
+      }
+    }
+}
+
+// =====================================================================================================
 // stream kernel: decode GEMMs (at most 128 stacked activation rows) as a weight stream through an LDS ring.
 // A block owns 64 output columns and a K range (the grid splits K when the column tiles alone do not fill the
 // chip). Its weight rows (NB planes x 64 x 128-byte k chunks) and all its activation rows (padded to RP, a
@@ -2056,8 +2222,85 @@ static bool xtile_fits(const LinArgs& p, const Plan& s) {
          2 * p.ld_plane + (int64_t)p.N * p.ld_row < kBufRange - 16 && (int64_t)p.M * p.ldq * 4 < kBufRange - 16;
 }
 
+// The itile kernel's shapes for NA limb planes: W waves, WM of them along the rows, each 32 TM x 32 TN outputs; S ring
+// stages. Four waves: 128 x 256, 128 x 128, 64 x 128 outputs a block and two blocks a CU; eight: 128 x 256 and one.
+template <int NA, int W>
+struct ItShape;
+template <>
+struct ItShape<1, 4> {
+  static constexpr int WM = 2, TM = 2, TN = 4, S = 3;
+};
+template <>
+struct ItShape<2, 4> {
+  static constexpr int WM = 2, TM = 2, TN = 2, S = 3;
+};
+template <>
+struct ItShape<2, 8> {
+  static constexpr int WM = 4, TM = 1, TN = 4, S = 4;
+};
+template <>
+struct ItShape<3, 4> {
+  static constexpr int WM = 2, TM = 1, TN = 2, S = 3;
+};
+template <>
+struct ItShape<3, 8> {
+  static constexpr int WM = 4, TM = 1, TN = 4, S = 3;
+};
+
+template <int NA, int W>
+static int64_t itile_tiles(const LinArgs& p) {
+  using I = ItShape<NA, W>;
+  constexpr int BM = 32 * I::TM * I::WM, BN = 32 * I::TN * (W / I::WM);
+  return (int64_t)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
+}
+
+// Waves of the itile shape for a product; 0: tile_kernel, which can split K.
+// A block walks all of K, so few tiles of a long K stay with the split: two limbs, K = 8192, 128 x 1024 outputs
+// (8 tiles) 42 us here and 24 split, 256 x 2048 (32 tiles) 51 and 37, 512 x 2048 (64 tiles) 53 and 65; three limbs
+// 256 x 2048 (64 tiles) 46 and 41, 384 x 2048 (96) 48 and 70. At K = 4096 the line is near 24 tiles (two limbs
+// 256 x 1024, 16 tiles: 24.0 and 25.9; 384 x 1024, 24 tiles: 24.3 and 29.7), at K = 2048 below 8 (256 x 256: 14.5 and
+// 15.3, 129 x 256: 14.5 and 13.3).
+// Eight waves re-read less and run a full chip faster (two limbs 2048 x 16384 of K = 2048: 154 us, four waves 159;
+// three: 216 and 241), four fill a part-empty last round better: the line is where the eight-wave tiles' rounds over
+// the CUs cover what the four-wave tiles need (two limbs 1024 x 4096 of K = 4096, 128 eight-wave tiles: 47 and 41 us;
+// 1500 x 4096, 192 tiles: 55 and 64; three limbs 700 x 16384, 384 tiles: 96 and 86).
+template <int NA>
+static int itile_waves(const LinArgs& p) {
+  // 32-bit sums over all of K (the split sums 64-bit parts) and 32-bit offsets
+  if (p.K % 64 || p.K >= 131072 || (int64_t)NA * p.M * p.K >= kBufRange - 16 ||
+      (int64_t)p.N * p.ld_row >= kBufRange - 16)
+    return 0;
+  const int64_t t4 = itile_tiles<NA, 4>(p);
+  if (t4 < (p.K <= 2048 ? 8 : p.K <= 4096 ? 24 : NA == 3 ? 96 : 64)) return 0;
+  if constexpr (NA == 1) {
+    return 4;
+  } else {
+    const int64_t cus = device_cus(), r8 = (itile_tiles<NA, 8>(p) + cus - 1) / cus;
+    return (NA == 2 ? 2 * r8 <= (t4 + cus - 1) / cus : 3 * r8 * cus <= t4) ? 8 : 4;
+  }
+}
+
+template <int NA, int MODE, int W>
+static int launch_itile(LinArgs& p, hipStream_t st) {
+  using I = ItShape<NA, W>;
+  constexpr int BM = 32 * I::TM * I::WM, WN = W / I::WM, BN = 32 * I::TN * WN;
+  constexpr size_t LDS = (size_t)I::S * (NA * BM + BN) * 64;
+  const int tx = (p.N + BN - 1) / BN, ty = (p.M + BM - 1) / BM;
+  p.xcd_remap = (tx * ty) % 8 == 0 && ty % 4 == 0 ? 4 : 0;
+  auto k = itile_kernel<NA, MODE, I::WM, WN, I::TM, I::TN, I::S>;
+  allow_lds(k, LDS);
+  k<<<dim3(tx, ty), 64 * W, LDS, st>>>(p);
+  return check_launch("itile_kernel");
+}
+
 template <int NA, int NB, int MODE>
 static int launch_tile(LinArgs& p, const Plan& s, hipStream_t st) {
+  if constexpr (NB == 1 && (MODE == JOIN || MODE == RAW32)) {
+    const int waves = itile_waves<NA>(p);
+    if (waves == 4) return launch_itile<NA, MODE, 4>(p, st);
+    if constexpr (NA > 1)
+      if (waves == 8) return launch_itile<NA, MODE, 8>(p, st);
+  }
   p.ks = s.kbytes;
   bind_ws(p, s);
   if (s.tile == T_BIG) {
@@ -2354,8 +2597,8 @@ extern "C" int bx_exact_linear_planes_plan(int32_t M, int32_t N, int32_t K, int3
 }
 
 // The int8 GEMM's plan for M output rows of nl stacked limbs (nl = 0: the raw int32 GEMM of M stacked rows):
-// out[0] = 1 gemv, 3 tile, 4 staged, 5 stream; out[1] = tile configuration (-1 otherwise); out[2] = K splits; out[3] =
-// blocks per split; out[4] = gemv column groups (16 columns each); out[5] = gemv row parts.
+// out[0] = 1 gemv, 3 tile (itile where its rule takes it: no split then), 4 staged, 5 stream; out[1] = tile
+// configuration (-1 otherwise); out[2] = K splits; out[3] = blocks per split; out[4] = gemv column groups (16 columns each); out[5] = gemv row parts.
 extern "C" int bx_int8_gemm_plan(int32_t M, int32_t N, int32_t K, int32_t nl, int32_t* out) {
   BX_REQUIRE(out && M > 0 && N > 0 && K > 0 && nl >= 0 && nl <= 3, "bad plan query");
   const Plan s = nl == 0 ? make_plan(M, M, N, K, 1, 1, false) : make_plan(nl * M, M, N, K, 1, nl, false);

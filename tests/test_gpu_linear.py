@@ -512,3 +512,23 @@ def test_int8_stream_wide(dev, N, K):
         a[0, :] = -128
         c = int_mm(torch.from_numpy(a).to(dev), wd)
         assert np.array_equal(c.cpu().numpy().astype(np.int64), R.imm(a, w)), (Rr, "raw")
+
+
+@pytest.mark.parametrize("M,N,K,nl", [(129, 2060, 64, 1), (300, 1800, 192, 1), (130, 513, 128, 2), (65, 1025, 320, 2),
+                                      (2049, 2050, 192, 2), (2040, 2302, 320, 2), (44, 1025, 64, 3), (257, 260, 2048, 3),
+                                      (2049, 3000, 128, 3), (2050, 3070, 256, 3), (200, 2050, 2112, 0),
+                                      (384, 4100, 64, 0)])
+def test_int8_pipelined_tiles(dev, M, N, K, nl):
+    """int8 prefill on the pipelined tiles (four- and eight-wave shapes, nl = 0: raw int32 rows): ragged last row and
+    column tiles, K of one to a few k tiles (fewer than the ring's stages too), extreme operands."""
+    from bitexact.int8.gemm_skinny import int_mm, int_mm_join
+    g = np.random.default_rng(M + N + K)
+    w = g.integers(-128, 128, (N, K)).astype(np.int8)
+    w[N - 1, :] = -128
+    a = g.integers(-128, 128, (max(nl, 1) * M, K)).astype(np.int8)
+    a[M - 1, :] = -128
+    a[0, :] = 127
+    ad, wd = torch.from_numpy(a).to(dev), torch.from_numpy(w).to(dev)
+    y = int_mm(ad, wd) if nl == 0 else int_mm_join(ad, wd, M, nl)
+    parts = [R.imm(a[i * M:(i + 1) * M], w) << (8 * i) for i in range(max(nl, 1))]
+    assert np.array_equal(y.cpu().numpy().astype(np.int64), sum(parts))
