@@ -162,6 +162,147 @@ __global__ __launch_bounds__(256 * RT) void bmm_mfma_kernel(const TA* a, int64_t
   }
 }
 
+// Rows kernel: 3 x 3 limbs of int32 operands, a's rows contiguous (p.v's weights). A's values never pass through LDS: lane (r, ch) of a wave loads k = 16 u + 4 ch .. + 3 (u = 0..3) of row r
+// as four 16-byte words (64 contiguous bytes of a row per four lanes), splits them in registers and has the MFMA's A
+// operand in place, with the step's k order permuted to 16 ch + 4 u + e; B's limb planes are written to LDS in the same
+// order, into one of two buffers, so a step has one barrier. A's next PA steps travel while the MFMAs run. Buffer loads
+// of four dwords need 4-byte alignment only; a part-filled last k step loads single values, those past K as zeros of a.
+// NW waves of 16 rows x 16 CB columns; BV: b's k contiguous; TAIL: K % 64 != 0. Bound by reading a: Z = 16, 4096 x 1024 by 64 columns
+// 116 -> 71 us (268 MB, 4.2 TB/s with the results), by 128 columns 209 -> 111; bmm_mfma_kernel has four bounds-checked
+// 4-byte loads for each of this kernel's 16-byte ones, two barriers a step, and A's planes through LDS.
+template <int CB, int NW, int PA, bool BV, bool TAIL>
+__global__ __launch_bounds__(64 * NW, 2) void bmm_rows_kernel(const int32_t* a, int64_t saz, int64_t sam, const int32_t* b,
+                                                           int64_t sbz, int64_t sbk, int64_t sbn, int64_t* c, int64_t scz,
+                                                           int64_t scm, int64_t scn, int M, int N, int K) {
+  constexpr int BN = 16 * CB, BP = BN * kBT, GB = BN * 16 / (64 * NW);   // B's load groups of four k per thread
+  __shared__ __align__(16) int8_t Bs[2][3 * BP];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, ch = lane >> 4;
+  const int mb = blockIdx.y * NW * 16, m0 = mb + wave * 16, n0 = blockIdx.x * BN;
+  const int64_t z = blockIdx.z;
+  const int nf = K / kBT, nk = (K + kBT - 1) / kBT;         // whole steps, steps
+  const auto ra = buf_rsrc(a + z * saz + mb * sam), rb = buf_rsrc(b + z * sbz);
+  const int oa = (min(m0 + r16, M - 1) - mb) * (int)sam * 4 + 16 * ch;   // rows past M: another's, not stored
+  const int sk4 = (int)sbk * 4;
+  int ob[GB], bw[GB];                     // the group's byte offsets in b's matrix and in a B plane
+#pragma unroll
+  for (int g = 0; g < GB; ++g) {
+    const int idx = tid + 64 * NW * g, n = BV ? idx / 16 : idx % BN, q = BV ? idx % 16 : idx / BN;
+    ob[g] = min(n0 + n, N - 1) * (int)sbn * 4 + 4 * q * sk4;
+    bw[g] = swz(n, q & 3) + (q >> 2) * 4;
+  }
+  v4i va[PA][4], vb[GB];
+  auto fetch_a = [&](int st, v4i (&v)[4]) {
+    if (!TAIL || st < nf) {               // block-uniform
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        v[u] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ra, oa + 64 * u, st * kBT * 4, 0));
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)       // past the buffer's range: reads 0
+          v[u][e] = __builtin_amdgcn_raw_buffer_load_b32(
+              ra, st * kBT + 16 * u + 4 * ch + e < K ? oa + (st * kBT + 16 * u + e) * 4 : kBufRange, 0, 0);
+    }
+  };
+  auto fetch_b = [&](int st) {
+#pragma unroll
+    for (int g = 0; g < GB; ++g) {
+      if (TAIL && st >= nf) {             // block-uniform; past K: any of the column's values (a has zeros there)
+        const int idx = tid + 64 * NW * g, k = st * kBT + 4 * (BV ? idx % 16 : idx / BN);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          vb[g][e] = __builtin_amdgcn_raw_buffer_load_b32(rb, ob[g] + (st * kBT + min(e, K - 1 - k)) * sk4, 0, 0);
+      } else if constexpr (BV) {
+        vb[g] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rb, ob[g], st * kBT * 4, 0));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vb[g][e] = __builtin_amdgcn_raw_buffer_load_b32(rb, ob[g], (st * kBT + e) * sk4, 0);
+      }
+    }
+  };
+  // the first three signed digits of four values: one word per limb
+  auto split4 = [](v4i v, uint32_t (&w)[3]) {
+    const uint32_t u0 = v[0] + 0x808080u, u1 = v[1] + 0x808080u, u2 = v[2] + 0x808080u, u3 = v[3] + 0x808080u;
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      const uint32_t sel = (uint32_t)l | ((uint32_t)(4 + l) << 8) | 0x0c0c0000u;
+      w[l] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(u3, u2, sel), __builtin_amdgcn_perm(u1, u0, sel), 0x05040100u) ^
+             0x80808080u;
+    }
+  };
+  v4i acc[5][CB];
+#pragma unroll
+  for (int s = 0; s < 5; ++s)
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) acc[s][cb] = v4i{0, 0, 0, 0};
+  fetch_b(0);
+#pragma unroll
+  for (int h = 0; h < PA; ++h)
+    if (h < nk) fetch_a(h, va[h]);
+  auto step = [&](int st, v4i (&vh)[4]) {
+      int8_t* bs = Bs[st & 1];            // last read two steps ago, before the previous step's barrier
+#pragma unroll
+      for (int g = 0; g < GB; ++g) {
+        uint32_t w[3];
+        split4(vb[g], w);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) *(uint32_t*)(bs + l * BP + bw[g]) = w[l];
+      }
+      __syncthreads();
+      if (st + 1 < nk) fetch_b(st + 1);
+      v4i af[3];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        uint32_t w[3];
+        split4(vh[u], w);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) af[l][u] = (int)w[l];
+      }
+      if (st + PA < nk) fetch_a(st + PA, vh);
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          const v4i bf = *(const v4i*)(bs + j * BP + swz(16 * cb + r16, ch));
+#pragma unroll
+          for (int i = 0; i < 3; ++i)
+            acc[i + j][cb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i], bf, acc[i + j][cb], 0, 0, 0);
+        }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int st = 0;
+  for (; st + PA <= nk; st += PA)
+#pragma unroll
+    for (int h = 0; h < PA; ++h) step(st + h, va[h]);
+#pragma unroll
+  for (int h = 0; h < PA - 1; ++h)
+    if (st + h < nk) step(st + h, va[h]);
+  // lane l holds column 16 cb + l % 16, rows 4 (l / 16) + e of the wave's 16 rows
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) {
+    const int n = n0 + 16 * cb + r16;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int m = m0 + 4 * ch + e;
+      int64_t v = 0;
+#pragma unroll
+      for (int s = 0; s < 5; ++s) v += (int64_t)acc[s][cb][e] << (8 * s);
+      if (m < M && n < N) c[z * scz + (int64_t)m * scm + (int64_t)n * scn] = v;
+    }
+  }
+}
+
+template <int CB, int NW, int PA>
+static void launch_rows(bool bv, hipStream_t st, const int32_t* a, int64_t saz, int64_t sam, const int32_t* b, int64_t sbz,
+                        int64_t sbk, int64_t sbn, int64_t* c, int64_t scz, int64_t scm, int64_t scn, int Z, int M, int N,
+                        int K) {
+  const dim3 grid((N + 16 * CB - 1) / (16 * CB), (M + 16 * NW - 1) / (16 * NW), Z);
+  auto k = K % kBT ? (bv ? bmm_rows_kernel<CB, NW, PA, true, true> : bmm_rows_kernel<CB, NW, PA, false, true>)
+                   : (bv ? bmm_rows_kernel<CB, NW, PA, true, false> : bmm_rows_kernel<CB, NW, PA, false, false>);
+  k<<<grid, 64 * NW, 0, st>>>(a, saz, sam, b, sbz, sbk, sbn, c, scz, scm, scn, M, N, K);
+}
+
 template <typename TA, typename TB, int NA, bool A1, int RT, int PF>
 static void launch_nb(int nb, dim3 grid, hipStream_t st, const TA* a, int64_t saz, int64_t sam, int64_t sak,
                       const TB* b, int64_t sbz, int64_t sbk, int64_t sbn, int64_t* c, int64_t scz, int64_t scm,
@@ -239,6 +380,23 @@ extern "C" int bx_limb_bmm(const void* a, int32_t a_bytes, int64_t saz, int64_t 
     bmm_mfma_kernel<int32_t, int32_t, 1, 1, false, 1, 1><<<grid, 256, 0, st>>>((const int32_t*)a, saz, sam, sak, (const int32_t*)b,
                                                                   sbz, sbk, sbn, c, scz, scm, scn, M, N, 0, nti);
     return check_launch("bmm_mfma_kernel");
+  }
+  // The rows kernel (32-bit offsets within a block's rows of a and within one matrix of b). At K = 64 its blocks split
+  // a again for each column tile, which bmm_mfma_kernel's walk over 16 tiles does once: that stays where the walk still
+  // fills the chip (16 x 4096 rows by 1024 columns, 512 blocks: 133 us, rows 158; 32 x 1024 rows, 256 blocks: 74 and
+  // 73; 8 x 128 rows by 4096, 32 blocks: 46 and 12). 128-column blocks of 128 rows read a once where there is one a CU
+  // (N = 128: 16 x 4096 rows, 512 blocks, 111 us, 64 x 64 blocks 157; 8 x 2048 rows, 128 blocks: 77 and 60).
+  const int64_t aspan = 127 * sam * 4 + (int64_t)K * 4, bspan = ((N - 1) * sbn + (K - 1) * sbk) * 4, yb = (M + 127) / 128;
+  if (a_bytes == 4 && b_bytes == 4 && na == 3 && nb == 3 && K >= kBT && sak == 1 && aspan < kBufRange - 16 &&
+      bspan < kBufRange - 16 &&
+      (K > kBT || Z * yb * ((N + 1023) / 1024) < device_cus())) {
+    const bool bv = sbk == 1;
+    const int32_t *a4 = (const int32_t*)a, *b4 = (const int32_t*)b;
+    if (M > 64 && N > 64 && Z * yb * ((N + 127) / 128) >= device_cus())
+      launch_rows<8, 8, 1>(bv, st, a4, saz, sam, b4, sbz, sbk, sbn, c, scz, scm, scn, Z, M, N, K);
+    else
+      launch_rows<4, 4, 2>(bv, st, a4, saz, sam, b4, sbz, sbk, sbn, c, scz, scm, scn, Z, M, N, K);
+    return check_launch("bmm_rows_kernel");
   }
   if (a_bytes == 4 && b_bytes == 4)
     launch_k<int32_t, int32_t>(na, nb, grid, st, a, saz, sam, sak, b, sbz, sbk, sbn, c, scz, scm, scn, M, N, K, nti);

@@ -354,6 +354,28 @@ def test_bmm_exact(dev):
         assert np.array_equal(bmm(at, b.to(dev)).cpu().numpy(), R.bmm(a.numpy(), b.numpy()))
 
 
+@pytest.mark.parametrize("Z,M,K,N", [(1, 1, 64, 1), (3, 17, 193, 40), (2, 65, 127, 65), (5, 130, 321, 200),
+                                     (40, 400, 64, 300), (64, 257, 128, 130), (33, 1030, 67, 70), (64, 130, 255, 140)])
+def test_bmm_rows(dev, Z, M, K, N):
+    """bmm where a's rows are contiguous (also at 4-byte alignment, inside a wider tensor) against rows that are not,
+    b contiguous along n and along k, whole and part-filled last k steps, row and column tiles, the largest
+    magnitudes."""
+    from bitexact.bmm import bmm
+    from bitexact.exact.consts import LIM3
+    g = torch.Generator().manual_seed(Z + M + K + N)
+    a = torch.randint(-LIM3, LIM3 + 1, (Z, M, K), generator=g, dtype=torch.int32)
+    b = torch.randint(-LIM3, LIM3 + 1, (Z, K, N), generator=g, dtype=torch.int32)
+    a[:, -1], b[:, :, -1] = LIM3, -LIM3
+    ref = R.bmm(a.numpy(), b.numpy())
+    wide = torch.full((Z, M, K + 5), LIM3, dtype=torch.int32)
+    wide[:, :, 1:K + 1] = a
+    bk = b.transpose(1, 2).contiguous().to(dev).transpose(1, 2)
+    at = a.transpose(1, 2).contiguous().to(dev).transpose(1, 2)
+    for x in (a.to(dev), wide.to(dev)[:, :, 1:K + 1], at):
+        for y in (b.to(dev), bk):
+            assert np.array_equal(bmm(x, y).cpu().numpy(), ref)
+
+
 def test_bmm_int32_bound(dev):
     """The int32 limb-weight sums at the reference's bound (K < 43690): every limb -128, the largest K, and a
     mixed-sign case, against Python-int products."""
