@@ -1678,25 +1678,30 @@ __global__ __launch_bounds__(256) void pre_split_kernel(AttnArgs p, int8_t* kp, 
 // attn_pre2_kernel then runs a (tile, KV head) per block. One wave per table row s counts the tokens of smaller rows
 // (its start in perm) and its own, then writes them in order. Tile slots [start / TT + s, (start + count) / TT + s + 1)
 // belong to sequence s: at least ceil(count / TT) of them, never two sequences' (the spare ones hold 0 tokens).
+// Tokens whose row is not in the table (padding) form a last sequence, s = nrow, that sees no key: their outputs are
+// 0, and every slot and every entry of perm is written whatever rmap holds.
 struct RowMap {
   const int32_t* perm;      // [R] token rows, sorted
-  const int4* slots;        // [nslot] (start in perm, tokens, table row, 0)
-  const int32_t* klen;      // [nrow] keys of each sequence visible to some token
-  int64_t sqpos;
-  int nslot, M, hkv;
+  const int4* slots;        // [nslot] (start in perm, tokens, table row or nrow, 0)
+  int nslot, nrow, M, hkv;
 };
+__device__ __forceinline__ int64_t row_of(const int64_t* rmap, int i, int R, int nrow) {   // past the step: nrow + 1
+  if (i >= R) return nrow + 1;
+  const int64_t r = rmap[i];
+  return r >= 0 && r < nrow ? r : nrow;
+}
 
 __global__ __launch_bounds__(256) void rows_group_kernel(const int64_t* rmap, const int64_t* qpos, int64_t sqpos, int R,
                                                          int M, int nrow, int S, int TT, int nslot, int32_t* perm,
                                                          int4* slots, int32_t* klen) {
   const int s = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (s >= nrow) return;
+  if (s > nrow) return;
   constexpr int U = 8;
   int lt = 0, eq = 0;
   for (int i0 = 0; i0 < R; i0 += 64 * U) {
     int64_t r[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) r[u] = i0 + u * 64 + lane < R ? rmap[i0 + u * 64 + lane] : nrow;
+    for (int u = 0; u < U; ++u) r[u] = row_of(rmap, i0 + u * 64 + lane, R, nrow);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       lt += __popcll(__builtin_amdgcn_ballot_w64(r[u] < s));
@@ -1708,25 +1713,25 @@ __global__ __launch_bounds__(256) void rows_group_kernel(const int64_t* rmap, co
   for (int i0 = 0; eq > 0 && i0 < R; i0 += 64 * U) {
     int64_t r[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) r[u] = i0 + u * 64 + lane < R ? rmap[i0 + u * 64 + lane] : nrow;
+    for (int u = 0; u < U; ++u) r[u] = row_of(rmap, i0 + u * 64 + lane, R, nrow);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint64_t m = __builtin_amdgcn_ballot_w64(r[u] == s);
       if (r[u] == s) {
         const int i = i0 + u * 64 + lane;
         perm[at + __popcll(m & ((1ULL << lane) - 1))] = i;
-        for (int j = 0; j < M; ++j) kmax = imax(kmax, qpos[i * sqpos + j]);
+        for (int j = 0; s < nrow && j < M; ++j) kmax = imax(kmax, qpos[i * sqpos + j]);
       }
       at += __popcll(m);
     }
   }
   kmax = wave_max64(kmax);
-  const int first = lt / TT + s, next = s + 1 < nrow ? (lt + eq) / TT + s + 1 : nslot;
+  const int first = lt / TT + s, next = s < nrow ? (lt + eq) / TT + s + 1 : nslot;
   for (int j = first + lane; j < next; j += 64) {
     const int o = (j - first) * TT;
     slots[j] = int4{lt + o, min(max(eq - o, 0), TT), s, 0};
   }
-  if (lane == 0) klen[s] = (int)imin(kmax + 1, S);
+  if (lane == 0 && s < nrow) klen[s] = (int)imin(kmax + 1, S);
 }
 
 // Block kTabBlocks + ((row HKV + h) ntile + tile): 64 keys of one (sequence, KV head). K rows are copied as they
@@ -1883,7 +1888,7 @@ __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArg
   // the lane's query (B operand rows) and its position / exponent
   int64_t qg;
   int qr;
-  const bool live = locate(16 * wr + kl, qg, qr);
+  const bool live = locate(16 * wr + kl, qg, qr), keys = !ROWS || slot.z < rm.nrow;   // keys: the query's row has some
   v4i qb[3][KK];
   {
     const int32_t* qp = p.q + qg * p.sq_tile + (int64_t)qr * p.sq_row;
@@ -1898,7 +1903,7 @@ __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArg
   }
   // (positions past S - 1 see every key: the caller's contract keeps qpos < S, so the clamp changes nothing)
   const int my_qpos =
-      live ? (int)imin(p.qpos[(qg / p.qpos_div) * p.qpos_tile + (int64_t)qr * p.qpos_row], (int64_t)p.S) : -1;
+      live && keys ? (int)imin(p.qpos[(qg / p.qpos_div) * p.qpos_tile + (int64_t)qr * p.qpos_row], (int64_t)p.S) : -1;
   const int64_t shift = live ? (int64_t)(kFK + 3 - kFZ) - p.sh[qg * p.sh_tile + qr] : 0;
   if (threadIdx.x == 0) s_kend = 0;
   __syncthreads();
@@ -2553,7 +2558,7 @@ struct RowsLayout {
 static RowsLayout rows_layout(int64_t R, int64_t nrow, int64_t HKV, int64_t M, int64_t HD, int64_t keys) {
   RowsLayout l;
   l.TT = (HD == 64 ? Pre2<64>::QR : Pre2<128>::QR) / (int)M;
-  l.nslot = (int)(R / l.TT + nrow);
+  l.nslot = (int)(R / l.TT + nrow + 1);
   l.Sp = (int)((keys + 63) / 64 * 64);
   auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
   l.slots = up(R * 4);
@@ -2607,10 +2612,10 @@ extern "C" int bx_exact_attn_paged_rows(const int32_t* q, const int64_t* sh, con
   p.num = num; p.den = den; p.snum_tile = (int64_t)M * HD; p.snum_row = HD; p.sden_tile = M;
   p.nsplit = 1;
   hipStream_t st = (hipStream_t)stream;
-  rows_group_kernel<<<(nrow + 3) / 4, 256, 0, st>>>(rmap, qpos, sqpos_r, R, M, nrow, p.S, l.TT, l.nslot, perm, slots, klen);
+  rows_group_kernel<<<(nrow + 4) / 4, 256, 0, st>>>(rmap, qpos, sqpos_r, R, M, nrow, p.S, l.TT, l.nslot, perm, slots, klen);
   if (int rc = check_launch("rows_group_kernel")) return rc;
   const int ntile = l.Sp / 64, Z = nrow * HKV;
-  const RowMap rm = {perm, slots, klen, sqpos_r, l.nslot, M, HKV};
+  const RowMap rm = {perm, slots, l.nslot, nrow, M, HKV};
   if (HD == 64) {
     paged_planes_kernel<64><<<kTabBlocks + Z * ntile, 256, 0, st>>>(p, klen, kp, vp, tab, l.Sp, ntile);
     if (int rc = check_launch("paged_planes_kernel")) return rc;

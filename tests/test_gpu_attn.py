@@ -265,6 +265,37 @@ def test_paged_rows_equal_decode_form(dev, HD, M, bs, order):
         assert torch.equal(n1, n2) and torch.equal(d1, d2)
 
 
+@pytest.mark.parametrize("HD,npad,pad", [(64, 1, -1), (64, 33, -1), (64, 300, -(1 << 40)), (128, 40, 3), (128, 200, 1 << 40),
+                                         (64, 513, None)])
+def test_paged_rows_outside_the_table(dev, HD, npad, pad):
+    """Tokens whose rmap names no table row (negative, nrow, beyond; None: all of them mixed) in a step that takes the
+    grouped form: their num and den are 0 and the other tokens' are the per-token form's. The counts cover a tile's
+    edges (32 tokens of 4 queries at heads of 64, 16 at 128), and scratch holds another step's slots before the call."""
+    from bitexact import _hip
+    from bitexact.vllm_plugin import tri_exact_attn, tri_paged
+    g = torch.Generator().manual_seed(HD + npad)
+    HKV, M, bs, nrow, nblk = 4, 4, 16, 3, 12
+    c = torch.randint(-R.LIM3, R.LIM3 + 1, (nrow * nblk, HKV, bs, 2 * HD), generator=g).to(torch.int32)
+    cl = tri_paged.to_limbs(c.to(dev))
+    bt = torch.randperm(nrow * nblk, generator=g).to(torch.int32).view(nrow, nblk).to(dev)
+    Rr = 400 + npad
+    live = torch.ones(Rr, dtype=torch.bool)
+    live[torch.randperm(Rr, generator=g)[:npad]] = False
+    rmap = torch.randint(0, nrow, (Rr,), generator=g)
+    qpos = torch.randint(-1, nblk * bs, (Rr, M), generator=g)
+    q = torch.randint(-(1 << 22), (1 << 22) + 1, (Rr, HKV, M, HD), generator=g).to(torch.int32).to(dev)
+    sh = torch.randint(-46, -36, (Rr, HKV, M), generator=g).to(dev)
+    args = lambda r, p: (q, sh, p.to(dev), cl, bt, r.to(dev), _lut(dev), R.L2E28_HD[HD])
+    n1, d1 = tri_exact_attn.attend(*args(rmap, torch.where(live[:, None], qpos, -1)), nsplit=1)
+    outside = torch.tensor([-1, nrow, 1 << 40, -(1 << 40), (1 << 32) + 1])
+    fill = torch.full((Rr,), pad) if pad is not None else outside[torch.randint(0, len(outside), (Rr,), generator=g)]
+    need = tri_exact_attn.rows_scratch(Rr, HKV, M, HD, nrow, nblk * bs)
+    assert need > 0
+    _hip.scratch(dev, need)[0].fill_(1)
+    n2, d2 = tri_exact_attn.attend(*args(torch.where(live, rmap, fill), qpos))
+    assert torch.equal(n1, n2) and torch.equal(d1, d2)
+
+
 @pytest.mark.parametrize("HD", [64, 128])
 @pytest.mark.parametrize("table", ["exp2", "noisy", "steps"])
 def test_prefill_weight_positions(dev, HD, table):
