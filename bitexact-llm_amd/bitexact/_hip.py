@@ -24,6 +24,7 @@ P, I32, I64 = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64
 SIGNATURES = {
     "bx_version": (ctypes.c_int, []),
     "bx_last_error": (ctypes.c_char_p, []),
+    "bx_capture_id": (I64, [P]),
     "bx_exact_linear": (ctypes.c_int, [P, I64, P, P, I64, I64, P, P, P, P, P, I32, P, I32, I32, I32, I32, I32, P,
                                        P, I64, P, I64, P]),
     "bx_exact_linear_planes": (ctypes.c_int, [P, I64, P, P, I64, I64, P, P, P, P, P, I32, P, I32, I32, I32, I32,
@@ -167,26 +168,62 @@ def require_cuda(*ts):
             raise AssertionError("bitexact HIP kernels take device tensors only (no CPU path)")
 
 
-# ---- per (device, stream) buffers: the split-K workspace (zero-filled; every call leaves it zeroed) and a
-# scratch buffer (no contents kept between calls) ----
-_ws = {}
+# ---- buffers of the calls on one (device, stream) ----
+# A captured graph keeps the addresses its calls were given, so an address that a capture may have seen is never given
+# back to the allocator while the graph could still be replayed:
+# - the split-K workspace (zero-filled; every call leaves it zeroed) at least doubles when it grows and the buffers it
+#   outgrew stay alive (together less than the current one). A capture that needs more than the stream's workspace
+#   holds takes one from its own graph's memory, whose fill is recorded with it; no other capture and no eager call
+#   uses that one, since it holds zeros only while its graph runs.
+# - scratch (no contents kept between calls) is one buffer of SCRATCH_KEPT bytes that is never replaced; a call that
+#   needs more allocates for itself, so large scratch goes back to the allocator (under capture: to the graph's memory)
+#   when the call returns.
+SCRATCH_KEPT = 8 << 20
+_ws, _ws_outgrown, _ws_graph, _tmp = {}, [], {}, {}
 
 
-def _buffer(kind, dev, nbytes):
-    if nbytes <= 0:
-        return None, 0
+def _stream_key(dev):
     i = dev.index
-    key = (kind, i, torch.cuda.current_stream(dev).cuda_stream if _raw_stream is None or i is None else _raw_stream(i))
-    buf = _ws.get(key)
-    if buf is None or buf.numel() < nbytes:
-        buf = (torch.zeros if kind == "ws" else torch.empty)(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
-        _ws[key] = buf
-    return buf, buf.numel()
+    return i, torch.cuda.current_stream(dev).cuda_stream if _raw_stream is None or i is None else _raw_stream(i)
+
+
+def _grow_workspace(dev, key, nbytes):
+    capture = lib().bx_capture_id(key[1])
+    if capture:
+        owner, buf = _ws_graph.get(key, (0, None))
+        if owner != capture or buf.numel() < nbytes:
+            buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
+            _ws_graph[key] = capture, buf
+        return buf
+    with _lock:
+        buf = _ws.get(key)
+        if buf is None or buf.numel() < nbytes:
+            _ws_graph.pop(key, None)
+            size = max(nbytes, 1 << 20)
+            if buf is not None:
+                _ws_outgrown.append(buf)
+                size = max(size, 2 * buf.numel())
+            buf = _ws[key] = torch.zeros(size, dtype=torch.uint8, device=dev)
+        return buf
 
 
 def workspace(dev, nbytes):
-    return _buffer("ws", dev, nbytes)
+    if nbytes <= 0:
+        return None, 0
+    key = _stream_key(dev)
+    buf = _ws.get(key)
+    if buf is None or buf.numel() < nbytes:
+        buf = _grow_workspace(dev, key, nbytes)
+    return buf, buf.numel()
 
 
 def scratch(dev, nbytes):
-    return _buffer("tmp", dev, nbytes)
+    if nbytes <= 0:
+        return None, 0
+    if nbytes > SCRATCH_KEPT:
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev), nbytes
+    key = _stream_key(dev)
+    buf = _tmp.get(key)
+    if buf is None:
+        buf = _tmp.setdefault(key, torch.empty(SCRATCH_KEPT, dtype=torch.uint8, device=dev))
+    return buf, SCRATCH_KEPT

@@ -40,3 +40,13 @@ int device_cus() {
 
 extern "C" const char* bx_last_error(void) { return bx::g_err; }
 extern "C" int bx_version(void) { return 1; }
+
+extern "C" int64_t bx_capture_id(bx_stream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo((hipStream_t)stream, &status, &id) != hipSuccess) {
+    (void)hipGetLastError();                         // (a launch check after this call sees its own errors only)
+    return 0;
+  }
+  return status == hipStreamCaptureStatusActive ? (int64_t)id : 0;
+}

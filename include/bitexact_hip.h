@@ -35,6 +35,11 @@ typedef struct ihipStream_t* bx_stream_t; /* hipStream_t */
 const char* bx_last_error(void);
 int bx_version(void);
 
+/* The id of the graph capture that `stream` is part of, 0 when it is not being captured (for a caller's buffers: a
+ * captured call's must stay valid while its graph is replayed, and a workspace zero-filled inside a capture holds
+ * zeros only when that graph runs). No reference counterpart. */
+int64_t bx_capture_id(bx_stream_t stream);
+
 /* ---- exact mode linear ---- */
 
 /* Replaces FusedLin.__call__ (src/bitexact/vllm_plugin/exact_gemm.py:284-316) and
