@@ -40,18 +40,20 @@ SCORES_MAX = 1 << 28        # bytes of kept scores at most
 
 @functools.lru_cache(4096)
 def auto_nsplit(T, keys, HD):
-    """(nsplit, kept-scores scratch bytes or 0) of T query tiles over `keys` keys. The exchange and one-block forms
-    read K once while a split has at most 512 keys or a tile at most 2048; past that they would read it twice, and two
-    launches that keep the scores in between (two blocks per CU) are faster: 16 x 8 tiles of 4096 keys 74 against 134
-    us (heads of 128: 113 / 203), 8 x 8 of 4096 45 / 52 (67 / 73). Of the one-block range only half a chip of tiles
-    over wide rows gains (16 x 8 tiles, 2048 keys, heads of 128: 66 / 75; of 64: 45 / 47)."""
+    """(nsplit, kept-scores scratch bytes or 0) of T query tiles over a table of `keys` keys. The exchange and one-block
+    forms read K once while a split has at most 512 keys or a tile at most 2048; past that they would read it twice, and
+    two launches that keep the scores in between, with three splits a tile or more in two blocks per CU (T <= 170), are
+    faster: 128 tiles of 4096 keys 62 against 114 us (heads of 128: 103 / 197), 168 tiles 83 / 118 (144 / 210), 64 tiles
+    39 / 44 (57 / 64). With two splits they are not worth their scratch: 256 tiles 123 / 143 at 4096 keys but 18 / 12 at
+    256, 512 tiles 276 / 248. The contexts are known on the device only: in a table past 2048 keys the two launches cost
+    short ones up to 4 us (128 tiles 11.7 / 8.6 at 128 keys, 14.6 / 11.9 at 256, 18.0 / 17.9 at 512) and gain from
+    512 keys on (22 / 27 at 768; int8 mode and 64 tiles: from 768 to 1024 on)."""
     ns = tile_nsplit(T, keys)
     twice = -(-(-(-keys // ns)) // 64) * 64 > 512 if ns > 1 else keys > 2048
-    if (twice and T >= 64) or (128 <= T < 192 and 2048 * 128 <= keys * HD and keys <= 2048):
+    if twice and T >= 64 and 512 // T >= 3:
         need = _hip.lib().bx_attn_paged_scores_scratch(T, 1, 4, keys)
-        split = min(max(2, 512 // T), max(1, min(64, 4096 // T)))
-        if need <= SCORES_MAX and split > 1:
-            return split, need
+        if need <= SCORES_MAX:
+            return 512 // T, need
     return ns, 0
 
 

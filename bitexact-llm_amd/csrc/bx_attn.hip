@@ -160,6 +160,7 @@ struct AttnArgs {
   int64_t* den_ws;                // [groups, nq]
   int32_t* sem;                   // [groups]
   int64_t* raw;                   // split launches that keep the scores (null: K read in both)
+  int one_keys;                   // there: a tile with at most this many keys is one block's
   uint64_t exch_ticks;            // attn_dec_exch_kernel: longest wait for the other splits' maxima (100 MHz ticks)
 };
 
@@ -742,14 +743,18 @@ __device__ __forceinline__ void dec_finish_ao(const AttnArgs& p, const AoArgs& a
 }
 
 // RAW (split launches): phase 0 writes every score to p.raw ([tile][key][query] int64, p.S keys a tile) and phase 1
-// reads them back, 32 bytes a key instead of K's 192 again. With enough splits for four blocks a CU in both launches
+// reads them back, 32 bytes a key instead of K's 3 HD again. With splits for about two blocks a CU in both launches
 // this is the form of long contexts and of grids that neither fill the chip unsplit nor fit the exchange kernel.
+// The host chooses it by the table's width; a tile whose context is short (p.one_keys) is one block's in phase 1, as
+// the exchange between the phases costs more than its keys: 128 tiles of 128 keys (heads of 64) 14.3 -> 11.7 us, of
+// 256 16.0 -> 14.6; at 384 both take 17.4, and heads of 128 cross at half the keys.
 template <int HD, int PHASE, bool RAW>
 __global__ __launch_bounds__(kDecWaves * 64) void attn_dec_kernel(AttnArgs p) {
   __shared__ DecSmem<HD> sm;
   constexpr int KK = HD / 64;
   const int tiles = (p.nq + 3) / 4;
-  const int tile = blockIdx.x, T = gridDim.x, sp = blockIdx.y, NS = gridDim.y;
+  const int tile = blockIdx.x, T = gridDim.x, sp = blockIdx.y;
+  int NS = gridDim.y;
   int64_t* raws = RAW ? p.raw + (int64_t)tile * p.S * 4 : nullptr;
   const int group = tile / tiles, q0 = (tile % tiles) * 4;
   const int nvalid = min(4, p.nq - q0);
@@ -771,7 +776,13 @@ __global__ __launch_bounds__(kDecWaves * 64) void attn_dec_kernel(AttnArgs p) {
   __syncthreads();
   int64_t kend = 0;
   for (int i = 0; i < 4; ++i) kend = imax(kend, sm.qpos[i] + 1);
-  if (RAW) kend = imin(kend, p.S);                 // (qpos < the block table's keys: the scores' bound in any case)
+  if (RAW) {
+    kend = imin(kend, p.S);                        // (qpos < the block table's keys: the scores' bound in any case)
+    if (kend <= p.one_keys) {                      // block-uniform: phase 1's split 0 alone, both sweeps
+      if (PHASE == 0 || sp > 0) return;
+      NS = 1;
+    }
+  }
   int64_t lo64, hi64;
   split_range(kend, NS, sp, lo64, hi64);
   const int lo = (int)lo64, hi = (int)hi64;
@@ -2231,6 +2242,7 @@ static int launch_attn(AttnArgs& p, int groups, hipStream_t st) {
 }
 
 constexpr int kDecRawKeys = 2048;               // single-launch score cache: 4 x 2048 x 8 B of LDS
+constexpr int kDecOneKeys = 256 * 64;           // kept scores: keys x head_dim of a tile that is one block's
 
 template <int HD>
 static int launch_dec(AttnArgs& p, int groups, int64_t max_keys, hipStream_t st) {
@@ -2247,6 +2259,7 @@ static int launch_dec(AttnArgs& p, int groups, int64_t max_keys, hipStream_t st)
   }
   if (p.raw != nullptr) {
     p.S = (int)max_keys;
+    p.one_keys = kDecOneKeys / HD;
     attn_dec_kernel<HD, 0, true><<<grid, kDecWaves * 64, 0, st>>>(p);
     if (int rc = check_launch("attn_dec_kernel(scores)")) return rc;
     attn_dec_kernel<HD, 1, true><<<grid, kDecWaves * 64, 0, st>>>(p);

@@ -196,11 +196,12 @@ def test_prefill_attention_full_size(dev, HD, T, Z):
 
 
 @pytest.mark.parametrize("mode", ["exact", "int8"])
-@pytest.mark.parametrize("HD,Rr,M,keys", [(64, 16, 4, 2064), (64, 8, 3, 4096), (128, 16, 1, 2048), (128, 9, 4, 4112)])
+@pytest.mark.parametrize("HD,Rr,M,keys", [(64, 16, 4, 2064), (64, 8, 3, 4096), (128, 16, 1, 2064), (128, 9, 4, 4112),
+                                            (64, 21, 2, 3072)])
 def test_paged_kept_scores(dev, mode, HD, Rr, M, keys):
     """Long contexts keep the scores between their two launches (attend chooses that by size): equal to the one-launch
     or K-twice forms on every row, with contexts that end anywhere in the table (one key, a split's first and last
-    key, none), and repeated (the workspace is left zero)."""
+    key, none, the longest that one block takes alone and one more), and repeated (the workspace is left zero)."""
     from bitexact.int8.consts import exp_table
     from bitexact.vllm_plugin import tri_exact_attn, tri_paged
     g = torch.Generator().manual_seed(keys)
@@ -213,8 +214,9 @@ def test_paged_kept_scores(dev, mode, HD, Rr, M, keys):
     cl = tri_paged.to_limbs(torch.randint(-lim, lim + 1, (Rr * nblk, HKV, bs, 2 * HD), generator=g).to(torch.int32).to(dev))
     bt = torch.randperm(Rr * nblk, generator=g).to(torch.int32).view(Rr, nblk).to(dev)
     qpos = torch.full((Rr, M), keys - 1)
-    ends = [0, 1, 63, 64, keys // split - 1, keys // split, keys - 2, -1]
-    for i, e in enumerate(ends):
+    one = 256 * 64 // HD
+    ends = [0, 1, 63, 64, keys // split - 1, keys // split, keys - 2, -1, one - 1, one, one - 17]
+    for i, e in enumerate(ends[:Rr]):
         qpos[i] = e
     qpos[3, 0] = 700
     qpos = qpos.to(dev)
