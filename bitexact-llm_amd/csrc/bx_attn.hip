@@ -1686,7 +1686,7 @@ __global__ __launch_bounds__(256) void pre_split_kernel(AttnArgs p, int8_t* kp, 
 // ---- the same attention over the paged cache, for steps of many tokens per sequence ----
 // rows_group_kernel sorts the step's token rows by their block-table row (stable) and cuts each sequence's into
 // tiles of TT tokens; paged_planes_kernel writes the sequences' cached K and V limbs as the planes above;
-// attn_pre2_kernel then runs a (tile, KV head) per block. One wave per table row s counts the tokens of smaller rows
+// attn_pre2_kernel then runs a (tile, KV head) per block. One block per table row s counts the tokens of smaller rows
 // (its start in perm) and its own, then writes them in order. Tile slots [start / TT + s, (start + count) / TT + s + 1)
 // belong to sequence s: at least ceil(count / TT) of them, never two sequences' (the spare ones hold 0 tokens).
 // Tokens whose row is not in the table (padding) form a last sequence, s = nrow, that sees no key: their outputs are
@@ -1696,53 +1696,69 @@ struct RowMap {
   const int4* slots;        // [nslot] (start in perm, tokens, table row or nrow, 0)
   int nslot, nrow, M, hkv;
 };
-__device__ __forceinline__ int64_t row_of(const int64_t* rmap, int i, int R, int nrow) {   // past the step: nrow + 1
-  if (i >= R) return nrow + 1;
-  const int64_t r = rmap[i];
-  return r >= 0 && r < nrow ? r : nrow;
-}
 
+// Each wave takes a quarter of the token rows, kRowU loads in flight: bound by their latency (R = 4096: two round trips;
+// 8 sequences of 512 tokens: 9.4 us; one wave a sequence with 8 in flight took 17).
+constexpr int kRowU = 16;
+__device__ __forceinline__ void rows_load(const int64_t* rmap, int i0, int i1, int nrow, int (&r)[kRowU]) {
+  int64_t v[kRowU];
+#pragma unroll
+  for (int u = 0; u < kRowU; ++u) v[u] = rmap[min(i0 + u * 64, i1 - 1)];
+#pragma unroll
+  for (int u = 0; u < kRowU; ++u)        // past the wave's part: no sequence's
+    r[u] = i0 + u * 64 >= i1 ? nrow + 1 : v[u] >= 0 && v[u] < nrow ? (int)v[u] : nrow;
+}
 __global__ __launch_bounds__(256) void rows_group_kernel(const int64_t* rmap, const int64_t* qpos, int64_t sqpos, int R,
                                                          int M, int nrow, int S, int TT, int nslot, int32_t* perm,
                                                          int4* slots, int32_t* klen) {
-  const int s = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (s > nrow) return;
-  constexpr int U = 8;
+  __shared__ int s_lt[4], s_eq[4];
+  __shared__ int64_t s_kmax[4];
+  const int s = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int i0 = (int)((int64_t)R * w / 4), i1 = (int)((int64_t)R * (w + 1) / 4);
   int lt = 0, eq = 0;
-  for (int i0 = 0; i0 < R; i0 += 64 * U) {
-    int64_t r[U];
+  for (int i = i0; i < i1; i += 64 * kRowU) {
+    int r[kRowU];
+    rows_load(rmap, i + lane, i1, nrow, r);
 #pragma unroll
-    for (int u = 0; u < U; ++u) r[u] = row_of(rmap, i0 + u * 64 + lane, R, nrow);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < kRowU; ++u) {
       lt += __popcll(__builtin_amdgcn_ballot_w64(r[u] < s));
       eq += __popcll(__builtin_amdgcn_ballot_w64(r[u] == s));
     }
   }
+  if (lane == 0) {
+    s_lt[w] = lt;
+    s_eq[w] = eq;
+  }
+  __syncthreads();
+  lt = s_lt[0] + s_lt[1] + s_lt[2] + s_lt[3];
   int at = lt;
+  for (int u = 0; u < w; ++u) at += s_eq[u];
   int64_t kmax = -1;
-  for (int i0 = 0; eq > 0 && i0 < R; i0 += 64 * U) {
-    int64_t r[U];
+  for (int i = i0; eq > 0 && i < i1; i += 64 * kRowU) {
+    int r[kRowU];
+    rows_load(rmap, i + lane, i1, nrow, r);
 #pragma unroll
-    for (int u = 0; u < U; ++u) r[u] = row_of(rmap, i0 + u * 64 + lane, R, nrow);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
+    for (int u = 0; u < kRowU; ++u) {
       const uint64_t m = __builtin_amdgcn_ballot_w64(r[u] == s);
       if (r[u] == s) {
-        const int i = i0 + u * 64 + lane;
-        perm[at + __popcll(m & ((1ULL << lane) - 1))] = i;
-        for (int j = 0; s < nrow && j < M; ++j) kmax = imax(kmax, qpos[i * sqpos + j]);
+        const int64_t row = i + u * 64 + lane;
+        perm[at + __popcll(m & ((1ULL << lane) - 1))] = (int)row;
+        for (int j = 0; s < nrow && j < M; ++j) kmax = imax(kmax, qpos[row * sqpos + j]);
       }
       at += __popcll(m);
     }
   }
   kmax = wave_max64(kmax);
+  if (lane == 0) s_kmax[w] = kmax;
+  __syncthreads();
+  kmax = imax(imax(s_kmax[0], s_kmax[1]), imax(s_kmax[2], s_kmax[3]));
+  eq = s_eq[0] + s_eq[1] + s_eq[2] + s_eq[3];
   const int first = lt / TT + s, next = s < nrow ? (lt + eq) / TT + s + 1 : nslot;
-  for (int j = first + lane; j < next; j += 64) {
+  for (int j = first + threadIdx.x; j < next; j += 256) {
     const int o = (j - first) * TT;
     slots[j] = int4{lt + o, min(max(eq - o, 0), TT), s, 0};
   }
-  if (lane == 0 && s < nrow) klen[s] = (int)imin(kmax + 1, S);
+  if (threadIdx.x == 0 && s < nrow) klen[s] = (int)imin(kmax + 1, S);
 }
 
 // Block kTabBlocks + ((row HKV + h) ntile + tile): 64 keys of one (sequence, KV head). K rows are copied as they
@@ -2625,7 +2641,7 @@ extern "C" int bx_exact_attn_paged_rows(const int32_t* q, const int64_t* sh, con
   p.num = num; p.den = den; p.snum_tile = (int64_t)M * HD; p.snum_row = HD; p.sden_tile = M;
   p.nsplit = 1;
   hipStream_t st = (hipStream_t)stream;
-  rows_group_kernel<<<(nrow + 4) / 4, 256, 0, st>>>(rmap, qpos, sqpos_r, R, M, nrow, p.S, l.TT, l.nslot, perm, slots, klen);
+  rows_group_kernel<<<nrow + 1, 256, 0, st>>>(rmap, qpos, sqpos_r, R, M, nrow, p.S, l.TT, l.nslot, perm, slots, klen);
   if (int rc = check_launch("rows_group_kernel")) return rc;
   const int ntile = l.Sp / 64, Z = nrow * HKV;
   const RowMap rm = {perm, slots, l.nslot, nrow, M, HKV};
