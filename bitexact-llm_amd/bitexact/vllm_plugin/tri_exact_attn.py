@@ -57,18 +57,19 @@ def auto_nsplit(T, keys, HD):
     return ns, 0
 
 
-# The grouped form for at least ROWS_MIN (token, KV head, dim)s and ROWS_PER_SEQ tokens per block-table row. Measured (8
-# KV heads of 64, grouped against per-token, us): 8 sequences of 512 181 / 1116, of 32 27 / 45, of 32 past 1000 keys 119
-# / 178, one of 256 41 / 56; below the line it loses: 8 of 16 26 / 23, one of 64 past 2000 keys 196 / 88 (two tiles per
-# head: 16 blocks). Heads of 128 cross at half the tokens (8 of 16 25 / 30).
-ROWS_PER_SEQ, ROWS_MIN = 8, 96 * 1024
+# The grouped form for at least ROWS_MIN (token, KV head)s and ROWS_PER_SEQ tokens per block-table row. Measured (8 KV
+# heads of 64, grouped against per-token, us): 8 sequences of 512 172 / 1128, of 32 29 / 43, of 24 28 / 32, of 32 past
+# 4000 keys 388 / 589, one of 192 37 / 38; a chunk of 192 with 3 decoding past 4096 keys 64 / 130 (with 15 past 512 it
+# loses, 56 / 40). Below the line it loses: 8 of 16 26 / 22, one of 128 32 / 25, one of 64 past 2000 keys 186 / 74 (two
+# tiles per head: 16 blocks). Heads of 128: one of 128 tokens 33 / 34, 8 of 16 32 / 29, 8 of 24 32 / 43.
+ROWS_PER_SEQ, ROWS_MIN = 8, {64: 1536, 128: 1152}
 
 
 def rows_scratch(R, HKV, M, HD, nrow, keys):
     """Scratch bytes of the grouped form (bx_exact_attn_paged_rows) where attend takes it, else 0: prefill steps (the
     table's row count bounds the sequences, the tokens' own rows being known on the device only) of enough tokens for
     its tiles to fill the chip, whose sequences' limb planes fit that form's 1 GiB."""
-    if R * HKV * HD < ROWS_MIN or R < ROWS_PER_SEQ * nrow:
+    if R * HKV < ROWS_MIN.get(HD, 0) or R < ROWS_PER_SEQ * nrow:
         return 0
     return _hip.lib().bx_attn_paged_rows_scratch(R, nrow, HKV, M, HD, keys)
 

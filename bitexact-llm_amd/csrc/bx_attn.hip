@@ -161,6 +161,7 @@ struct AttnArgs {
   int32_t* sem;                   // [groups]
   int64_t* raw;                   // split launches that keep the scores (null: K read in both)
   int one_keys;                   // there: a tile with at most this many keys is one block's
+  const int32_t* list;            // attn_dec_kernel's LIST form: count, then token rows
   uint64_t exch_ticks;            // attn_dec_exch_kernel: longest wait for the other splits' maxima (100 MHz ticks)
 };
 
@@ -748,21 +749,33 @@ __device__ __forceinline__ void dec_finish_ao(const AttnArgs& p, const AoArgs& a
 // The host chooses it by the table's width; a tile whose context is short (p.one_keys) is one block's in phase 1, as
 // the exchange between the phases costs more than its keys: 128 tiles of 128 keys (heads of 64) 14.3 -> 11.7 us, of
 // 256 16.0 -> 14.6; at 384 both take 17.4, and heads of 128 cross at half the keys.
-template <int HD, int PHASE, bool RAW>
+// LIST: the token rows of p.list, whose number only the device knows: block b takes tile b % T of T and split b / T, with
+// as many splits as make kDecListBlocks blocks (at least 128 keys of the table each); one split: phase 1 alone.
+constexpr int kDecListBlocks = 512;
+template <int HD, int PHASE, bool RAW, bool LIST = false>
 __global__ __launch_bounds__(kDecWaves * 64) void attn_dec_kernel(AttnArgs p) {
   __shared__ DecSmem<HD> sm;
   constexpr int KK = HD / 64;
   const int tiles = (p.nq + 3) / 4;
-  const int tile = blockIdx.x, T = gridDim.x, sp = blockIdx.y;
-  int NS = gridDim.y;
+  int tile = blockIdx.x, T = gridDim.x, sp = blockIdx.y, NS = gridDim.y;
+  if constexpr (LIST) {
+    T = p.list[0] * p.hkv;
+    if (T == 0) return;
+    NS = max(min(min(kDecListBlocks / T, kDecMaxSplit), p.S / 128), 1);
+    sp = tile / T;
+    tile -= sp * T;
+    if (sp >= NS || (PHASE == 0 && NS == 1)) return;         // block-uniform
+  }
   int64_t* raws = RAW ? p.raw + (int64_t)tile * p.S * 4 : nullptr;
-  const int group = tile / tiles, q0 = (tile % tiles) * 4;
+  const int group = LIST ? p.list[1 + tile / p.hkv] * p.hkv + tile % p.hkv : tile / tiles;
+  const int q0 = LIST ? 0 : (tile % tiles) * 4;
   const int nvalid = min(4, p.nq - q0);
   const int h = group % p.hkv;
   const int64_t brow = p.rmap ? p.rmap[group / p.hkv] : group / p.hkv;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int kl = lane & 15, qo = lane >> 4;
-  const DecWs ws = dec_ws(p, T, NS, HD);
+  DecWs ws = dec_ws(p, T, NS, HD);
+  if constexpr (LIST) ws.sem = p.sem;                // (a place that does not depend on T)
 
   if (threadIdx.x < 4) {
     const int i = threadIdx.x;
@@ -776,8 +789,8 @@ __global__ __launch_bounds__(kDecWaves * 64) void attn_dec_kernel(AttnArgs p) {
   __syncthreads();
   int64_t kend = 0;
   for (int i = 0; i < 4; ++i) kend = imax(kend, sm.qpos[i] + 1);
+  if (RAW || LIST) kend = imin(kend, p.S);         // (qpos < the block table's keys: the scores' bound in any case)
   if (RAW) {
-    kend = imin(kend, p.S);                        // (qpos < the block table's keys: the scores' bound in any case)
     if (kend <= p.one_keys) {                      // block-uniform: phase 1's split 0 alone, both sweeps
       if (PHASE == 0 || sp > 0) return;
       NS = 1;
@@ -1691,6 +1704,14 @@ __global__ __launch_bounds__(256) void pre_split_kernel(AttnArgs p, int8_t* kp, 
 // belong to sequence s: at least ceil(count / TT) of them, never two sequences' (the spare ones hold 0 tokens).
 // Tokens whose row is not in the table (padding) form a last sequence, s = nrow, that sees no key: their outputs are
 // 0, and every slot and every entry of perm is written whatever rmap holds.
+// A sequence of fewer than kFewTokens tokens (one that decodes beside another's prefill chunk) gets no tile and no
+// planes: laying out all its keys and a block over them cost more than its tokens. Its token rows go on a list that
+// attn_dec_kernel works off, scores kept (heads of 64, 8 KV heads; every sequence grouped / none / so): a chunk of 512
+// and 31 tokens past 4096 keys 465 / 258 / 200 us, 256 and 15 past 4096 313 / 147 / 103, 512 and 63 past 1024 276 / 197
+// / 124. The line: 32 sequences of 4 past 4096 433 grouped and 341 not, of 8 451 and 632; 8 sequences of 8 276 and
+// 157, of 12 283 and 244. Steps without such sequences pay for the empty list (8 of 32 tokens 23.8 -> 29.0, 8 of 512 the
+// same as before with the faster grouping).
+constexpr int kFewTokens = 8;
 struct RowMap {
   const int32_t* perm;      // [R] token rows, sorted
   const int4* slots;        // [nslot] (start in perm, tokens, table row or nrow, 0)
@@ -1710,14 +1731,14 @@ __device__ __forceinline__ void rows_load(const int64_t* rmap, int i0, int i1, i
 }
 __global__ __launch_bounds__(256) void rows_group_kernel(const int64_t* rmap, const int64_t* qpos, int64_t sqpos, int R,
                                                          int M, int nrow, int S, int TT, int nslot, int32_t* perm,
-                                                         int4* slots, int32_t* klen) {
+                                                         int4* slots, int32_t* klen, int2* few) {
   __shared__ int s_lt[4], s_eq[4];
   __shared__ int64_t s_kmax[4];
   const int s = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int i0 = (int)((int64_t)R * w / 4), i1 = (int)((int64_t)R * (w + 1) / 4);
-  int lt = 0, eq = 0;
+  const bool held = i1 - i0 <= 64 * kRowU;           // one pass over the part: its rows stay in registers
+  int lt = 0, eq = 0, r[kRowU];
   for (int i = i0; i < i1; i += 64 * kRowU) {
-    int r[kRowU];
     rows_load(rmap, i + lane, i1, nrow, r);
 #pragma unroll
     for (int u = 0; u < kRowU; ++u) {
@@ -1735,8 +1756,7 @@ __global__ __launch_bounds__(256) void rows_group_kernel(const int64_t* rmap, co
   for (int u = 0; u < w; ++u) at += s_eq[u];
   int64_t kmax = -1;
   for (int i = i0; eq > 0 && i < i1; i += 64 * kRowU) {
-    int r[kRowU];
-    rows_load(rmap, i + lane, i1, nrow, r);
+    if (!held) rows_load(rmap, i + lane, i1, nrow, r);
 #pragma unroll
     for (int u = 0; u < kRowU; ++u) {
       const uint64_t m = __builtin_amdgcn_ballot_w64(r[u] == s);
@@ -1754,24 +1774,63 @@ __global__ __launch_bounds__(256) void rows_group_kernel(const int64_t* rmap, co
   kmax = imax(imax(s_kmax[0], s_kmax[1]), imax(s_kmax[2], s_kmax[3]));
   eq = s_eq[0] + s_eq[1] + s_eq[2] + s_eq[3];
   const int first = lt / TT + s, next = s < nrow ? (lt + eq) / TT + s + 1 : nslot;
+  const bool is_few = s < nrow && eq < kFewTokens;
   for (int j = first + threadIdx.x; j < next; j += 256) {
     const int o = (j - first) * TT;
-    slots[j] = int4{lt + o, min(max(eq - o, 0), TT), s, 0};
+    slots[j] = int4{lt + o, is_few ? 0 : min(max(eq - o, 0), TT), s, 0};
   }
-  if (threadIdx.x == 0 && s < nrow) klen[s] = (int)imin(kmax + 1, S);
+  if (threadIdx.x == 0 && s < nrow) {
+    klen[s] = is_few ? 0 : (int)imin(kmax + 1, S);
+    few[s] = int2{lt, is_few ? eq : 0};
+  }
 }
 
-// Block kTabBlocks + ((row HKV + h) ntile + tile): 64 keys of one (sequence, KV head). K rows are copied as they
+// Block kTabBlocks of paged_planes_kernel: the token rows of the sequences with few tokens, in table order, after their
+// number, and their kernel's counters set to 0.
+__device__ void rows_list_block(const int32_t* perm, const int2* few, int nrow, int32_t* list, int32_t* sem) {
+  __shared__ int s_at;
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x == 0) s_at = 0;
+  for (int u = threadIdx.x; u < kDecListBlocks; u += 256) sem[u] = 0;
+  __syncthreads();
+  for (int s0 = 0; s0 < nrow; s0 += 256) {           // 256 sequences at a time, a lane each; waves in turn
+    const int s = s0 + threadIdx.x;
+    const int2 f = s < nrow ? few[s] : int2{0, 0};
+    int incl = f.y;                                  // counts up to this lane's
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    int base = 0;
+    for (int w = 0; w < 4; ++w) {
+      if ((int)(threadIdx.x >> 6) == w) {
+        base = s_at;
+        if (lane == 63) s_at = base + incl;
+      }
+      __syncthreads();
+    }
+    for (int j = 0; j < f.y; ++j) list[1 + base + incl - f.y + j] = perm[f.x + j];
+  }
+  if (threadIdx.x == 0) list[0] = s_at;
+}
+
+// Block kTabBlocks + 1 + ((row HKV + h) ntile + tile): 64 keys of one (sequence, KV head). K rows are copied as they
 // stand; V goes 4 keys x 4 dims at a time through a byte transpose. Keys past klen are left as they are: no query
 // sees them, so their weights are 0.
 template <int HD>
 __global__ __launch_bounds__(256) void paged_planes_kernel(AttnArgs p, const int32_t* klen, int8_t* kp, int8_t* vp,
-                                                           uint32_t* tab, int Sp, int ntile) {
+                                                           uint32_t* tab, int Sp, int ntile, const int32_t* perm,
+                                                           const int2* few, int nrow, int32_t* list) {
   if (blockIdx.x < kTabBlocks) {
     pre_table_block(p.lut, tab, blockIdx.x);
     return;
   }
-  const int b = blockIdx.x - kTabBlocks, z = b / ntile, k0 = (b - z * ntile) * 64;
+  if (blockIdx.x == kTabBlocks) {
+    rows_list_block(perm, few, nrow, list, p.sem);
+    return;
+  }
+  const int b = blockIdx.x - kTabBlocks - 1, z = b / ntile, k0 = (b - z * ntile) * 64;
   const int row = z / p.hkv, h = z - row * p.hkv;
   const int nk = min(klen[row] - k0, 64);
   if (nk <= 0) return;
@@ -2579,11 +2638,13 @@ extern "C" int64_t bx_attn_prefill_scratch(int32_t Z, int32_t S, int32_t HD) {
   return b < kBufRange - 16 ? b : 0;                 // larger: the register-staged form (no scratch)
 }
 
-// bx_exact_attn_paged_rows's scratch: the token order, the tile slots and key counts, the weight table, the planes
+// bx_exact_attn_paged_rows's scratch: the token order, the tile slots and key counts, the rows of sequences with few
+// tokens and their splits' workspace, the weight table, the planes
 struct RowsLayout {
-  int TT, nslot, Sp;
-  int64_t slots, klen, tab, planes, total;   // byte offsets (perm at 0)
+  int TT, nslot, Sp, nfew;                   // nfew: at most so many rows of sequences with few tokens
+  int64_t slots, klen, few, list, sem, ws, raw, tab, planes, total;   // byte offsets (perm at 0; raw -1: no kept scores)
 };
+constexpr int64_t kFewScoresMax = 1LL << 28;
 static RowsLayout rows_layout(int64_t R, int64_t nrow, int64_t HKV, int64_t M, int64_t HD, int64_t keys) {
   RowsLayout l;
   l.TT = (HD == 64 ? Pre2<64>::QR : Pre2<128>::QR) / (int)M;
@@ -2592,7 +2653,15 @@ static RowsLayout rows_layout(int64_t R, int64_t nrow, int64_t HKV, int64_t M, i
   auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
   l.slots = up(R * 4);
   l.klen = l.slots + up(l.nslot * 16LL);
-  l.tab = l.klen + up(nrow * 4);
+  l.nfew = (int)std::min(R, nrow * (kFewTokens - 1));
+  l.few = l.klen + up(nrow * 4);
+  l.list = l.few + up(nrow * 8);
+  l.sem = l.list + up(4LL * (1 + l.nfew));
+  l.ws = l.sem + up(4LL * kDecListBlocks);
+  l.raw = l.ws + up(dec_ws_bytes(kDecListBlocks, 1, (int)HD));
+  const int64_t scores = 32LL * l.nfew * HKV * keys;
+  l.tab = l.raw + (scores <= kFewScoresMax ? up(scores) : 0);
+  if (scores > kFewScoresMax) l.raw = -1;
   l.planes = l.tab + up(4LL * (kTabPad + kTabBlocks));
   l.total = l.planes + 6 * nrow * HKV * l.Sp * HD;
   return l;
@@ -2603,6 +2672,15 @@ extern "C" int64_t bx_attn_paged_rows_scratch(int32_t R, int32_t nrow, int32_t H
   if (R <= 0 || nrow <= 0 || HKV <= 0 || M < 1 || M > 4 || (HD != 64 && HD != 128) || keys <= 0 || keys >= 43690) return 0;
   const int64_t b = rows_layout(R, nrow, HKV, M, HD, keys).total;
   return b <= kRowsScratchMax ? b : 0;
+}
+
+template <int HD, bool RAW>
+static int launch_few(const AttnArgs& p, int nfew, hipStream_t st) {
+  const int grid = std::max(nfew * p.hkv, kDecListBlocks);
+  attn_dec_kernel<HD, 0, RAW, true><<<grid, kDecWaves * 64, 0, st>>>(p);
+  if (int rc = check_launch("attn_dec_kernel(list, scores)")) return rc;
+  attn_dec_kernel<HD, 1, RAW, true><<<grid, kDecWaves * 64, 0, st>>>(p);
+  return check_launch("attn_dec_kernel(list)");
 }
 
 extern "C" int bx_exact_attn_paged_rows(const int32_t* q, const int64_t* sh, const int64_t* qpos, int64_t sqpos_r,
@@ -2627,7 +2705,8 @@ extern "C" int bx_exact_attn_paged_rows(const int32_t* q, const int64_t* sh, con
   char* t = (char*)tmp;
   int32_t* perm = (int32_t*)t;
   int4* slots = (int4*)(t + l.slots);
-  int32_t* klen = (int32_t*)(t + l.klen);
+  int32_t *klen = (int32_t*)(t + l.klen), *list = (int32_t*)(t + l.list);
+  int2* few = (int2*)(t + l.few);
   uint32_t* tab = (uint32_t*)(t + l.tab);
   int8_t* kp = (int8_t*)(t + l.planes);
   int8_t* vp = kp + 3LL * nrow * HKV * l.Sp * HD;
@@ -2640,23 +2719,28 @@ extern "C" int bx_exact_attn_paged_rows(const int32_t* q, const int64_t* sh, con
   p.lut = lut; p.l2e = l2e;
   p.num = num; p.den = den; p.snum_tile = (int64_t)M * HD; p.snum_row = HD; p.sden_tile = M;
   p.nsplit = 1;
+  p.rmap = rmap; p.list = list; p.sem = (int32_t*)(t + l.sem); p.mx_ws = (int64_t*)(t + l.ws);
+  p.raw = l.raw < 0 ? nullptr : (int64_t*)(t + l.raw);
+  p.one_keys = kDecOneKeys / HD;
   hipStream_t st = (hipStream_t)stream;
-  rows_group_kernel<<<nrow + 1, 256, 0, st>>>(rmap, qpos, sqpos_r, R, M, nrow, p.S, l.TT, l.nslot, perm, slots, klen);
+  rows_group_kernel<<<nrow + 1, 256, 0, st>>>(rmap, qpos, sqpos_r, R, M, nrow, p.S, l.TT, l.nslot, perm, slots, klen, few);
   if (int rc = check_launch("rows_group_kernel")) return rc;
   const int ntile = l.Sp / 64, Z = nrow * HKV;
   const RowMap rm = {perm, slots, l.nslot, nrow, M, HKV};
   if (HD == 64) {
-    paged_planes_kernel<64><<<kTabBlocks + Z * ntile, 256, 0, st>>>(p, klen, kp, vp, tab, l.Sp, ntile);
+    paged_planes_kernel<64><<<kTabBlocks + 1 + Z * ntile, 256, 0, st>>>(p, klen, kp, vp, tab, l.Sp, ntile, perm, few, nrow, list);
     if (int rc = check_launch("paged_planes_kernel")) return rc;
     allow_lds_attn((const void*)attn_pre2_kernel<64, true>, Pre2<64>::LDS);
     attn_pre2_kernel<64, true><<<l.nslot * HKV, 64 * Pre2<64>::NW, Pre2<64>::LDS, st>>>(p, kp, Z, l.Sp, tab, rm);
   } else {
-    paged_planes_kernel<128><<<kTabBlocks + Z * ntile, 256, 0, st>>>(p, klen, kp, vp, tab, l.Sp, ntile);
+    paged_planes_kernel<128><<<kTabBlocks + 1 + Z * ntile, 256, 0, st>>>(p, klen, kp, vp, tab, l.Sp, ntile, perm, few, nrow, list);
     if (int rc = check_launch("paged_planes_kernel")) return rc;
     allow_lds_attn((const void*)attn_pre2_kernel<128, true>, Pre2<128>::LDS);
     attn_pre2_kernel<128, true><<<l.nslot * HKV, 64 * Pre2<128>::NW, Pre2<128>::LDS, st>>>(p, kp, Z, l.Sp, tab, rm);
   }
-  return check_launch("attn_pre2_kernel(rows)");
+  if (int rc = check_launch("attn_pre2_kernel(rows)")) return rc;
+  if (l.raw < 0) return HD == 64 ? launch_few<64, false>(p, l.nfew, st) : launch_few<128, false>(p, l.nfew, st);
+  return HD == 64 ? launch_few<64, true>(p, l.nfew, st) : launch_few<128, true>(p, l.nfew, st);
 }
 
 extern "C" int bx_exact_attn_prefill(const int32_t* qg, int64_t sq_z, int64_t sq_row, const int64_t* shg,

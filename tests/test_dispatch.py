@@ -22,3 +22,16 @@ def test_kept_scores_rule(HD):
     for T in (128, 144, 160, 176, 184, 191, 192):
         for keys in (16, 1024, 2032, 2048):
             assert auto_nsplit(T, keys, HD) == (1, 0), (T, keys)
+
+
+def test_grouped_rule():
+    """The grouped form from its number of (token, KV head)s and of tokens per table row on, never past its scratch."""
+    from bitexact.vllm_plugin.tri_exact_attn import rows_scratch
+    for HD, tokens in ((64, 192), (128, 144)):
+        for HKV in (1, 8):
+            t = tokens * 8 // HKV
+            assert rows_scratch(t, HKV, 4, HD, 8, 512) > 0 and rows_scratch(t - 1, HKV, 4, HD, 8, 512) == 0
+        assert rows_scratch(8 * 40, 8, 4, HD, 40, 512) > 0 and rows_scratch(8 * 40 - 1, 8, 4, HD, 40, 512) == 0
+        assert rows_scratch(4096, 8, 4, HD, 64, 16384) == 0
+        assert rows_scratch(4096, 8, 4, HD, 8, 43700) == rows_scratch(4096, 8, 5, HD, 8, 512) == 0
+    assert rows_scratch(4096, 8, 4, 96, 8, 512) == 0

@@ -267,6 +267,43 @@ def test_paged_rows_equal_decode_form(dev, HD, M, bs, order):
         assert torch.equal(n1, n2) and torch.equal(d1, d2)
 
 
+@pytest.mark.parametrize("HD,HKV,M,keys,few,chunks", [
+    (64, 4, 4, 2048, [7, 8, 9, 1, 0, 6], [300, 130]),          # the line; few rows: many splits
+    (128, 4, 3, 4096, [1] * 20 + [7], [400]),
+    (64, 4, 4, 640, [7] * 40 + [3] * 20, [260, 1]),            # more tiles than blocks: one split
+    (128, 4, 2, 1024, [5] * 11 + [8], [250]),                  # 220 tiles: two splits
+    (64, 8, 4, 16384, [1] * 15, [200]),                        # scores past their limit: K read twice
+    (128, 8, 1, 16384, [7] * 3 + [1] * 6, [150])])
+def test_paged_rows_mixed_steps(dev, HD, HKV, M, keys, few, chunks):
+    """Steps of prefill chunks and sequences with few tokens (decoding ones) in the grouped form against the per-token
+    form, bit for bit: counts at the line between the two, contexts of any length (none, one key, the last), tokens of a
+    sequence in any order, padding rows outside the table, repeated on the same scratch."""
+    from bitexact.vllm_plugin import tri_exact_attn, tri_paged
+    g = torch.Generator().manual_seed(HD + keys + len(few))
+    bs, nphys = 16, 96
+    nblk, counts = keys // bs, few + chunks
+    nrow = len(counts)
+    c = torch.randint(-R.LIM3, R.LIM3 + 1, (nphys, HKV, bs, 2 * HD), generator=g).to(torch.int32)
+    cl = tri_paged.to_limbs(c.to(dev))
+    bt = torch.randint(0, nphys, (nrow, nblk), generator=g).to(torch.int32).to(dev)
+    rmap = torch.cat([torch.full((n,), i) for i, n in enumerate(counts)])
+    rmap = rmap[torch.randperm(len(rmap), generator=g)]
+    Rr = len(rmap)
+    qpos = torch.randint(-1, keys, (Rr, M), generator=g)
+    qpos[::5] = torch.randint(-1, 300, (len(qpos[::5]), 1), generator=g)
+    qpos[1], qpos[2], qpos[3] = keys - 1, 0, -1
+    inside = torch.ones(Rr, dtype=torch.bool)
+    inside[7::31] = False
+    q = torch.randint(-(1 << 22), (1 << 22) + 1, (Rr, HKV, M, HD), generator=g).to(torch.int32).to(dev)
+    sh = torch.randint(-46, -36, (Rr, HKV, M), generator=g).to(dev)
+    args = lambda r, p: (q, sh, p.to(dev), cl, bt, r.to(dev), _lut(dev), R.L2E28_HD[HD])
+    assert tri_exact_attn.rows_scratch(Rr, HKV, M, HD, nrow, keys) > 0
+    n1, d1 = tri_exact_attn.attend(*args(rmap, torch.where(inside[:, None], qpos, -1)), nsplit=1)
+    for _ in range(3):
+        n2, d2 = tri_exact_attn.attend(*args(torch.where(inside, rmap, nrow), qpos))
+        assert torch.equal(n1, n2) and torch.equal(d1, d2)
+
+
 @pytest.mark.parametrize("HD,npad,pad", [(64, 1, -1), (64, 33, -1), (64, 300, -(1 << 40)), (128, 40, 3), (128, 200, 1 << 40),
                                          (64, 513, None)])
 def test_paged_rows_outside_the_table(dev, HD, npad, pad):
