@@ -1909,6 +1909,7 @@ struct Plan {
   int rb, cg, ks_waves, u, spw;   // gemv
   int parts, mp;                  // gemv row parts, output rows per part
   int tile;                       // tile config
+  int itile;                      // itile kernel: waves per block (0: none)
   int tiles_x, tiles_y, split, kbytes;
   size_t lds;
   int64_t ws_bytes;               // zero-invariant split-K region
@@ -2061,6 +2062,75 @@ static bool stream_plan(int rows_a, int M_out, int N, int K, bool exact, bool pl
   return true;
 }
 
+// The itile kernel's shapes for NA limb planes: W waves, WM of them along the rows, each 32 TM x 32 TN outputs; S ring
+// stages. Four waves: 128 x 256, 128 x 128, 64 x 128 outputs a block and two blocks a CU; eight: 128 x 256 and one.
+template <int NA, int W>
+struct ItShape;
+template <>
+struct ItShape<1, 4> {
+  static constexpr int WM = 2, TM = 2, TN = 4, S = 3;
+};
+template <>
+struct ItShape<2, 4> {
+  static constexpr int WM = 2, TM = 2, TN = 2, S = 3;
+};
+template <>
+struct ItShape<2, 8> {
+  static constexpr int WM = 4, TM = 1, TN = 4, S = 4;
+};
+template <>
+struct ItShape<3, 4> {
+  static constexpr int WM = 2, TM = 1, TN = 2, S = 3;
+};
+template <>
+struct ItShape<3, 8> {
+  static constexpr int WM = 4, TM = 1, TN = 4, S = 3;
+};
+
+template <int NA, int W>
+static void itile_grid(int M, int N, int& tx, int& ty) {
+  using I = ItShape<NA, W>;
+  constexpr int BM = 32 * I::TM * I::WM, BN = 32 * I::TN * (W / I::WM);
+  tx = (N + BN - 1) / BN;
+  ty = (M + BM - 1) / BM;
+}
+
+// Whether the itile kernel takes an int8 product, and its shape; else tile_kernel, which can split K.
+// A block walks all of K, so few tiles of a long K stay with the split: two limbs, K = 8192, 128 x 1024 outputs
+// (8 tiles) 42 us here and 24 split, 256 x 2048 (32 tiles) 51 and 37, 512 x 2048 (64 tiles) 53 and 65; three limbs
+// 256 x 2048 (64 tiles) 46 and 41, 384 x 2048 (96) 48 and 70. At K = 4096 the line is near 24 tiles (two limbs
+// 256 x 1024, 16 tiles: 24.0 and 25.9; 384 x 1024, 24 tiles: 24.3 and 29.7), at K = 2048 below 8 (256 x 256: 14.5 and
+// 15.3, 129 x 256: 14.5 and 13.3).
+// Eight waves re-read less and run a full chip faster (two limbs 2048 x 16384 of K = 2048: 154 us, four waves 159;
+// three: 216 and 241), four fill a part-empty last round better: the line is where the eight-wave tiles' rounds over
+// the CUs cover what the four-wave tiles need (two limbs 1024 x 4096 of K = 4096, 128 eight-wave tiles: 47 and 41 us;
+// 1500 x 4096, 192 tiles: 55 and 64; three limbs 700 x 16384, 384 tiles: 96 and 86).
+template <int NA>
+static bool itile_plan(int M, int N, int K, Plan& s) {
+  // 32-bit sums over all of K (the split sums 64-bit parts) and 32-bit offsets
+  if (K % 64 || K >= 131072 || (int64_t)NA * M * K >= kBufRange - 16 || (int64_t)N * K >= kBufRange - 16) return false;
+  int tx, ty;
+  itile_grid<NA, 4>(M, N, tx, ty);
+  const int64_t t4 = (int64_t)tx * ty;
+  if (t4 < (K <= 2048 ? 8 : K <= 4096 ? 24 : NA == 3 ? 96 : 64)) return false;
+  s.itile = 4;
+  if constexpr (NA > 1) {
+    int tx8, ty8;
+    itile_grid<NA, 8>(M, N, tx8, ty8);
+    const int64_t cus = device_cus(), r8 = ((int64_t)tx8 * ty8 + cus - 1) / cus;
+    if (NA == 2 ? 2 * r8 <= (t4 + cus - 1) / cus : 3 * r8 * cus <= t4) {
+      s.itile = 8;
+      tx = tx8;
+      ty = ty8;
+    }
+  }
+  s.tiles_x = tx;
+  s.tiles_y = ty;
+  s.split = 1;
+  s.kbytes = K;
+  return true;
+}
+
 // planes: the caller supplies q's limb planes (exact mode), so a plane-reading kernel costs no split launch
 static Plan make_plan(int rows_a, int M_out, int N, int K, int nb, int na, bool exact, bool planes = false) {
   Plan s = {};
@@ -2111,6 +2181,10 @@ static Plan make_plan(int rows_a, int M_out, int N, int K, int nb, int na, bool 
     s.lds = (((size_t)RA * (s.kbytes + 16) + 15) & ~(size_t)15) + (size_t)nb * RA * BNC * 4 + 64;
   } else {
     s.gemv = false;
+    if (nb == 1 && (na == 1   ? itile_plan<1>(M_out, N, K, s)
+                    : na == 2 ? itile_plan<2>(M_out, N, K, s)
+                              : itile_plan<3>(M_out, N, K, s)))
+      return s;
     const int64_t big = (int64_t)((M_out + 127) / 128) * ((N + 127) / 128);
     if (dec_tile)
       s.tile = T_DEC;
@@ -2222,84 +2296,24 @@ static bool xtile_fits(const LinArgs& p, const Plan& s) {
          2 * p.ld_plane + (int64_t)p.N * p.ld_row < kBufRange - 16 && (int64_t)p.M * p.ldq * 4 < kBufRange - 16;
 }
 
-// The itile kernel's shapes for NA limb planes: W waves, WM of them along the rows, each 32 TM x 32 TN outputs; S ring
-// stages. Four waves: 128 x 256, 128 x 128, 64 x 128 outputs a block and two blocks a CU; eight: 128 x 256 and one.
-template <int NA, int W>
-struct ItShape;
-template <>
-struct ItShape<1, 4> {
-  static constexpr int WM = 2, TM = 2, TN = 4, S = 3;
-};
-template <>
-struct ItShape<2, 4> {
-  static constexpr int WM = 2, TM = 2, TN = 2, S = 3;
-};
-template <>
-struct ItShape<2, 8> {
-  static constexpr int WM = 4, TM = 1, TN = 4, S = 4;
-};
-template <>
-struct ItShape<3, 4> {
-  static constexpr int WM = 2, TM = 1, TN = 2, S = 3;
-};
-template <>
-struct ItShape<3, 8> {
-  static constexpr int WM = 4, TM = 1, TN = 4, S = 3;
-};
-
-template <int NA, int W>
-static int64_t itile_tiles(const LinArgs& p) {
-  using I = ItShape<NA, W>;
-  constexpr int BM = 32 * I::TM * I::WM, BN = 32 * I::TN * (W / I::WM);
-  return (int64_t)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-}
-
-// Waves of the itile shape for a product; 0: tile_kernel, which can split K.
-// A block walks all of K, so few tiles of a long K stay with the split: two limbs, K = 8192, 128 x 1024 outputs
-// (8 tiles) 42 us here and 24 split, 256 x 2048 (32 tiles) 51 and 37, 512 x 2048 (64 tiles) 53 and 65; three limbs
-// 256 x 2048 (64 tiles) 46 and 41, 384 x 2048 (96) 48 and 70. At K = 4096 the line is near 24 tiles (two limbs
-// 256 x 1024, 16 tiles: 24.0 and 25.9; 384 x 1024, 24 tiles: 24.3 and 29.7), at K = 2048 below 8 (256 x 256: 14.5 and
-// 15.3, 129 x 256: 14.5 and 13.3).
-// Eight waves re-read less and run a full chip faster (two limbs 2048 x 16384 of K = 2048: 154 us, four waves 159;
-// three: 216 and 241), four fill a part-empty last round better: the line is where the eight-wave tiles' rounds over
-// the CUs cover what the four-wave tiles need (two limbs 1024 x 4096 of K = 4096, 128 eight-wave tiles: 47 and 41 us;
-// 1500 x 4096, 192 tiles: 55 and 64; three limbs 700 x 16384, 384 tiles: 96 and 86).
-template <int NA>
-static int itile_waves(const LinArgs& p) {
-  // 32-bit sums over all of K (the split sums 64-bit parts) and 32-bit offsets
-  if (p.K % 64 || p.K >= 131072 || (int64_t)NA * p.M * p.K >= kBufRange - 16 ||
-      (int64_t)p.N * p.ld_row >= kBufRange - 16)
-    return 0;
-  const int64_t t4 = itile_tiles<NA, 4>(p);
-  if (t4 < (p.K <= 2048 ? 8 : p.K <= 4096 ? 24 : NA == 3 ? 96 : 64)) return 0;
-  if constexpr (NA == 1) {
-    return 4;
-  } else {
-    const int64_t cus = device_cus(), r8 = (itile_tiles<NA, 8>(p) + cus - 1) / cus;
-    return (NA == 2 ? 2 * r8 <= (t4 + cus - 1) / cus : 3 * r8 * cus <= t4) ? 8 : 4;
-  }
-}
-
 template <int NA, int MODE, int W>
-static int launch_itile(LinArgs& p, hipStream_t st) {
+static int launch_itile(LinArgs& p, const Plan& s, hipStream_t st) {
   using I = ItShape<NA, W>;
   constexpr int BM = 32 * I::TM * I::WM, WN = W / I::WM, BN = 32 * I::TN * WN;
   constexpr size_t LDS = (size_t)I::S * (NA * BM + BN) * 64;
-  const int tx = (p.N + BN - 1) / BN, ty = (p.M + BM - 1) / BM;
-  p.xcd_remap = (tx * ty) % 8 == 0 && ty % 4 == 0 ? 4 : 0;
+  p.xcd_remap = (s.tiles_x * s.tiles_y) % 8 == 0 && s.tiles_y % 4 == 0 ? 4 : 0;
   auto k = itile_kernel<NA, MODE, I::WM, WN, I::TM, I::TN, I::S>;
   allow_lds(k, LDS);
-  k<<<dim3(tx, ty), 64 * W, LDS, st>>>(p);
+  k<<<dim3(s.tiles_x, s.tiles_y), 64 * W, LDS, st>>>(p);
   return check_launch("itile_kernel");
 }
 
 template <int NA, int NB, int MODE>
 static int launch_tile(LinArgs& p, const Plan& s, hipStream_t st) {
   if constexpr (NB == 1 && (MODE == JOIN || MODE == RAW32)) {
-    const int waves = itile_waves<NA>(p);
-    if (waves == 4) return launch_itile<NA, MODE, 4>(p, st);
+    if (s.itile == 4) return launch_itile<NA, MODE, 4>(p, s, st);
     if constexpr (NA > 1)
-      if (waves == 8) return launch_itile<NA, MODE, 8>(p, st);
+      if (s.itile == 8) return launch_itile<NA, MODE, 8>(p, s, st);
   }
   p.ks = s.kbytes;
   bind_ws(p, s);
@@ -2597,13 +2611,14 @@ extern "C" int bx_exact_linear_planes_plan(int32_t M, int32_t N, int32_t K, int3
 }
 
 // The int8 GEMM's plan for M output rows of nl stacked limbs (nl = 0: the raw int32 GEMM of M stacked rows):
-// out[0] = 1 gemv, 3 tile (itile where its rule takes it: no split then), 4 staged, 5 stream; out[1] = tile
-// configuration (-1 otherwise); out[2] = K splits; out[3] = blocks per split; out[4] = gemv column groups (16 columns each); out[5] = gemv row parts.
+// out[0] = 1 gemv, 3 tile, 4 staged, 5 stream, 6 itile; out[1] = tile configuration (itile: waves per block; -1
+// otherwise); out[2] = K splits; out[3] = blocks per split; out[4] = gemv column groups (16 columns each); out[5] = gemv
+// row parts.
 extern "C" int bx_int8_gemm_plan(int32_t M, int32_t N, int32_t K, int32_t nl, int32_t* out) {
   BX_REQUIRE(out && M > 0 && N > 0 && K > 0 && nl >= 0 && nl <= 3, "bad plan query");
   const Plan s = nl == 0 ? make_plan(M, M, N, K, 1, 1, false) : make_plan(nl * M, M, N, K, 1, nl, false);
-  out[0] = s.stream ? 5 : s.staged ? 4 : s.gemv ? 1 : 3;
-  out[1] = (s.gemv || s.staged || s.stream) ? -1 : s.tile;
+  out[0] = s.stream ? 5 : s.staged ? 4 : s.gemv ? 1 : s.itile ? 6 : 3;
+  out[1] = (s.gemv || s.staged || s.stream) ? -1 : s.itile ? s.itile : s.tile;
   out[2] = s.split;
   out[3] = s.gemv ? s.tiles_x * s.parts : s.tiles_x * s.tiles_y;
   out[4] = s.gemv ? s.cg : 0;

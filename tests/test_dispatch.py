@@ -1,5 +1,7 @@
 """Which form the attention entry points choose by size (no GPU call is made)."""
 
+import ctypes
+
 import pytest
 
 
@@ -35,3 +37,32 @@ def test_grouped_rule():
         assert rows_scratch(4096, 8, 4, HD, 64, 16384) == 0
         assert rows_scratch(4096, 8, 4, HD, 8, 43700) == rows_scratch(4096, 8, 5, HD, 8, 512) == 0
     assert rows_scratch(4096, 8, 4, 96, 8, 512) == 0
+
+
+def test_int8_tile_plan():
+    """The int8 product's plan names the kernel that is launched and asks for that kernel's workspace: the pipelined
+    tiles (6) on both sides of their number of tiles at short, middle and long K, each with its waves; else the tile
+    kernel (3), which splits K."""
+    from bitexact import _hip
+    L = _hip.lib()
+    out = (ctypes.c_int32 * 6)()
+
+    def plan(M, N, K, nl):
+        assert L.bx_int8_gemm_plan(M, N, K, nl, out) == 0
+        ws = L.bx_int8_gemm_workspace(M, N, K, max(nl, 1))
+        assert (ws > 0) == (out[2] > 1)
+        return tuple(out[:4])
+    bn, bm = {0: 256, 1: 256, 2: 128, 3: 128}, {0: 128, 1: 128, 2: 128, 3: 64}
+    for nl in (0, 1, 2, 3):
+        long = 96 if nl == 3 else 64
+        for K, line in ((64, 8), (2048, 8), (2112, 24), (4096, 24), (4160, long), (8192, long)):
+            M, N = 4 * bm[nl], line // 4 * bn[nl]          # four row tiles
+            assert plan(M, N, K, nl) == (6, 4, 1, line), (nl, K)
+            kernel, tile, split, blocks = plan(M, N - bn[nl], K, nl)
+            assert kernel == 3 and tile != 4 and blocks > 0, (nl, K)
+            assert plan(M, N, K + 16, nl)[0] == 3
+    assert plan(2048, 16384, 2048, 1) == (6, 4, 1, 16 * 64)
+    assert plan(2048, 16384, 2048, 2) == plan(2048, 16384, 2048, 3) == (6, 8, 1, 16 * 64)
+    assert plan(1024, 4096, 4096, 2) == (6, 4, 1, 8 * 32) and plan(1500, 4096, 4096, 2) == (6, 8, 1, 12 * 16)
+    assert plan(704, 16384, 2048, 3) == (6, 4, 1, 11 * 128) and plan(705, 16384, 2048, 3) == (6, 8, 1, 6 * 64)
+    assert plan(2048, 1 << 20, 2048, 1)[0] == 3            # weights past the 32-bit offsets
