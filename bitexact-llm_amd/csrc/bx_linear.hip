@@ -1232,7 +1232,7 @@ __global__ __launch_bounds__(WM * WN * 64) void xtile_kernel(LinArgs p) {
 // other's MFMAs. M = 2048, N = 16384, K = 2048: one limb 118 -> 110 us, two 231 -> 154, three 309 -> 217, against
 // tile_kernel's 128 x 128 tile, which waits for its operands; M = 256, N = 4096, K = 4096: 28 -> 27, 35 -> 26, 40 -> 26.
 // =====================================================================================================
-template <int NA, int MODE, int WM, int WN, int TM, int TN, int S>
+template <int NA, int MODE, int WM, int WN, int TM, int TN, int S, bool STREAM>
 __global__ __launch_bounds__(64 * WM * WN, 2) void itile_kernel(LinArgs p) {
   constexpr int NW = WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN, BK = 64;
   constexpr int SA = NA * BM * BK, STAGE = SA + BN * BK;
@@ -1376,13 +1376,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void itile_kernel(LinArgs p) {
         const int m = m0 + (wm * TM + a2) * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
         if (!full && !(m < p.M && n < p.N)) continue;
         const int64_t o = (int64_t)m * p.N + n;
+        auto put = [](auto* d, auto v) {
+          if constexpr (STREAM) __builtin_nontemporal_store(v, d);
+          else *d = v;
+        };
         if constexpr (MODE == RAW32) {
-          __builtin_nontemporal_store(acc[0][a2][t][e], (int32_t*)p.out + o);
+          put((int32_t*)p.out + o, acc[0][a2][t][e]);
         } else {
           int64_t v = acc[0][a2][t][e];
           if constexpr (NA > 1) v += (int64_t)acc[1][a2][t][e] << 8;
           if constexpr (NA > 2) v += (int64_t)acc[2][a2][t][e] << 16;
-          __builtin_nontemporal_store(v, (int64_t*)p.out + o);
+          put((int64_t*)p.out + o, v);
         }
       }
     }
@@ -2307,7 +2311,11 @@ static int launch_itile(LinArgs& p, const Plan& s, hipStream_t st) {
   constexpr int BM = 32 * I::TM * I::WM, WN = W / I::WM, BN = 32 * I::TN * WN;
   constexpr size_t LDS = (size_t)I::S * (NA * BM + BN) * 64;
   p.xcd_remap = (s.tiles_x * s.tiles_y) % 8 == 0 && s.tiles_y % 4 == 0 ? 4 : 0;
-  auto k = itile_kernel<NA, MODE, I::WM, WN, I::TM, I::TN, I::S>;
+  // rows that do not start on a 128-byte line share lines with their neighbours: streamed past the caches, each part of
+  // one went to HBM by itself (one limb, 1873 x 4039 of K = 1024 33.8 us, stored plainly 20.9; 2015 x 16343 of K = 2048
+  // 159.7 and 123.8)
+  auto k = p.N % (MODE == RAW32 ? 32 : 16) == 0 ? itile_kernel<NA, MODE, I::WM, WN, I::TM, I::TN, I::S, true>
+                                                : itile_kernel<NA, MODE, I::WM, WN, I::TM, I::TN, I::S, false>;
   allow_lds(k, LDS);
   k<<<dim3(s.tiles_x, s.tiles_y), 64 * W, LDS, st>>>(p);
   return check_launch("itile_kernel");
