@@ -2100,15 +2100,16 @@ static void itile_grid(int M, int N, int& tx, int& ty) {
 }
 
 // Whether the itile kernel takes an int8 product, and its shape; else tile_kernel, which can split K.
-// A block walks all of K, so few tiles of a long K stay with the split: two limbs, K = 8192, 128 x 1024 outputs
-// (8 tiles) 42 us here and 24 split, 256 x 2048 (32 tiles) 51 and 37, 512 x 2048 (64 tiles) 53 and 65; three limbs
-// 256 x 2048 (64 tiles) 46 and 41, 384 x 2048 (96) 48 and 70. At K = 4096 the line is near 24 tiles (two limbs
-// 256 x 1024, 16 tiles: 24.0 and 25.9; 384 x 1024, 24 tiles: 24.3 and 29.7), at K = 2048 below 8 (256 x 256: 14.5 and
-// 15.3, 129 x 256: 14.5 and 13.3). One limb has the least work per tile: where tile_kernel's 64 x 128 tiles fill half
-// the chip or more without a split they are faster up to 80 tiles here (K = 4096: 48 tiles 28.9 and 27.8, 64 29.3 and
-// 28.7, 80 30.2 and 31.8; K = 8192: 64 52.6 and 50.5, 80 54.3 and 56.9), at K <= 2048 up to 40 (K = 2048: 32 tiles 16.6
-// and 16.1, 40 16.6 and 16.9; K = 1024: 32 11.6 and 10.4, 48 11.4 and 11.2); where they split the lines above hold
-// (K = 4096: 16 tiles 27.5 and 27.7, 24 28.6 and 31.4; K = 2048: 8 16.1 and 17.4, 24 16.3 and 27.9).
+// A block walks all of K, so few tiles of a long K stay with the split. Past K = 4096 the split's tiles decide: two
+// limbs, K = 8192, 256 x 2048 outputs 51 us here and 37 split, 400 x 2048 (112 of its tiles) 51 and 45, 512 x 2048 (128:
+// no split any more) 53 and 63; three limbs 256 x 2048 (64 tiles) 45 and 39, 384 x 2048 (96) 46 and 69. At K = 4096 the
+// line is near 24 tiles here (two limbs 256 x 1024, 16 tiles: 24.0 and 25.6; 256 x 2048, 32 tiles: 27.2 and 29.6; one
+// limb 16 tiles: 27.5 and 27.7, 24 28.6 and 31.4), at K = 2048 below 8 (two limbs 129 x 512, 8 tiles: 14.4 and 14.3,
+// one limb 129 x 1024, 8 tiles: 16.1 and 17.4).
+// One limb has the least work per tile: where tile_kernel runs unsplit it is faster up to 64 tiles here at K <= 2048 (K
+// = 2048: 32 tiles 16.6 and 16.1, 64 17.9 and 18.0, 96 18.7 and 20.3) and up to 80 above (K = 4096: 48 tiles 28.9 and
+// 27.8, 64 29.3 and 28.7, 80 30.2 and 31.8; K = 8192: 64 52.6 and 50.5, 80 54.3 and 56.9), with rows that share lines
+// up to 112 (K = 1024, N = 4038: 64 tiles 13.1 and 11.2; K = 2048, N = 3038: 96 20.2 and 19.6).
 // Eight waves re-read less and run a full chip faster (two limbs 2048 x 16384 of K = 2048: 154 us, four waves 159;
 // three: 216 and 241), four fill a part-empty last round better: the line is where the eight-wave tiles' rounds over
 // the CUs cover what the four-wave tiles need (two limbs 1024 x 4096 of K = 4096, 128 eight-wave tiles: 47 and 41 us;
@@ -2120,8 +2121,12 @@ static bool itile_plan(int M, int N, int K, Plan& s) {
   int tx, ty;
   itile_grid<NA, 4>(M, N, tx, ty);
   const int64_t t4 = (int64_t)tx * ty;
-  const bool unsplit = 2LL * ((M + 63) / 64) * ((N + 127) / 128) >= device_cus();   // tile_kernel without a K split
-  if (t4 < (NA == 1 && unsplit ? (K <= 2048 ? 40 : 80) : K <= 2048 ? 8 : K <= 4096 ? 24 : NA == 3 ? 96 : 64)) return false;
+  const int64_t mid = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
+  const bool unsplit = 2 * mid >= device_cus();             // tile_kernel's 64 x 128 tiles need no K split
+  bool take = t4 >= (K <= 2048 ? 8 : 24);
+  if (K > 4096) take = NA == 2 ? unsplit : NA == 3 && mid >= 96;
+  if (NA == 1 && unsplit) take = t4 >= (N % 16 ? 112 : K <= 2048 ? 64 : 80);
+  if (!take) return false;
   s.itile = 4;
   if constexpr (NA > 1) {
     int tx8, ty8;

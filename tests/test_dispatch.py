@@ -54,16 +54,20 @@ def test_int8_tile_plan():
         return tuple(out[:4])
     bn, bm = {0: 256, 1: 256, 2: 128, 3: 128}, {0: 128, 1: 128, 2: 128, 3: 64}
     for nl in (0, 1, 2, 3):
-        long = {0: 80, 1: 80, 2: 64, 3: 96}[nl]
-        for K, line in ((64, 8), (2048, 8), (2112, 24), (4096, 24), (4160, long), (8192, long)):
+        for K, line in ((64, 8), (2048, 8), (2112, 24), (4096, 24)):
             M, N = 4 * bm[nl], line // 4 * bn[nl]          # four row tiles
             assert plan(M, N, K, nl) == (6, 4, 1, line), (nl, K)
             kernel, tile, split, blocks = plan(M, N - bn[nl], K, nl)
             assert kernel == 3 and tile != 4 and blocks > 0, (nl, K)
             assert plan(M, N, K + 16, nl)[0] == 3
-    # one limb where the tile kernel's own tiles fill half the chip unsplit
-    for K, M in ((2048, 640), (2112, 1280), (4096, 1280)):
+    for K in (4160, 8192):                                 # by the tile kernel's 64 x 128 tiles
+        assert plan(512, 2048, K, 2)[0] == 6 and plan(448, 2048, K, 2)[0] == 3 and plan(400, 2048, K, 2)[0] == 3
+        assert plan(384, 2048, K, 3)[0] == 6 and plan(320, 2048, K, 3)[0] == 3
+    # one limb where the tile kernel runs unsplit
+    for K, M in ((64, 1024), (2048, 1024), (2112, 1280), (4096, 1280), (8192, 1280)):
         assert plan(M, 2048, K, 1)[:3] == (6, 4, 1) and plan(M - 128, 2048, K, 1)[::2] == (3, 1), K
+        assert plan(1792, 2047, K, 0)[:3] == (6, 4, 1) and plan(1664, 2047, K, 1)[::2] == (3, 1), K
+    assert plan(256, 2048, 8192, 1)[0] == 3                # a split, past K = 4096
     assert plan(2048, 16384, 2048, 1) == (6, 4, 1, 16 * 64)
     assert plan(2048, 16384, 2048, 2) == plan(2048, 16384, 2048, 3) == (6, 8, 1, 16 * 64)
     assert plan(1024, 4096, 4096, 2) == (6, 4, 1, 8 * 32) and plan(1500, 4096, 4096, 2) == (6, 8, 1, 12 * 16)

@@ -517,7 +517,7 @@ def test_int8_stream_wide(dev, N, K):
 @pytest.mark.parametrize("M,N,K,nl", [(129, 2060, 64, 1), (300, 1800, 192, 1), (130, 513, 128, 2), (65, 1025, 320, 2),
                                       (2049, 2050, 192, 2), (2040, 2302, 320, 2), (44, 1025, 64, 3), (257, 260, 2048, 3),
                                       (2049, 3000, 128, 3), (2050, 3070, 256, 3), (384, 2050, 2112, 0),
-                                      (384, 4100, 64, 0), (384, 2500, 64, 0), (129, 2048, 64, 1), (130, 512, 128, 2), (2049, 2048, 192, 2),
+                                      (384, 2500, 64, 0), (129, 2048, 64, 1), (130, 512, 128, 2), (2049, 2048, 192, 2),
                                       (257, 256, 2048, 3), (2050, 3072, 256, 3), (384, 2560, 64, 0)])
 def test_int8_pipelined_tiles(dev, M, N, K, nl):
     """int8 prefill on the pipelined tiles (four- and eight-wave shapes, nl = 0: raw int32 rows): ragged last row and
