@@ -1987,9 +1987,10 @@ __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArg
       for (int i = 0; i < 3; ++i) qb[i][kk] = v4i{(int)l[i][0], (int)l[i][1], (int)l[i][2], (int)l[i][3]};
     }
   }
-  // (positions past S - 1 see every key: the caller's contract keeps qpos < S, so the clamp changes nothing)
+  // (positions past S - 1 see every key, negative ones, whatever their 64 bits, none: the clamp changes neither)
   const int my_qpos =
-      live && keys ? (int)imin(p.qpos[(qg / p.qpos_div) * p.qpos_tile + (int64_t)qr * p.qpos_row], (int64_t)p.S) : -1;
+      live && keys ? (int)imax(imin(p.qpos[(qg / p.qpos_div) * p.qpos_tile + (int64_t)qr * p.qpos_row], (int64_t)p.S), -1)
+                   : -1;
   const int64_t shift = live ? (int64_t)(kFK + 3 - kFZ) - p.sh[qg * p.sh_tile + qr] : 0;
   if (threadIdx.x == 0) s_kend = 0;
   __syncthreads();

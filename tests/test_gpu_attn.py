@@ -304,6 +304,39 @@ def test_paged_rows_mixed_steps(dev, HD, HKV, M, keys, few, chunks):
         assert torch.equal(n1, n2) and torch.equal(d1, d2)
 
 
+@pytest.mark.parametrize("HD", [64, 128])
+def test_positions_below_int32_see_no_key(dev, HD):
+    """Rows masked by a position of any negative value (the type's lowest, low words that read as a position) see no
+    key, as with -1: the grouped paged form against the per-token one, and the limb-plane prefill."""
+    from bitexact.exact.attention import prefill
+    from bitexact.vllm_plugin import tri_exact_attn, tri_paged
+    g = torch.Generator().manual_seed(HD)
+    HKV, M, bs, nrow, nblk, Rr = 4, 4, 16, 3, 12, 400
+    S = nblk * bs
+    c = torch.randint(-R.LIM3, R.LIM3 + 1, (nrow * nblk, HKV, bs, 2 * HD), generator=g).to(torch.int32)
+    cl = tri_paged.to_limbs(c.to(dev))
+    bt = torch.randperm(nrow * nblk, generator=g).to(torch.int32).view(nrow, nblk).to(dev)
+    rmap = torch.randint(0, nrow, (Rr,), generator=g).to(dev)
+    low = torch.tensor([-(1 << 63), -(1 << 32), 100 - (1 << 40), -(1 << 31) - 1, -1])
+    masked = torch.rand(Rr, M, generator=g) < 0.5
+    masked[rmap.cpu() == 0] = True                         # a sequence without any visible key
+    qpos = torch.randint(0, S, (Rr, M), generator=g)
+    lowest = low[torch.randint(0, len(low), (Rr, M), generator=g)]
+    q = torch.randint(-(1 << 22), (1 << 22) + 1, (Rr, HKV, M, HD), generator=g).to(torch.int32).to(dev)
+    sh = torch.randint(-46, -36, (Rr, HKV, M), generator=g).to(dev)
+    assert tri_exact_attn.rows_scratch(Rr, HKV, M, HD, nrow, S) > 0
+    run = lambda p, ns: tri_exact_attn.attend(q, sh, p.to(dev), cl, bt, rmap, _lut(dev), R.L2E28_HD[HD], nsplit=ns)
+    (n1, d1), (n2, d2) = run(torch.where(masked, -1, qpos), 1), run(torch.where(masked, lowest, qpos), None)
+    assert torch.equal(n1, n2) and torch.equal(d1, d2)
+    Z, gT = 2, M * 100
+    K, V = (torch.randint(-R.LIM3, R.LIM3 + 1, (Z, S, HD), generator=g).to(torch.int32).to(dev) for _ in range(2))
+    qz, shz = q.view(-1, HD)[:Z * gT].view(Z, gT, HD), sh.view(-1)[:Z * gT].view(Z, gT, 1)
+    pz = lambda p: p.view(-1)[:Z * gT].view(Z, gT, 1).to(dev)
+    (n1, d1), (n2, d2) = (prefill(qz, shz, K, V, pz(torch.where(masked, m, qpos)), _lut(dev), R.L2E28_HD[HD])
+                          for m in (torch.tensor(-1), lowest))
+    assert torch.equal(n1, n2) and torch.equal(d1, d2)
+
+
 @pytest.mark.parametrize("HD,npad,pad", [(64, 1, -1), (64, 33, -1), (64, 300, -(1 << 40)), (128, 40, 3), (128, 200, 1 << 40),
                                          (64, 513, None)])
 def test_paged_rows_outside_the_table(dev, HD, npad, pad):
