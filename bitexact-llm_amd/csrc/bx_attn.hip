@@ -55,23 +55,6 @@ __device__ __forceinline__ WeightAt weight_at(int64_t z, int64_t zshift, int64_t
   return w;
 }
 
-// weight_at for zshift >= 0, 0 <= l2e < 2^31 and 0 <= z < 2^62 (z = mx - raw of a visible key): zf = rshc(z, zshift)
-// is then >= 0 and at most 48 2^26 after the clamp, so zf l2e is one 32 x 32 -> 64-bit product below 3 2^61
-// and t, n, f come from 64-bit shifts of it; the same position as weight_at. Negative z (hidden keys, whose
-// weight is discarded) is clamped to 0, which keeps the position inside the table.
-__device__ __forceinline__ WeightAt weight_at_nn(int64_t z, int64_t zshift, int64_t l2e) {
-  int64_t zf = rshc(z, zshift);
-  zf = zf < 0 ? 0 : zf > (48LL << kFZ) ? (48LL << kFZ) : zf;
-  const uint64_t prod = (uint64_t)(uint32_t)zf * (uint64_t)(uint32_t)l2e;
-  const uint64_t t = (prod + (1ULL << (kFZ + 28 - kFT2 - 1))) >> (kFZ + 28 - kFT2);
-  const uint32_t f = (uint32_t)t & ((1u << kFT2) - 1);
-  WeightAt w;
-  w.n = (int64_t)(t >> kFT2);
-  w.idx = w.n < kZeroN ? (int)(f >> (kFT2 - kExp2Bits)) : 0;
-  w.rr = f & ((1u << (kFT2 - kExp2Bits)) - 1);
-  return w;
-}
-
 __device__ __forceinline__ int64_t weight_of(const WeightAt& w, int64_t a, int64_t b) {
   const int64_t v = add_wrap(a, rshc(mul_wrap(b - a, w.rr), kFT2 - kExp2Bits));
   return rshc(v, kExp2One - kFP + w.n);
@@ -2568,11 +2551,10 @@ extern "C" int bx_exact_attn_paged_rope_out_planes(const int64_t* y, int64_t ldy
                        (hipStream_t)stream);
 }
 
-static int int8_paged(const int64_t* q, const int64_t* qpos, int64_t sqpos_r, const int8_t* cache,
-                                  int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs, const int32_t* bt, int64_t sbt,
-                                  int32_t nblk, const int32_t* ptab, int32_t ptab_len, int64_t* num, int64_t* den,
-                                  int32_t R, int32_t HKV, int32_t M, int32_t HD, int32_t nsplit, void* ws,
-                                  int64_t ws_bytes, void* tmp, int64_t tmp_bytes,
+static int int8_paged(const int64_t* q, const int64_t* qpos, int64_t sqpos_r, const int8_t* cache, int64_t sc_nb,
+                      int64_t sc_h, int64_t sc_bs, int32_t bs, const int32_t* bt, int64_t sbt, int32_t nblk,
+                      const int32_t* ptab, int32_t ptab_len, int64_t* num, int64_t* den, int32_t R, int32_t HKV,
+                      int32_t M, int32_t HD, int32_t nsplit, void* ws, int64_t ws_bytes, void* tmp, int64_t tmp_bytes,
                       bx_stream_t stream) {
   BX_REQUIRE(R >= 0 && HKV > 0 && M >= 1, "need M >= 1 queries per (row, KV head)");
   BX_REQUIRE(HD == 64 || HD == 128, "head_dim must be 64 or 128");
@@ -2629,9 +2611,11 @@ extern "C" int bx_int8_attn_paged_scores(const int64_t* q, const int64_t* qpos, 
                     R, HKV, M, HD, nsplit, ws, ws_bytes, tmp, tmp_bytes, stream);
 }
 
-// the limb-plane form's scratch: K and V planes, 3 Z Sp HD bytes each (Sp = S rounded up to 64 keys)
+// the limb-plane form's scratch: K and V planes, 3 Z Sp HD bytes each (Sp = S rounded up to 64 keys), and the weight table
 static int64_t pre2_planes(int64_t Z, int64_t S, int64_t HD) { return 2 * 3 * Z * ((S + 63) / 64 * 64) * HD; }
-static int64_t pre2_scratch(int64_t Z, int64_t S, int64_t HD) { return pre2_planes(Z, S, HD) + (16LL << kExp2Bits); }
+static int64_t pre2_scratch(int64_t Z, int64_t S, int64_t HD) {
+  return pre2_planes(Z, S, HD) + (4LL * (kTabPad + kTabBlocks) + 255) / 256 * 256;
+}
 
 extern "C" int64_t bx_attn_prefill_scratch(int32_t Z, int32_t S, int32_t HD) {
   if (Z <= 0 || S <= 0 || (HD != 64 && HD != 128)) return 0;

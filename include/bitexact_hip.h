@@ -155,9 +155,10 @@ int bx_exact_attn_paged_scores(const int32_t* q, const int64_t* sh, const int64_
 /* The same attention for steps of many tokens per sequence (prefill chunks; the same reference call): the token rows
  * are grouped by block-table row on the device, each sequence's cached K / V limbs are laid out once per call as
  * planes in tmp, and a block runs many tokens of one sequence against each key tile (bx_exact_attn_prefill's main
- * kernel); the tokens of sequences that have few in the step run as in bx_exact_attn_paged_scores. bt has nrow rows; a token whose rmap lies outside [0, nrow) (padding) sees no key: its num and den are 0. q
- * 16-byte aligned. tmp: 16-byte aligned, bx_attn_paged_rows_scratch bytes, no contents kept; the query returns 0 where
- * that form is not available (planes of all nrow sequences above 1 GiB, or sizes bx_exact_attn_paged rejects). */
+ * kernel); the tokens of sequences that have few in the step run as in bx_exact_attn_paged_scores. bt has nrow rows;
+ * a token whose rmap lies outside [0, nrow) (padding) sees no key: its num and den are 0. q 16-byte aligned. tmp:
+ * 16-byte aligned, bx_attn_paged_rows_scratch bytes, no contents kept; the query returns 0 where that form is not
+ * available (planes of all nrow sequences above 1 GiB, or sizes bx_exact_attn_paged rejects). */
 int64_t bx_attn_paged_rows_scratch(int32_t R, int32_t nrow, int32_t HKV, int32_t M, int32_t HD, int32_t keys);
 int bx_exact_attn_paged_rows(const int32_t* q, const int64_t* sh, const int64_t* qpos, int64_t sqpos_r,
                              const int8_t* cache, int64_t sc_nb, int64_t sc_h, int64_t sc_bs, int32_t bs, const int32_t* bt,
