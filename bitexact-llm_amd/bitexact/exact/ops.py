@@ -416,7 +416,8 @@ def _gu_silu(y, lut, flag, split, planes):
     assert split or not planes, "limb planes come from the column-chunked path"
     pl = torch.empty((3, M, ff) if planes else (0,), dtype=torch.int8, device=y.device)
     if split and M > 0:
-        tmp, tmpb = _hip.workspace(y.device, _hip.size_query("bx_silu_quant_scratch", y.device.index, M, ff))   # zero-filled, kept so
+        # zero-filled, kept so
+        tmp, tmpb = _hip.workspace(y.device, _hip.size_query("bx_silu_quant_scratch", y.device.index, M, ff))
         _hip.call("bx_silu_quant_ws", _hip.ptr(y), y.stride(0), ff, _hip.ptr(lut), FR, _hip.ptr(q), ff, _hip.ptr(sh),
                   _hip.ptr(pl) if planes else None, M, _hip.ptr(flag), _hip.ptr(tmp), tmpb, _hip.stream_of(y))
         return q, pl, sh

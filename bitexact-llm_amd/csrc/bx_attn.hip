@@ -1599,9 +1599,10 @@ __device__ __forceinline__ int pre_vpos(int key) {   // tile key -> its Vp posit
 }
 
 // The 2^-f table as the main kernel keeps it in LDS: U[i] = floor((2^60 - lut[i]) / 2^29), 32 bits an entry (64 KiB
-// for the table instead of the 128 KiB of its int64 entries, so it fits beside the ring). pre_table_block (one block per 256 entries) writes it
-// to scratch with one word per block: 1 when its entries can take the short weight rule, i.e. 2^59 <= lut[i] <=
-// 2^60, 0 <= U[i + 1] - U[i] < 2^20 and U[i + 1] > 0 (true of the 2^-f table; any other table takes the general rule).
+// for the table instead of the 128 KiB of its int64 entries, so it fits beside the ring). pre_table_block (one block
+// per 256 entries) writes it to scratch with one word per block: 1 when its entries can take the short weight rule,
+// i.e. 2^59 <= lut[i] <= 2^60, 0 <= U[i + 1] - U[i] < 2^20 and U[i + 1] > 0 (true of the 2^-f table; any other table
+// takes the general rule).
 constexpr int kTabN = 1 << kExp2Bits;                  // entries [0, kTabN]
 constexpr int kTabBlocks = kTabN / 256;
 constexpr int kTabPad = kTabN + 4;                     // words of U in scratch and LDS (16-byte multiple)
@@ -1865,7 +1866,7 @@ struct Pre2 {
   static constexpr int PB = 3 * 64 * HD;             // one operand's three planes of a tile (bytes): a ring slot
   static constexpr int SLOTS = 3;                    // ring: K of tile t, V of tile t, K of tile t + 1, V of t + 1, ...
   static constexpr int KI = PB / 1024;               // 1 KiB instructions per slot
-  // Waves that share 16 query rows, and waves of a block: two waves per SIMD (200 and 219 registers). Measured at
+  // Waves that share 16 query rows, and waves of a block: two waves per SIMD (198 and 213 registers). Measured at
   // head_dim 64 (4 x 1024 tokens): 8 waves 198 us, 12 waves (168 registers, spills) 305, 12 waves of pairs (156
   // registers) 221; at head_dim 128 (1337 tokens): 8 waves of pairs 157 us, 4 single waves (one per SIMD) 234.
   static constexpr int SW = HD == 64 ? 1 : 2;
@@ -1901,17 +1902,18 @@ __device__ __forceinline__ void pin_v(uint32_t& x) { asm("" : "+v"(x)); }
 // MFMAs are issued before a block's weights are formed.
 //
 // The short weight rule (`fast`: no query of the wave has a negative exponent shift, 0 <= l2e < 2^31, and the table
-// passed pre_table_block's check). With U the LDS table, y = (2^60 - v) / 2^29 of the interpolated value v lies in
-// [Uc - 2^-30, Uc + 2) for Uc = U0 + ((U1 - U0) rr >> 12): both entries (fractions at most 1 - 2^-29) and the
-// product are floors, v's own rounding is 2^-30 of the unit. The weight rshc(v, 38 + n) = floor((2^31 + 2^(8+n) - y) / 2^(9+n)) for n <= 22 is
-// then 2^(22-n) + (T >> (9+n)), T = 2^(8+n) - Uc, whatever y is, unless T mod 2^(9+n) <= 1: such a score (2 in
-// 2^(9+n)) takes its value from the table's float64 factors, and from the int64 table where even that is within
-// 2^-25 of a rounding boundary. From n = 23 the weight is 0, v being below 2^60, except at the single position n =
-// 23, f = 0 (Uc = 0: T = 2^31 marks it). Before, every score gathered
-// its 16-byte table pair through L1: with attention scores of unit spread that was 140 of 341 us (4 x 1024 tokens,
-// 32 / 8 heads of 64), the lanes' lines missing the 32 KiB L1. Now 198 us (1337 tokens, heads of 128: 233 -> 157):
-// bound by the integer work per score (about 40 VALU instructions), with sweep 1 about 55 us of it. The second-step
-// values come from LDS too because one wave's memory round trip holds its block at the tile's barrier (238 us).
+// passed pre_table_block's check). With U the LDS table, y = (2^60 - v) / 2^29 of the interpolated value v lies in [Uc
+// - 2^-30, Uc + 2) for Uc = U0 + ((U1 - U0) rr >> 12): both entries (fractions at most 1 - 2^-29) and the product are
+// floors, v's own rounding is 2^-30 of the unit. The weight rshc(v, 38 + n) = floor((2^31 + 2^(8+n) - y) / 2^(9+n))
+// for n <= 22 is then 2^(22-n) + (T >> (9+n)), T = 2^(8+n) - Uc, whatever y is, unless T mod 2^(9+n) <= 1: such a
+// score (2 in 2^(9+n)) takes its value from the table's float64 factors, and from the int64 table where even that is
+// within 2^-25 of a rounding boundary. From n = 23 the weight is 0, v being below 2^60, except at the single position
+// n = 23, f = 0 (Uc = 0: T = 2^31 marks it).
+// Before, every score gathered its 16-byte table pair through L1: with attention scores of unit spread that was 140 of
+// 341 us (4 x 1024 tokens, 32 / 8 heads of 64), the lanes' lines missing the 32 KiB L1. Now 198 us (1337 tokens, heads
+// of 128: 233 -> 157): bound by the integer work per score (54 VALU instructions over both sweeps), with sweep 1 about
+// 55 us of it. The second-step values come from LDS too because one wave's memory round trip holds its block at the
+// tile's barrier (238 us).
 // ROWS: the paged form. Block (slot, KV head h); the block's query i is query i % M of the slot's token i / M.
 template <int HD, bool ROWS>
 __global__ __launch_bounds__(64 * Pre2<HD>::NW, 1) void attn_pre2_kernel(AttnArgs p, const int8_t* planes, int Z,

@@ -162,14 +162,15 @@ __global__ __launch_bounds__(256 * RT) void bmm_mfma_kernel(const TA* a, int64_t
   }
 }
 
-// Rows kernel: 3 x 3 limbs of int32 operands, a's rows contiguous (p.v's weights). A's values never pass through LDS: lane (r, ch) of a wave loads k = 16 u + 4 ch .. + 3 (u = 0..3) of row r
-// as four 16-byte words (64 contiguous bytes of a row per four lanes), splits them in registers and has the MFMA's A
-// operand in place, with the step's k order permuted to 16 ch + 4 u + e; B's limb planes are written to LDS in the same
-// order, into one of two buffers, so a step has one barrier. A's next PA steps travel while the MFMAs run. Buffer loads
-// of four dwords need 4-byte alignment only; a part-filled last k step loads single values, those past K as zeros of a.
-// NW waves of 16 rows x 16 CB columns; BV: b's k contiguous; TAIL: K % 64 != 0. Bound by reading a: Z = 16, 4096 x 1024 by 64 columns
-// 116 -> 71 us (268 MB, 4.2 TB/s with the results), by 128 columns 209 -> 111; bmm_mfma_kernel has four bounds-checked
-// 4-byte loads for each of this kernel's 16-byte ones, two barriers a step, and A's planes through LDS.
+// Rows kernel: 3 x 3 limbs of int32 operands, a's rows contiguous (p.v's weights). A's values never pass through LDS:
+// lane (r, ch) of a wave loads k = 16 u + 4 ch .. + 3 (u = 0..3) of row r as four 16-byte words (64 contiguous bytes
+// of a row per four lanes), splits them in registers and has the MFMA's A operand in place, with the step's k order
+// permuted to 16 ch + 4 u + e; B's limb planes are written to LDS in the same order, into one of two buffers, so a
+// step has one barrier. A's next PA steps travel while the MFMAs run. Buffer loads of four dwords need 4-byte
+// alignment only; a part-filled last k step loads single values, those past K as zeros of a. NW waves of 16 rows x 16
+// CB columns; BV: b's k contiguous; TAIL: K % 64 != 0. Bound by reading a: Z = 16, 4096 x 1024 by 64 columns 116 -> 71
+// us (268 MB, 4.2 TB/s with the results), by 128 columns 209 -> 111; bmm_mfma_kernel has four bounds-checked 4-byte
+// loads for each of this kernel's 16-byte ones, two barriers a step, and A's planes through LDS.
 template <int CB, int NW, int PA, bool BV, bool TAIL>
 __global__ __launch_bounds__(64 * NW, 2) void bmm_rows_kernel(const int32_t* a, int64_t saz, int64_t sam, const int32_t* b,
                                                            int64_t sbz, int64_t sbk, int64_t sbn, int64_t* c, int64_t scz,

@@ -1,9 +1,9 @@
 // Row-wise integer stages around the GEMMs and the attention, one block per row (1024 threads for few rows, as in a
 // decode step, so each row spreads over a whole CU; smaller blocks for many; softmax rows use 256; the SiLU stage of
-// few rows goes over column chunks, that of many walks rows with its table in LDS) with DPP wavefront int64 reductions: RMSNorm + per-row quantization (segs.norm_quant,
-// optionally after the residual add or the
-// embedding gather), SiLU gating + quantization (segs.silu_y + quant_silu), the masked softmax weights
-// (segs.softmax), and the attention output rule (segs.attn_out = div_round + regroup + quant).
+// few rows goes over column chunks, that of many walks rows with its table in LDS) with DPP wavefront int64
+// reductions: RMSNorm + per-row quantization (segs.norm_quant, optionally after the residual add or the embedding
+// gather), SiLU gating + quantization (segs.silu_y + quant_silu), the masked softmax weights (segs.softmax), and the
+// attention output rule (segs.attn_out = div_round + regroup + quant).
 #include "bx_common.h"
 #include "bx_introws.h"
 
